@@ -823,6 +823,7 @@ struct AddrGradArgs {
   float* part_k;             // [n_blk][2][H][2][n_sub][HALF]: d unit sub-keys
   int B, T, H, n_sub, kk;
   int set0;                  // the first address set (grid z covers set0 .. set0 + gridDim.z - 1)
+  int wave_tokens;           // tokens per wave (addr_grad_tile_kernel: a multiple of its 32-token tile)
 };
 
 
@@ -947,7 +948,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
   double acc_lam = 0.0;
   const int64_t N = static_cast<int64_t>(a.B) * a.T;
   const int64_t cg_stride = N * a.H * KP;
-  int64_t n = static_cast<int64_t>(blockIdx.x) * W * kAddrGradWaveTokens + w;
+  int64_t n = static_cast<int64_t>(blockIdx.x) * W * a.wave_tokens + w;
   int b = static_cast<int>(n / a.T);
   int t = static_cast<int>(n - static_cast<int64_t>(b) * a.T);
   // one token's loads, issued a token ahead: unconditional, at indexes clamped into the arrays (masked after use)
@@ -971,7 +972,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
     return x;
   };
   TokIn cur = load(n < N ? n : 0, n < N ? b : 0, n < N ? t : 0);
-  for (int i = 0; i < kAddrGradWaveTokens; ++i) {
+  for (int i = 0; i < a.wave_tokens; ++i) {
     if (n >= N) break;   // wave-uniform
     // the next token (W positions on) and its loads
     const int64_t n2 = n + W;
@@ -981,7 +982,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
       ++b2;
     }
     TokIn nxt = cur;
-    if (i + 1 < kAddrGradWaveTokens && n2 < N) nxt = load(n2, b2, t2);
+    if (i + 1 < a.wave_tokens && n2 < N) nxt = load(n2, b2, t2);
     const int64_t prow = ((static_cast<int64_t>(b) * a.H + h) * a.T + t) * KP;
     const float z = (DA == 64 || e < DA) ? to_f32(cur.z) + ab : 0.f;
     const float glv = gated ? to_f32(cur.gl) : 0.f;
@@ -1073,6 +1074,346 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
   for (int i = tid; i < KS; i += blockDim.x) {
     float s = 0.f;
     for (int q = 0; q < W; ++q) s += dk[q * KS + i];
+    a.part_k[pid * KS + i] = s;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// addr_grad_tile_kernel: the same gradients for n_sub <= 64, 32 tokens of one (head, address set) at a time on the
+// matrix cores.  Per tile a wave
+//   picks   holds KP lanes per token (64 / KP tokens side by side, so every lane has a pick): softmax and gate
+//           backward by DPP over the token's lanes, then g_j = dsv_j / 2 added into the token's row of G, its
+//           sparse gradient by unit sub-key (LDS, [32 tokens][both halves' sub-keys]; picks in pick order)
+//   du      = G K^ (v_mfma_f32_32x32x2f32: rows tokens, columns address elements)
+//   dz      from du, u and |z|, held in the product's own layout: lane l keeps column l % 32 of 16 tokens, so the
+//           sums over an address half are sums over lanes of a half-wave
+//   dk^    += G^T U (the products' tokens in the order U's registers hold them)
+// Everything stays float32 (the products are fused multiply-adds in float32).  The kernel below does the same one
+// token at a time, one lane per address element: per token 8 dependent LDS read-modify-writes for dk^, 24 readlanes
+// and the pick math on 8 of 64 lanes.  B=8, T=2048, 12 heads, k=8, bfloat16: 218 -> 117 us; the table layer's
+// (B=4, T=1024, one head, 64 sub-keys, k=16, float32): 50 -> 28 us.  What bounds it: 220 MB in and out (46 us at a
+// copy's rate) and the latency of a tile's chain (loads, k LDS additions, products) with two waves per SIMD: the
+// kernel takes 256 registers, and at three waves (168, 73 of them spilled) it took 141 us.
+// Sub-keys past n_sub, columns past the address and tokens past the end are zero rows and columns of the tiles.
+// Waves per block 4; tiles per wave chosen by addr_tiles (enough blocks for the chip first, then longer waves, since
+// every wave loads the head's sub-keys and leaves a partial sum).
+constexpr int kAddrTile = 32;
+constexpr int kAddrTileWaves = 4;
+
+// sum over the 32 lanes of the lane's half-wave
+__device__ __forceinline__ float sum32(float v) {
+  v = sum16(v);
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
+
+// orders the LDS accesses of a wave's lanes among themselves (the hardware runs a wave's LDS operations in order)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// sum over the columns of the lane's address half: columns 0 .. HALF - 1 of a half-wave with HALF > 16 (a tile per
+// half), else columns [0, HALF) or [HALF, 2 HALF); columns past them hold zero
+template <int HALF>
+__device__ __forceinline__ float col_sum(float v, int col) {
+  if constexpr (HALF > 16) {
+    return sum32(v);
+  } else if constexpr (HALF == 16) {
+    return sum16(v);
+  } else if constexpr (HALF == 8) {
+    return sum8(v);
+  } else {
+    const float s1 = sum32(col < HALF ? v : 0.f);
+    const float s2 = sum32(col >= HALF ? v : 0.f);
+    return col < HALF ? s1 : s2;
+  }
+}
+
+// LDS of one addr_grad_tile block: the waves' G tiles and the unit sub-keys, in the same bytes at the end their dk^ and partial records
+__host__ __device__ constexpr int addr_tile_pitch(int nsb) { return 64 * nsb + 4; }
+__host__ __device__ constexpr size_t addr_tile_lds(int n_sub, int half, int nsb) {
+  const size_t g = sizeof(float) * (kAddrTileWaves * kAddrTile * addr_tile_pitch(nsb) + 64 * nsb * 32);
+  const size_t d = sizeof(float) * kAddrTileWaves * 2 * static_cast<size_t>(n_sub) * half;
+  return (g > d ? g : d) + kAddrTileWaves * (sizeof(double) + sizeof(float) * (2 * half + 2));
+}
+
+template <int HALF, int NSB, int KP, typename InT>
+__global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(AddrGradArgs a) {
+  constexpr int DA = 2 * HALF;
+  constexpr int NT = HALF > 16 ? 2 : 1;          // column tiles: one per half, or both halves in one
+  constexpr int SB = 32 * NSB;                   // G columns of one half
+  constexpr int GP = addr_tile_pitch(NSB);
+  constexpr int TPI = 64 / KP;                   // tokens per pick step
+  constexpr int NIT = kAddrTile / TPI;
+  extern __shared__ __attribute__((aligned(16))) unsigned char albuf[];
+  const int n_sub = a.n_sub;
+  const int KS = 2 * n_sub * HALF;
+  const int h = blockIdx.y;
+  const int set = a.set0 + blockIdx.z;   // 0: write keys, 1: read queries
+  const int tid = threadIdx.x;
+  const int w = tid >> 6;
+  const int lane = tid & 63;
+  const int col = lane & 31;             // column of a tile; in G's products also a token or a sub-key
+  const int hw = lane >> 5;
+  const int pj = lane & (KP - 1);        // the lane's pick in the pick steps
+  const int kk = a.kk;
+  float* G = reinterpret_cast<float*>(albuf) + w * kAddrTile * GP;
+
+  // the unit sub-keys, [half][sub-key][column of its tile]: zero past n_sub and, with both halves in one tile, in the
+  // other half's columns
+  float* kn = reinterpret_cast<float*>(albuf) + kAddrTileWaves * kAddrTile * GP;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const float* keys = a.keys[p] + static_cast<int64_t>(h) * n_sub * HALF;
+    const int c = NT == 2 ? col : col - p * HALF;
+    const bool own = c >= 0 && c < HALF;
+    for (int i0 = 2 * w; i0 < SB; i0 += 2 * kAddrTileWaves) {   // two rows a wave: one per half-wave
+      const int i = i0 + hw;
+      const float v = own && i < n_sub ? keys[i * HALF + c] : 0.f;
+      const float nrm = fmaxf(sqrtf(col_sum<HALF>(v * v, col)), 1e-12f);
+      kn[(p * SB + i) * 32 + col] = v / nrm;
+    }
+  }
+  __syncthreads();
+  const float tau = expf(a.log_scale[h]);
+  float ab[NT];
+#pragma unroll
+  for (int p = 0; p < NT; ++p) {
+    const int e = p * HALF + col;
+    ab[p] = a.addr_b && (NT == 2 ? col < HALF : col < DA) ? a.addr_b[h * DA + e] : 0.f;
+  }
+  const float gb = a.gate_bias ? a.gate_bias[h] : 0.f;
+  // slot -> (i1, i2) = (s / n_sub, s % n_sub) by a multiply-high: exact for s < 2^16, n_sub <= 256
+  const uint32_t magic = n_sub > 1 ? 0xFFFFFFFFu / static_cast<uint32_t>(n_sub) + 1u : 0u;
+  const InT* zb = static_cast<const InT*>(set == 0 ? a.kz : a.qz) + static_cast<int64_t>(h) * DA;
+  const int zs = static_cast<int>(set == 0 ? a.kz_stride : a.qz_stride);   // below 2^25 (the launcher's rule)
+  const bool gated = set == 0 && a.gl;
+  const int32_t* slot = a.slot[set];
+  const float* wtp = a.wt[set];
+  const float* scp = a.score[set];
+  const float* dotp = a.dot[set];
+  float* dzp = a.dz[set] + static_cast<int64_t>(h) * DA;
+  const int dzs = static_cast<int>(a.dz_stride[set]);
+  const bool live_col = NT == 2 ? col < HALF : col < DA;
+  const int64_t N = static_cast<int64_t>(a.B) * a.T;   // below 2^31: each token has picks of 4 * 32 bytes and more
+  const int64_t cg_stride = N * a.H * KP;
+  float acc_tau = 0.f, acc_gb = 0.f, acc_ab[NT];
+  double acc_lam = 0.0;
+  floatx16 dk[2][NSB];
+#pragma unroll
+  for (int p = 0; p < NT; ++p) acc_ab[p] = 0.f;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < NSB; ++q)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dk[p][q][r] = 0.f;
+
+  int64_t n0 = (static_cast<int64_t>(blockIdx.x) * kAddrTileWaves + w) * a.wave_tokens;
+  for (int i = 0; i < a.wave_tokens && n0 < N; i += kAddrTile, n0 += kAddrTile) {   // wave-uniform
+    // loads: unconditional, a missing token reads token 0 and a dead pick the token's first (masked after use)
+    int slr[NIT], tr[NIT];
+    float svr[NIT], wtr[NIT], dwr[NIT];
+    InT glr[NIT];
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      const int64_t nn = n0 + it * TPI + lane / KP;
+      const uint32_t n = nn < N ? static_cast<uint32_t>(nn) : 0u;
+      const uint32_t b = n / static_cast<uint32_t>(a.T);
+      const uint32_t t = n - b * static_cast<uint32_t>(a.T);
+      const int64_t e = ((static_cast<int64_t>(b) * a.H + h) * a.T + t) * KP + (pj < kk ? pj : 0);
+      tr[it] = static_cast<int>(t);
+      slr[it] = slot[e];
+      svr[it] = scp[e];
+      wtr[it] = wtp[e];
+      dwr[it] = dotp[e];
+      for (int c = 1; c < a.n_cg; ++c) dwr[it] += dotp[c * cg_stride + e];
+      glr[it] = gated ? static_cast<const InT*>(a.gl)[n * a.g_stride + h] : zb[0];
+    }
+    const InT* zt = zb + n0 * zs;   // the tile's rows: offsets from here in 32 bits
+    const int left = static_cast<int>(N - n0 < kAddrTile ? N - n0 : kAddrTile);
+    InT zr[NT][16];
+#pragma unroll
+    for (int p = 0; p < NT; ++p)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 8 * (r / 4) + 4 * hw + r % 4;
+        zr[p][r] = zt[(row < left ? row : 0) * zs + (live_col ? p * HALF + col : 0)];
+      }
+    float* dzt = dzp + n0 * dzs;
+    // G to zero, then the picks' gradients
+#pragma unroll
+    for (int k = 0; k < (kAddrTile * GP + 255) / 256; ++k) {
+      const int at = 4 * (lane + 64 * k);
+      if (at < kAddrTile * GP) *reinterpret_cast<float4*>(&G[at]) = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float hs[NIT];
+    int g1[NIT], g2[NIT];
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      const bool valid = n0 + it * TPI + lane / KP < N;
+      const bool pl = valid && pj < kk;
+      int sl = pl ? slr[it] : 0;
+      sl = (sl >= 0 && sl < n_sub * n_sub) ? sl : 0;
+      const float sv = pl ? svr[it] : 0.f;
+      const float wt = pl ? wtr[it] : 0.f;
+      const float dw = pl ? dwr[it] : 0.f;
+      const float P = pick_sum<KP>(wt * dw);
+      float dx;
+      if (set == 1) {   // read: softmax
+        dx = wt * (dw - P);
+        if (pj == 0) acc_lam += static_cast<double>(tr[it]) * static_cast<double>(P);
+      } else {          // write: gated softmax
+        if (pj == 0) acc_lam -= static_cast<double>(tr[it] + 1) * static_cast<double>(P);
+        const float x0 = __shfl(sv, lane & ~(KP - 1)) * tau;
+        float pr = pl ? __expf(sv * tau - x0) : 0.f;
+        const float ps = pick_sum<KP>(pr);
+        pr *= fast_rcp(valid ? ps : 1.f);
+        const float gt = gated ? fast_rcp(1.f + __expf(-(to_f32(glr[it]) + gb))) : 1.f;
+        const float S = pick_sum<KP>(pr * gt * dw);
+        const float dg = pick_sum<KP>(pr * dw);
+        dx = pr * (gt * dw - S);
+        if (gated && valid && pj == 0) {
+          const float dlogit = dg * gt * (1.f - gt);
+          if (a.dgl) a.dgl[(n0 + it * TPI + lane / KP) * a.dgl_stride + h] = dlogit;
+          acc_gb += dlogit;
+        }
+      }
+      if (!pl) dx = 0.f;
+      acc_tau = fmaf(sv, dx, acc_tau);
+      hs[it] = 0.5f * tau * dx;
+      const int i1 = n_sub > 1 ? static_cast<int>(__umulhi(static_cast<uint32_t>(sl), magic)) : sl;
+      const int row = (it * TPI + lane / KP) * GP;
+      g1[it] = row + i1;
+      g2[it] = row + SB + (sl - i1 * n_sub);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int j = 0; j < KP; ++j) {
+      if (j >= kk) break;   // uniform
+      if (pj == j) {        // one lane per token: picks of a token that share a sub-key add up in pick order
+        float x1[NIT], x2[NIT];
+#pragma unroll
+        for (int it = 0; it < NIT; ++it) {
+          x1[it] = G[g1[it]];
+          x2[it] = G[g2[it]];
+        }
+#pragma unroll
+        for (int it = 0; it < NIT; ++it) {
+          G[g1[it]] = x1[it] + hs[it];
+          G[g2[it]] = x2[it] + hs[it];
+        }
+      }
+      wave_lds_fence();
+    }
+#pragma unroll
+    for (int p = 0; p < NT; ++p) {
+      // du: rows tokens, columns address elements; lane l's sub-keys at step s are 16 (l / 32) + s of each block
+      floatx16 du;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) du[r] = 0.f;
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp) {
+        if (NT == 2 && pp != p) continue;
+#pragma unroll
+        for (int q = 0; q < NSB; ++q)
+#pragma unroll
+          for (int s4 = 0; s4 < 4; ++s4) {
+            const float4 g4 = *reinterpret_cast<const float4*>(&G[col * GP + pp * SB + 32 * q + 16 * hw + 4 * s4]);
+            const float* kr = &kn[(pp * SB + 32 * q + 16 * hw + 4 * s4) * 32 + col];
+            du = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.x, kr[0], du, 0, 0, 0);
+            du = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.y, kr[32], du, 0, 0, 0);
+            du = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.z, kr[64], du, 0, 0, 0);
+            du = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.w, kr[96], du, 0, 0, 0);
+          }
+      }
+      float u[16], inz[16], nz[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const bool live = live_col && 8 * (r / 4) + 4 * hw + r % 4 < left;
+        const float z = live ? to_f32(zr[p][r]) + ab[p] : 0.f;
+        nz[r] = __builtin_amdgcn_sqrtf(col_sum<HALF>(z * z, col));
+        inz[r] = fast_rcp(fmaxf(nz[r], 1e-12f));
+        u[r] = z * inz[r];
+      }
+      // dk^: rows sub-keys, columns address elements; register r's two tokens are the step's two
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp) {
+        if (NT == 2 && pp != p) continue;
+#pragma unroll
+        for (int q = 0; q < NSB; ++q)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const float gt = G[(8 * (r / 4) + 4 * hw + r % 4) * GP + pp * SB + 32 * q + col];
+            dk[pp][q] = __builtin_amdgcn_mfma_f32_32x32x2f32(gt, u[r], dk[pp][q], 0, 0, 0);
+          }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 8 * (r / 4) + 4 * hw + r % 4;
+        const float ud = col_sum<HALF>(u[r] * du[r], col);
+        const float dz = nz[r] > 1e-12f ? (du[r] - u[r] * ud) * inz[r] : du[r] * 1e12f;
+        if (live_col && row < left) {
+          dzt[row * dzs + p * HALF + col] = dz;
+          acc_ab[p] += dz;
+        }
+      }
+    }
+    wave_lds_fence();
+  }
+  // block sums in a fixed order: waves -> LDS -> threads
+  acc_tau = wave_sum(acc_tau);
+  acc_gb = wave_sum(acc_gb);
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) acc_lam += __shfl_xor(acc_lam, off);
+#pragma unroll
+  for (int p = 0; p < NT; ++p) acc_ab[p] += __shfl_xor(acc_ab[p], 32);
+  __syncthreads();   // every wave's G is done with
+  float* dkb = reinterpret_cast<float*>(albuf);
+  unsigned char* tail = albuf + (addr_tile_lds(n_sub, HALF, NSB) -
+                                 kAddrTileWaves * (sizeof(double) + sizeof(float) * (2 * HALF + 2)));
+  double* redd = reinterpret_cast<double*>(tail);
+  float* red = reinterpret_cast<float*>(tail + kAddrTileWaves * sizeof(double));
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int c = NT == 2 ? col : col - p * HALF;
+    if (c < 0 || c >= HALF) continue;
+#pragma unroll
+    for (int q = 0; q < NSB; ++q)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * q + 8 * (r / 4) + 4 * hw + r % 4;
+        if (i < n_sub) dkb[w * KS + (p * n_sub + i) * HALF + c] = dk[p][q][r];
+      }
+  }
+  if (hw == 0) {
+#pragma unroll
+    for (int p = 0; p < NT; ++p)
+      if (NT == 2 ? col < HALF : col < DA) red[w * (DA + 2) + p * HALF + col] = acc_ab[p];
+  }
+  if (lane == 0) {
+    red[w * (DA + 2) + DA] = acc_tau;
+    red[w * (DA + 2) + DA + 1] = acc_gb;
+    redd[w] = acc_lam;
+  }
+  __syncthreads();
+  const int64_t pid = (static_cast<int64_t>(blockIdx.x) * gridDim.z + blockIdx.z) * a.H + h;
+  for (int c = tid; c < DA + 2; c += blockDim.x) {
+    float s = 0.f;
+    for (int q = 0; q < kAddrTileWaves; ++q) s += red[q * (DA + 2) + c];
+    // record order: dtau, d gate bias, d addr_b[DA]
+    const int f = c == DA ? 0 : c == DA + 1 ? 1 : 2 + c;
+    a.part_f[pid * (2 + DA) + f] = s;
+  }
+  if (tid == 0) {
+    double s = 0.0;
+    for (int q = 0; q < kAddrTileWaves; ++q) s += redd[q];
+    a.part_d[pid] = s;
+  }
+  for (int i = tid; i < KS; i += blockDim.x) {
+    float s = 0.f;
+    for (int q = 0; q < kAddrTileWaves; ++q) s += dkb[q * KS + i];
     a.part_k[pid * KS + i] = s;
   }
 }
@@ -1304,9 +1645,25 @@ int addr_grad_waves(int n_sub, int half, int KP) {
   return 0;
 }
 
+// 32-token tiles per wave of addr_grad_tile_kernel: the fewest that leave no more than two blocks for each of the 256
+// compute units (two fit), at most 8; 0 for more than 64 sub-keys per half, which addr_grad_kernel serves
+int addr_tiles(const Plan& p, int sets) {
+  if (p.n_sub > 64) return 0;
+  const int64_t N = static_cast<int64_t>(p.B) * p.T;
+  int tiles = 1;
+  while (tiles < 8 && (N + 128 * tiles - 1) / (128 * tiles) * p.H * sets > 512) ++tiles;
+  return tiles;
+}
+
+// tokens per block of the addressing backward
+int64_t addr_block_tokens(int tiles, int waves) {
+  return tiles ? static_cast<int64_t>(tiles) * kAddrTile * kAddrTileWaves
+               : static_cast<int64_t>(waves) * kAddrGradWaveTokens;
+}
+
 struct GradPlan {
   Plan p;
-  int cw, n_cg, n_rb, n_blk, addr_waves;
+  int cw, n_cg, n_rb, n_blk, addr_waves, tiles;
   size_t off_dnum, off_dden, off_dotw, off_dotr, off_p1, off_pf, off_pd, off_pk, off_sums, off_chains, total;
 };
 
@@ -1329,7 +1686,8 @@ int make_grad_plan(const sdm_rt_dims* d, GradPlan* g) {
   g->n_cg = p.dh / g->cw;
   const int64_t N = static_cast<int64_t>(p.B) * p.T;
   g->n_rb = static_cast<int>((N + kReadGradRows - 1) / kReadGradRows);
-  const int64_t tpb = static_cast<int64_t>(g->addr_waves) * kAddrGradWaveTokens;
+  g->tiles = addr_tiles(p, 2);
+  const int64_t tpb = addr_block_tokens(g->tiles, g->addr_waves);
   g->n_blk = static_cast<int>((N + tpb - 1) / tpb);
   const size_t hd = static_cast<size_t>(p.H) * p.dh;
   const size_t picks = static_cast<size_t>(N) * p.H * p.pitch;
@@ -1400,8 +1758,25 @@ int launch_grad_scan(const GradPlan& g, const GradScanArgs& a, hipStream_t st) {
 
 template <int HALF, typename InT>
 struct AddrGradLaunch {
-  static int run(const GradPlan& g, const AddrGradArgs& a, hipStream_t st) {
+  template <int NSB, int KP>
+  static int run_tiles(const GradPlan& g, AddrGradArgs a, hipStream_t st) {
+    static const bool ok = allow_lds(reinterpret_cast<const void*>(&addr_grad_tile_kernel<HALF, NSB, KP, InT>));
+    if (!ok) return lds_err("addr grad");
+    a.wave_tokens = g.tiles * kAddrTile;
+    hipLaunchKernelGGL((addr_grad_tile_kernel<HALF, NSB, KP, InT>), dim3(g.n_blk, g.p.H, 2 - a.set0),
+                       dim3(64 * kAddrTileWaves), addr_tile_lds(g.p.n_sub, HALF, NSB), st, a);
+    return check_launch("addr grad");
+  }
+
+  static int run(const GradPlan& g, AddrGradArgs a, hipStream_t st) {
     const Plan& p = g.p;
+    // the tile kernel's offsets inside a tile are 32 bits
+    const int64_t far = std::max(std::max(a.kz_stride, a.qz_stride), std::max(a.dz_stride[0], a.dz_stride[1]));
+    if (g.tiles && far < (1 << 25)) {
+      if (p.n_sub <= 32) return p.pitch == 8 ? run_tiles<1, 8>(g, a, st) : run_tiles<1, 16>(g, a, st);
+      return p.pitch == 8 ? run_tiles<2, 8>(g, a, st) : run_tiles<2, 16>(g, a, st);
+    }
+    a.wave_tokens = static_cast<int>((addr_block_tokens(g.tiles, g.addr_waves) + g.addr_waves - 1) / g.addr_waves);
     const size_t lds = addr_grad_lds(p.n_sub, HALF, g.addr_waves);
     dim3 grid(g.n_blk, p.H, 2 - a.set0);
     dim3 block(64 * g.addr_waves);
@@ -1429,7 +1804,7 @@ int check_saved(const sdm_rt_saved* s, bool need_den) {
 // workspace of sdm_rt_table_backward: per-pick gradients, addressing partials (read set only), float64 sums
 struct TablePlan {
   Plan p;
-  int n_blk, addr_waves, key_bits;
+  int n_blk, addr_waves, tiles, key_bits;
   int64_t n_entries;
   size_t off_dw, off_pf, off_pd, off_pk, off_sums, off_keys, off_count, off_offsets, off_cub, cub_bytes, total;
 };
@@ -1443,7 +1818,8 @@ int make_table_plan(const sdm_rt_dims* d, TablePlan* g) {
   g->addr_waves = addr_grad_waves(p.n_sub, p.half, p.pitch);
   if (!g->addr_waves) return set_err(SDM_RT_EUNSUPPORTED, "table backward: n_sub = %d sub-keys do not fit in LDS", p.n_sub);
   const int64_t N = static_cast<int64_t>(p.B) * p.T;
-  const int64_t tpb = static_cast<int64_t>(g->addr_waves) * kAddrGradWaveTokens;
+  g->tiles = addr_tiles(p, 1);
+  const int64_t tpb = addr_block_tokens(g->tiles, g->addr_waves);
   g->n_blk = static_cast<int>((N + tpb - 1) / tpb);
   const size_t KSH = static_cast<size_t>(p.H) * 2 * p.n_sub * p.half;
   size_t o = 0;
@@ -1859,6 +2235,7 @@ int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, 
     gp.p = p;
     gp.n_blk = g.n_blk;
     gp.addr_waves = g.addr_waves;
+    gp.tiles = g.tiles;
     AddrGradArgs a{};
     a.kz = q;
     a.kz_stride = q_row_stride;

@@ -148,6 +148,19 @@ def test_grad_layer_shape_bf16():
     check_case("layer-bf16", 15, 1, 256, 12, 64, 64, 32, 8, dtype=torch.bfloat16, overlap=0.8, reset_p=0.01)
 
 
+@pytest.mark.parametrize("B,T,H,dh,d_a,n_sub,k,dtype", [
+    (1, 1, 1, 8, 64, 32, 8, torch.float32),          # one token in a tile of 32
+    (1, 31, 2, 8, 64, 33, 8, torch.bfloat16),        # a second sub-key block of one row
+    (3, 43, 2, 16, 48, 32, 16, torch.float32),       # tiles across batch rows, half width 24 in 32 columns
+    (1, 129, 2, 8, 32, 50, 16, torch.float32),       # one token past a block of four tiles
+    (2, 97, 3, 8, 6, 5, 4, torch.float32),           # both halves of 3 columns in one tile
+    (7, 700, 12, 8, 32, 12, 8, torch.bfloat16),      # several tiles per wave, the last blocks short
+])
+def test_address_gradients_at_tile_edges(B, T, H, dh, d_a, n_sub, k, dtype):
+    """addr_grad_tile_kernel where its 32-token tiles, 32-row sub-key blocks and 32-column address tiles end."""
+    check_case("tile", 31, B, T, H, dh, d_a, n_sub, k, dtype=dtype, overlap=0.8)
+
+
 def test_backward_is_deterministic():
     t, reset = make(16, 1, 200, 4, 32, 16, 8, overlap=0.7)
     cfg = dict(k=8, read_mode="mean", out_norm=True, read_eps=1e-3, out_norm_eps=1e-2)

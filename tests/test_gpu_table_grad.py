@@ -64,6 +64,12 @@ def test_table_grad_trained_sdm_layer_shape():
     check_table("layer", 3, 1, 128, 1, 768, 32, 64, 16, dtype=torch.bfloat16)
 
 
+@pytest.mark.parametrize("n_sub", [64, 65])
+def test_table_grad_at_the_sub_key_limit_of_the_tiles(n_sub):
+    """64 sub-keys per half on addr_grad_tile_kernel, 65 on addr_grad_kernel."""
+    check_table("limit", 5, 3, 45, 1, 16, 32, n_sub, 16)
+
+
 def _trained64(P, pre, x, si, H, d_a):
     B, T, d = x.shape
     q = (_rms64(x, P[pre + "norm.w"]) @ P[pre + "wq.weight"].T).view(B, T, H, d_a)
