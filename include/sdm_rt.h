@@ -383,6 +383,45 @@ int sdm_rt_backward(const sdm_rt_dims* dims, const sdm_rt_params* params,
                     const void* dy, int64_t dy_row_stride, sdm_rt_dtype dy_dtype,
                     const sdm_rt_grads* grads, void* workspace, size_t workspace_bytes, void* stream);
 
+/* sdm_rt_backward with the row gradients (d_kz, d_qz, d_v, d_gate_logits) in grad_dtype: with SDM_RT_BF16 their
+ * pointers hold bfloat16 rows (strides in elements), each value rounded once from the float32 result.  The parameter
+ * gradients stay float32.  sdm_rt_backward is this with SDM_RT_F32. */
+int sdm_rt_backward_typed(const sdm_rt_dims* dims, const sdm_rt_params* params,
+                          const void* kz, int64_t kz_row_stride, const void* qz, int64_t qz_row_stride,
+                          const void* v, int64_t v_row_stride, const void* gate_logits, int64_t gate_row_stride,
+                          sdm_rt_dtype in_dtype, const uint8_t* reset, const sdm_rt_saved* saved,
+                          const void* dy, int64_t dy_row_stride, sdm_rt_dtype dy_dtype,
+                          const sdm_rt_grads* grads, sdm_rt_dtype grad_dtype, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace sdm_rt_weight_grad needs (0: none). */
+size_t sdm_rt_weight_grad_workspace_bytes(int64_t rows, int32_t n, int32_t k);
+
+/* The weight gradient of a map y = x W^T: out[n][k] (float32, contiguous, 16-byte aligned) = sum over the rows of
+ * dy[row][n] x[row][k], dy and x bfloat16, float32 sums in a fixed order (deterministic).  n and k multiples of 8,
+ * rows 16-byte aligned. */
+int sdm_rt_weight_grad(const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride, int64_t rows,
+                       int32_t n, int32_t k, float* out, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace sdm_rt_rms_norm_backward needs when it writes dw. */
+size_t sdm_rt_rms_norm_backward_workspace_bytes(int64_t rows, int32_t d);
+
+/* The backward of sdm_rt_rms_norm (its roundings taken as identities): dx (rows in x's type, or NULL) and dw ([d]
+ * float32, or NULL) for dy, the gradient of the normed rows; float32 arithmetic, the sum over rows in a fixed order.
+ * d a multiple of 8 up to 2,048, rows and w 16-byte aligned, at least one row. */
+int sdm_rt_rms_norm_backward(const void* x, int64_t x_row_stride, sdm_rt_dtype x_dtype,
+                             const void* dy, int64_t dy_row_stride, sdm_rt_dtype dy_dtype, int64_t rows, int32_t d,
+                             const float* w, float eps, void* dx, int64_t dx_row_stride, float* dw,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
+/* The mixer's projection weights (track4_onesdm_models.py:199-206) packed for its two maps, in out_dtype: out
+ * [first_rows + d][d] = [wk; wq; wg; zero rows up to first_rows; wv], bias_out [first_rows + d] (or NULL) zero except
+ * gate_bias on wg's rows.  wk, wq [addr_rows][d], wg [heads][d] (NULL without the write gate), wv [d][d], gate_bias
+ * [heads], all contiguous in src_dtype, 16-byte aligned. */
+int sdm_rt_pack_projection(const void* wk, const void* wq, const void* wg, const void* wv, const void* gate_bias,
+                           sdm_rt_dtype src_dtype, int32_t addr_rows, int32_t heads, int32_t first_rows, int32_t d,
+                           void* out, void* bias_out, sdm_rt_dtype out_dtype, void* stream);
+
 /* Bytes of workspace sdm_rt_table_backward needs (0 on invalid dims or a shape it does not cover). */
 size_t sdm_rt_table_backward_workspace_bytes(const sdm_rt_dims* dims);
 

@@ -146,6 +146,21 @@ SIGNATURES = {
                                        ctypes.c_int, c_void_p, ctypes.POINTER(SdmRtSaved),
                                        c_void_p, c_i64, ctypes.c_int,
                                        ctypes.POINTER(SdmRtGrads), c_void_p, ctypes.c_size_t, c_void_p]),
+    "sdm_rt_backward_typed": (ctypes.c_int, [ctypes.POINTER(SdmRtDims), ctypes.POINTER(SdmRtParams),
+                                             c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_i64,
+                                             ctypes.c_int, c_void_p, ctypes.POINTER(SdmRtSaved),
+                                             c_void_p, c_i64, ctypes.c_int, ctypes.POINTER(SdmRtGrads), ctypes.c_int,
+                                             c_void_p, ctypes.c_size_t, c_void_p]),
+    "sdm_rt_weight_grad_workspace_bytes": (ctypes.c_size_t, [c_i64, ctypes.c_int32, ctypes.c_int32]),
+    "sdm_rt_weight_grad": (ctypes.c_int, [c_void_p, c_i64, c_void_p, c_i64, c_i64, ctypes.c_int32, ctypes.c_int32,
+                                          c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
+    "sdm_rt_rms_norm_backward_workspace_bytes": (ctypes.c_size_t, [c_i64, ctypes.c_int32]),
+    "sdm_rt_rms_norm_backward": (ctypes.c_int, [c_void_p, c_i64, ctypes.c_int, c_void_p, c_i64, ctypes.c_int, c_i64,
+                                                ctypes.c_int32, c_void_p, ctypes.c_float, c_void_p, c_i64, c_void_p,
+                                                c_void_p, ctypes.c_size_t, c_void_p]),
+    "sdm_rt_pack_projection": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_int,
+                                              ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+                                              c_void_p, c_void_p, ctypes.c_int, c_void_p]),
     "sdm_rt_table_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(SdmRtDims)]),
     "sdm_rt_table_backward": (ctypes.c_int, [ctypes.POINTER(SdmRtDims), ctypes.POINTER(SdmRtParams),
                                              c_void_p, c_i64, ctypes.c_int,

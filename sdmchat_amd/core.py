@@ -7,6 +7,7 @@ stream; nothing synchronises.
 import ctypes
 
 import torch
+from torch.autograd.function import once_differentiable
 from torch.utils.weak import WeakIdKeyDictionary
 
 from . import _lib
@@ -63,16 +64,17 @@ def _rows2(x, name, B, width):
     return x.stride(0) if B > 1 else max(x.shape[1], width)
 
 
-def _params(device, keys1, keys2, addr_b, log_scale, decay, onorm_w, gate_bias):
+def _params(device, keys1, keys2, addr_b, log_scale, decay, onorm_w, gate_bias, pieces=True):
     """The SdmRtParams of these parameters (float32, contiguous copies where needed) with the sub-key pieces of the
-    bfloat16 scoring prepared from them (sdm_rt_prepare_key_pieces, one launch).  Returns (params, held tensors);
-    build them again after a parameter changes (ParamCache does)."""
+    bfloat16 scoring prepared from them (sdm_rt_prepare_key_pieces, one launch; not with ``pieces`` False, for calls
+    that address nothing).  Returns (params, held tensors); build them again after a parameter changes (ParamCache
+    does)."""
     held = [_f32(t, device) for t in (keys1, keys2, addr_b, log_scale, decay, onorm_w, gate_bias)]
     prm = _lib.SdmRtParams(*[_ptr(t) for t in held])
     H, n_sub, half = held[0].shape
     dims = make_dims(1, 1, H, 8, 2 * half, n_sub, 1)
     lib = _lib.load()
-    nbytes = lib.sdm_rt_key_pieces_bytes(ctypes.byref(dims))
+    nbytes = lib.sdm_rt_key_pieces_bytes(ctypes.byref(dims)) if pieces else 0
     if nbytes:
         pieces = torch.empty(nbytes, dtype=torch.uint8, device=held[0].device)
         stream = torch.cuda.current_stream(pieces.device).cuda_stream
@@ -547,8 +549,7 @@ def rms_norm(x, w, eps=1e-6, out_dtype=None, out=None):
 
 class RmsNormFunction(torch.autograd.Function):
     """rms_norm as an autograd function: the forward on the RMSNorm kernel (the reference's rounding, SM:63-71), the
-    backward of y = x * rsqrt(mean(x^2) + eps) * w in float32 with the casts taken as identities, as autograd takes
-    the reference's ``.to(x.dtype)``.  apply(x, w, eps, out_dtype) -> y."""
+    backward rms_norm_backward.  apply(x, w, eps, out_dtype) -> y."""
 
     @staticmethod
     def forward(ctx, x, w, eps, out_dtype):
@@ -559,14 +560,117 @@ class RmsNormFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
+        dx, dw = rms_norm_backward(x, w, dy, ctx.eps, *ctx.needs_input_grad[:2])
+        return dx, dw, None, None
+
+
+def _aligned(w):
+    """A tensor whose data starts 16-byte aligned and is contiguous, a copy where it is not."""
+    w = w.contiguous()
+    return w if w.data_ptr() % 16 == 0 else w.clone()
+
+
+def rms_norm_backward(x, w, dy, eps, need_x=True, need_w=True):
+    """The gradients of rms_norm(x, w, eps) for dy, the gradient of its output: (dx in x's dtype, dw in w's), None where
+    not needed.  float32 arithmetic with the forward's roundings taken as identities, as autograd takes the reference's
+    ``.to(x.dtype)``; the sum over rows in a fixed order.  On sdm_rt_rms_norm_backward for rows of up to 2,048 values
+    (its row stays in registers), as torch ops past them."""
+    d = x.shape[-1]
+    rows = x.numel() // d if d else 0
+    if not (need_x or need_w):
+        return None, None
+    if rows == 0 or d > 2048 or d % 8 or x.dtype not in _DT or dy.dtype not in _DT:
         xf = x.float()
-        r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + ctx.eps)
+        r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
         n = xf * r
         g = dy.float()
         gw = g * w.float()
-        dx = r * (gw - n * (gw * n).mean(-1, keepdim=True)) if ctx.needs_input_grad[0] else None
-        dw = (g * n).reshape(-1, n.shape[-1]).sum(0) if ctx.needs_input_grad[1] else None
-        return (None if dx is None else dx.to(x.dtype), None if dw is None else dw.to(w.dtype), None, None)
+        dx = r * (gw - n * (gw * n).mean(-1, keepdim=True)) if need_x else None
+        dw = (g * n).reshape(-1, d).sum(0) if need_w else None
+        return None if dx is None else dx.to(x.dtype), None if dw is None else dw.to(w.dtype)
+    x2, dy2 = x.reshape(rows, d), dy.reshape(rows, d)
+    if not _rows16(x2):
+        x2 = _aligned(x2)
+    if not _rows16(dy2):
+        dy2 = _aligned(dy2)
+    dx = torch.empty(x.shape, dtype=x.dtype, device=x.device) if need_x else None
+    wf = _aligned(_f32_weight(w, x.device))
+    dw = torch.empty(d, dtype=torch.float32, device=x.device) if need_w else None
+    lib = _lib.load()
+    nbytes = lib.sdm_rt_rms_norm_backward_workspace_bytes(rows, d) if need_w else 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+    stream = torch.cuda.current_stream(x.device).cuda_stream
+    _lib.check(lib.sdm_rt_rms_norm_backward(_ptr(x2), x2.stride(0), _DT[x.dtype], _ptr(dy2), dy2.stride(0),
+                                            _DT[dy.dtype], rows, d, _ptr(wf), float(eps), _ptr(dx), d, _ptr(dw),
+                                            _ptr(ws), nbytes, ctypes.c_void_p(stream)), lib)
+    return dx, None if dw is None else dw.to(w.dtype)
+
+
+def weight_grad_fits(dy, x):
+    """Whether sdm_rt_weight_grad serves the weight gradient of a map: bfloat16 rows of widths that are multiples of
+    8."""
+    return (dy.is_cuda and dy.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and dy.shape[-1] % 8 == 0
+            and x.shape[-1] % 8 == 0 and dy.numel() > 0 and x.numel() > 0)
+
+
+def weight_grad(dy, x):
+    """dy^T x of rows dy [rows, n] and x [rows, k], bfloat16 (weight_grad_fits): the weight gradient [n, k] of
+    y = x W^T in float32 (sdm_rt_weight_grad: float32 sums in a fixed order)."""
+    lib = _lib.load()
+    rows, n = dy.shape
+    k = x.shape[1]
+    dy = dy if _rows16(dy) else _aligned(dy)
+    x = x if _rows16(x) else _aligned(x)
+    out = torch.empty(n, k, dtype=torch.float32, device=dy.device)
+    nbytes = lib.sdm_rt_weight_grad_workspace_bytes(rows, n, k)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dy.device) if nbytes else None
+    stream = torch.cuda.current_stream(dy.device).cuda_stream
+    _lib.check(lib.sdm_rt_weight_grad(_ptr(dy), dy.stride(0), _ptr(x), x.stride(0), rows, n, k, _ptr(out), _ptr(ws),
+                                      nbytes, ctypes.c_void_p(stream)), lib)
+    return out
+
+
+class LinearFunction(torch.autograd.Function):
+    """F.linear(x, w) under bfloat16 autocast, w any float type, with the weight gradient on sdm_rt_weight_grad: the
+    same product in bfloat16, returned in ``out_dtype``.  The gradient of w stays float32 until it is cast to w's dtype
+    (autocast's own rounds it to bfloat16 on the way).  apply(x, w, out_dtype) -> y."""
+
+    @staticmethod
+    def forward(ctx, x, w, out_dtype):
+        with torch.autocast("cuda", enabled=False):
+            x16, w16 = x.to(torch.bfloat16), w.to(torch.bfloat16)
+            ctx.save_for_backward(x16, w16)
+            ctx.dtypes = (x.dtype, w.dtype)
+            return torch.nn.functional.linear(x16, w16).to(out_dtype)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy):
+        x16, w16 = ctx.saved_tensors
+        with torch.autocast("cuda", enabled=False):
+            dy16 = dy.to(torch.bfloat16)
+            dx = torch.matmul(dy16, w16).to(ctx.dtypes[0]) if ctx.needs_input_grad[0] else None
+            dw = None
+            if ctx.needs_input_grad[1]:
+                d2, x2 = dy16.reshape(-1, dy16.shape[-1]), x16.reshape(-1, x16.shape[-1])
+                dw = (weight_grad(d2, x2) if weight_grad_fits(d2, x2) else torch.matmul(d2.t(), x2)).to(ctx.dtypes[1])
+        return dx, dw, None
+
+
+def autocast_bf16():
+    return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+
+
+def train_linear(lin, x, out_dtype):
+    """lin(x).to(out_dtype) with autograd recording: on LinearFunction under bfloat16 autocast where ``lin`` is a plain
+    nn.Linear without a bias or hooks; else the module itself."""
+    hooks = torch.nn.modules.module
+    if (autocast_bf16() and type(lin) is torch.nn.Linear and lin.bias is None and x.is_cuda and x.dtype in _DT
+            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
+                     or hooks._global_forward_hooks or hooks._global_forward_pre_hooks
+                     or hooks._global_backward_hooks or hooks._global_backward_pre_hooks)):
+        return LinearFunction.apply(x, lin.weight, out_dtype)
+    return lin(x).to(out_dtype)
 
 
 # -- training: forward with saved tensors, backward, and the autograd Function -------------------------------------
@@ -791,8 +895,10 @@ def core_forward_train(kz, qz, v, gate_logits, *, params, k, read_mode="mean", o
 
 
 def core_backward(kz, qz, v, gate_logits, saved, dy, *, params, k, read_mode="mean", out_norm=True, read_eps=1e-3,
-                  out_norm_eps=1e-2, workspace=None):
+                  out_norm_eps=1e-2, workspace=None, rows_out=None):
     """Gradients of the core for dy = d loss / d r (r from core_forward_train with the same inputs and params).
+    rows_out: (kz, qz, v, gate_logits) tensors to write the row gradients into, float32 or bfloat16 (one type for
+    all), each of any uniform row stride; gate_logits None without the gate.
 
     Returns a dict of float32 device tensors: kz, qz [B, T, H * d_a], v [B, T, H * dh], gate_logits [B, T, H] (None
     without the gate), keys1, keys2, addr_b, log_scale, onorm_w (None without the out-norm), gate_bias, log_decay
@@ -816,23 +922,30 @@ def core_backward(kz, qz, v, gate_logits, saved, dy, *, params, k, read_mode="me
     dys = _rows(dy, "dy", B, T, H * dh)
     dev = v.device
     f32 = dict(dtype=torch.float32, device=dev)
-    g = dict(kz=torch.empty(B, T, H * d_a, **f32), qz=torch.empty(B, T, H * d_a, **f32),
-             v=torch.empty(B, T, H * dh, **f32), gate_logits=torch.empty(B, T, H, **f32) if gated else None,
+    if rows_out is None:
+        rows_out = (torch.empty(B, T, H * d_a, **f32), torch.empty(B, T, H * d_a, **f32),
+                    torch.empty(B, T, H * dh, **f32), torch.empty(B, T, H, **f32) if gated else None)
+    strides = [0 if t is None else _rows(t, "rows_out", B, T, w)
+               for t, w in zip(rows_out, (H * d_a, H * d_a, H * dh, H))]
+    gdt = rows_out[0].dtype
+    if any(t is not None and t.dtype != gdt for t in rows_out):
+        raise ValueError("rows_out must share one dtype")
+    g = dict(kz=rows_out[0], qz=rows_out[1], v=rows_out[2], gate_logits=rows_out[3] if gated else None,
              keys1=torch.empty(H, n_sub, half, **f32), keys2=torch.empty(H, n_sub, half, **f32),
              addr_b=torch.empty(H, d_a, **f32), log_scale=torch.empty(H, **f32),
              onorm_w=torch.empty(H, dh, **f32) if out_norm else None, gate_bias=torch.empty(H, **f32),
              log_decay=torch.empty(H, **f32))
-    gr = _lib.SdmRtGrads(_ptr(g["kz"]), H * d_a, _ptr(g["qz"]), H * d_a, _ptr(g["v"]), H * dh,
-                         _ptr(g["gate_logits"]), H, _ptr(g["keys1"]), _ptr(g["keys2"]), _ptr(g["addr_b"]),
+    gr = _lib.SdmRtGrads(_ptr(g["kz"]), strides[0], _ptr(g["qz"]), strides[1], _ptr(g["v"]), strides[2],
+                         _ptr(g["gate_logits"]), strides[3], _ptr(g["keys1"]), _ptr(g["keys2"]), _ptr(g["addr_b"]),
                          _ptr(g["log_scale"]), _ptr(g["onorm_w"]), _ptr(g["gate_bias"]), _ptr(g["log_decay"]))
-    sv = _lib.SdmRtSaved(*[_ptr(saved[n]) for n in ("slots_w", "weights_w", "scores_w", "slots_r", "weights_r",
-                                                    "scores_r", "read", "den")])
+    sv = _lib.SdmRtSaved(*[_ptr(saved[n]) for n in _SAVED])
     nbytes = lib.sdm_rt_backward_workspace_bytes(ctypes.byref(dims))
     ws = (workspace or CoreWorkspace()).get(nbytes, dev)
     stream = torch.cuda.current_stream(dev).cuda_stream
-    rc = lib.sdm_rt_backward(ctypes.byref(dims), ctypes.byref(params[0]), _ptr(kz), ks, _ptr(qz), qs, _ptr(v), vs,
-                             _ptr(gate_logits), gs, _DT[v.dtype], _ptr(saved["reset"]), ctypes.byref(sv), _ptr(dy),
-                             dys, _DT[dy.dtype], ctypes.byref(gr), _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
+    rc = lib.sdm_rt_backward_typed(ctypes.byref(dims), ctypes.byref(params[0]), _ptr(kz), ks, _ptr(qz), qs, _ptr(v),
+                                   vs, _ptr(gate_logits), gs, _DT[v.dtype], _ptr(saved["reset"]), ctypes.byref(sv),
+                                   _ptr(dy), dys, _DT[dy.dtype], ctypes.byref(gr), _DT[gdt], _ptr(ws), ws.numel(),
+                                   ctypes.c_void_p(stream))
     _lib.check(rc, lib)
     return g
 
@@ -875,11 +988,7 @@ class SdmCoreFunction(torch.autograd.Function):
 
         def cast(t, like_dtype, i):
             return t.to(like_dtype) if (t is not None and need[i]) else None
-        d_decay = None
-        if need[8]:
-            lam = decay.detach().to(torch.float32)
-            d_decay = torch.where(lam > 0, g["log_decay"] / torch.where(lam > 0, lam, torch.ones_like(lam)),
-                                  torch.zeros_like(lam)).to(decay.dtype)
+        d_decay = _decay_grad(decay, g["log_decay"]) if need[8] else None
         return (cast(g["kz"], dt, 0), cast(g["qz"], dt, 1), cast(g["v"], dt, 2),
                 cast(g["gate_logits"], dt, 3) if has_g else None,
                 cast(g["keys1"], ctx.dtypes[1], 4), cast(g["keys2"], ctx.dtypes[1], 5),
@@ -887,6 +996,112 @@ class SdmCoreFunction(torch.autograd.Function):
                 cast(g["log_scale"], ctx.dtypes[2], 7), d_decay,
                 cast(g["onorm_w"], ctx.dtypes[1], 9) if has_on else None,
                 cast(g["gate_bias"], ctx.dtypes[1], 10) if has_gb else None, None)
+
+
+_SAVED = ("slots_w", "weights_w", "scores_w", "slots_r", "weights_r", "scores_r", "read", "den")
+
+
+def _decay_grad(decay, log_decay):
+    """d loss / d decay from lam * d loss / d lam (0 at lam = 0)."""
+    lam = decay.detach().to(torch.float32)
+    return torch.where(lam > 0, log_decay / torch.where(lam > 0, lam, torch.ones_like(lam)),
+                       torch.zeros_like(lam)).to(decay.dtype)
+
+
+def mixer_train_fits(x, weights):
+    """Whether MixerFunction serves a training forward: rows of float32 or bfloat16 whose width is a multiple of 8, the
+    projection weights of one type on x's device, run in bfloat16 under bfloat16 autocast or in float32 without
+    autocast on float32 weights.  Returns the compute dtype, or None."""
+    dt = weights[0].dtype
+    if not (x.is_cuda and x.dtype in _DT and x.numel() > 0 and x.shape[-1] % 8 == 0 and dt in _DT
+            and all(w.dtype == dt and w.device == x.device for w in weights)):
+        return None
+    if torch.is_autocast_enabled("cuda"):
+        return torch.bfloat16 if autocast_bf16() else None
+    return torch.float32 if dt == torch.float32 else None
+
+
+class MixerFunction(torch.autograd.Function):
+    """RunTimeSdm's training forward up to wo as one autograd function: the input norm, the two projection maps
+    [wk; wq; wg] and wv (prepare, track4_onesdm_models.py:195-206) and the SDM core, in bfloat16 or float32.
+
+    The backward writes the core's row gradients straight into one [rows, [kz; qz; gate; zeros; v]] buffer in the
+    compute type, so the projections' input gradient and weight gradients are one product each, and the norm's backward
+    takes the product as it is.  Op by op (slices of the maps' outputs, casts, two products each way, their sums) the
+    same step moved every row about thirty times: a training step of the layer at B=8, T=2048 under bfloat16 autocast took
+    1.99 ms that way and takes 1.25 ms (84 launches, now 40).
+
+    apply(x, norm_w, wk, wq, wv, wg, bg, keys1, keys2, addr_b, log_scale, decay, onorm_w, cfg) -> r [B, T, H * dh] in
+    the compute type.  wg and bg may be None (no write gate), onorm_w too.  cfg: dict with dtype (mixer_train_fits),
+    eps, first_rows (the padded rows of the first map), k, read_mode, out_norm, read_eps, out_norm_eps, reset and
+    workspace.  After the call cfg["gate_logits"] holds the gate logits [B, T, H] (a view of the first map's output)."""
+
+    @staticmethod
+    def forward(ctx, x, norm_w, wk, wq, wv, wg, bg, keys1, keys2, addr_b, log_scale, decay, onorm_w, cfg):
+        dt, ra = cfg["dtype"], cfg["first_rows"]
+        B, T, d = x.shape
+        H, za = keys1.shape[0], wk.shape[0]
+        gated = wg is not None
+        with torch.autocast("cuda", enabled=False):
+            hx = rms_norm(x, norm_w, cfg["eps"], out_dtype=dt)
+            W = torch.empty(ra + d, d, dtype=dt, device=x.device)
+            bias = torch.empty(ra + d, dtype=dt, device=x.device) if gated else None
+            ws = [None if w is None else _aligned(w.detach()) for w in (wk, wq, wg, wv)]
+            bgc = None if bg is None else bg.detach().to(ws[0].dtype).contiguous()
+            lib = _lib.load()
+            stream = torch.cuda.current_stream(x.device).cuda_stream
+            _lib.check(lib.sdm_rt_pack_projection(*[_ptr(w) for w in ws], _ptr(bgc), _DT[ws[0].dtype], za, H, ra, d,
+                                                  _ptr(W), _ptr(bias), _DT[dt], ctypes.c_void_p(stream)), lib)
+            pa = torch.nn.functional.linear(hx, W[:ra], None if bias is None else bias[:ra])
+            V = torch.nn.functional.linear(hx, W[ra:])
+            g = pa[..., 2 * za:2 * za + H] if gated else None
+            params = _params(x.device, keys1, keys2, addr_b, log_scale, decay, onorm_w, None)
+            opts = {n: cfg[n] for n in ("k", "read_mode", "out_norm", "read_eps", "out_norm_eps")}
+            r, saved = core_forward_train(pa[..., :za], pa[..., za:2 * za], V, g, params=params, out_dtype=dt,
+                                          reset=cfg["reset"], workspace=cfg["workspace"], **opts)
+        cfg["gate_logits"] = g
+        ctx.opts, ctx.eps, ctx.workspace, ctx.shape = opts, cfg["eps"], cfg["workspace"], (ra, za, gated)
+        ctx.dtypes = [None if t is None else t.dtype for t in (wk, wq, wv, wg, bg)]
+        ctx.save_for_backward(x, norm_w, hx, W, pa, V, keys1, keys2, addr_b, log_scale, decay, onorm_w,
+                              saved["reset"], *[saved[n] for n in _SAVED])
+        return r
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dr):
+        (x, norm_w, hx, W, pa, V, keys1, keys2, addr_b, log_scale, decay, onorm_w, reset), rest = \
+            ctx.saved_tensors[:13], ctx.saved_tensors[13:]
+        saved = dict(zip(_SAVED, rest), reset=reset)
+        ra, za, gated = ctx.shape
+        B, T, d = x.shape
+        H = keys1.shape[0]
+        need = ctx.needs_input_grad
+        with torch.autocast("cuda", enabled=False):
+            params = _params(x.device, keys1, keys2, addr_b, log_scale, decay, onorm_w, None, pieces=False)
+            dp = torch.empty(B, T, ra + d, dtype=pa.dtype, device=x.device)
+            g = pa[..., 2 * za:2 * za + H] if gated else None
+            live = 2 * za + (H if gated else 0)
+            if live < ra:
+                dp[..., live:ra].zero_()
+            gr = core_backward(pa[..., :za], pa[..., za:2 * za], V, g, saved, dr, params=params,
+                               workspace=ctx.workspace, rows_out=(dp[..., :za], dp[..., za:2 * za], dp[..., ra:],
+                                                                  dp[..., 2 * za:live] if gated else None), **ctx.opts)
+            dx = dnw = None
+            if need[0] or need[1]:
+                dx, dnw = rms_norm_backward(x, norm_w, torch.matmul(dp, W), ctx.eps, need[0], need[1])
+            dws = [None] * 4
+            if any(need[2:6]):
+                d2, h2 = dp.view(B * T, ra + d), hx.view(B * T, d)
+                dW = weight_grad(d2, h2) if weight_grad_fits(d2, h2) else torch.matmul(d2.t(), h2)
+                parts = (dW[:za], dW[za:2 * za], dW[ra:], dW[2 * za:live] if gated else None)
+                dws = [t.to(ctx.dtypes[i]) if t is not None and need[2 + i] else None for i, t in enumerate(parts)]
+
+            def cast(n, like, i):
+                return gr[n].to(like.dtype) if like is not None and need[i] else None
+            return (dx, dnw, *dws, gr["gate_bias"].to(ctx.dtypes[4]) if gated and need[6] else None,
+                    cast("keys1", keys1, 7), cast("keys2", keys2, 8), cast("addr_b", addr_b, 9),
+                    cast("log_scale", log_scale, 10), _decay_grad(decay, gr["log_decay"]) if need[11] else None,
+                    cast("onorm_w", onorm_w, 12), None)
 
 
 def table_backward(q, slots, weights, scores, values, dy, *, k, params, workspace=None):
@@ -931,8 +1146,8 @@ class TableSdmFunction(torch.autograd.Function):
     sdm_rt_table_read, backward sdm_rt_table_backward.
 
     apply(q, keys1, keys2, log_scale, values, cfg) -> r float32 [B, T, H * dh]; q [B, T, H * d_a] float32 or
-    bfloat16; cfg: dict with k and optionally workspace.  After the call cfg["slots"] holds the picks
-    [B, H, T, pitch].  The picks carry no gradient (as topk in the reference)."""
+    bfloat16; cfg: dict with k and optionally workspace and out_dtype (r's, float32 by default).  After the call
+    cfg["slots"] holds the picks [B, H, T, pitch].  The picks carry no gradient (as topk in the reference)."""
 
     @staticmethod
     def forward(ctx, q, keys1, keys2, log_scale, values, cfg):
@@ -940,7 +1155,7 @@ class TableSdmFunction(torch.autograd.Function):
             raise RuntimeError("the table layer needs ROCm device tensors")
         params = _params(q.device, keys1, keys2, None, log_scale, None, None, None)
         slots, scores, weights = address(q, keys1, keys2, cfg["k"], log_scale, padded=True, params=params)
-        r = table_read(slots, weights, values, cfg["k"], out_dtype=torch.float32)
+        r = table_read(slots, weights, values, cfg["k"], out_dtype=cfg.get("out_dtype", torch.float32))
         cfg["slots"] = slots
         ctx.k = cfg["k"]
         ctx.params = params

@@ -21,6 +21,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "sdm_reduce.h"
 #include "sdm_scan.h"
 
 namespace sdmrt {
@@ -328,8 +329,9 @@ struct GradScanArgs {
   const uint8_t* reset;    // [B*T] or nullptr
   const float* decay;      // [H]
   float* dot_out;          // [dh / CW][B][H][T][KP] per-pick dots of this column group (count term in group 0)
-  float* sum_out;          // rows of H * dh float32 (weighted sums of the rows read), or nullptr
+  void* sum_out;           // rows of H * dh (weighted sums of the rows read; float32, bfloat16 with sum_bf16), or nullptr
   int64_t sum_stride;
+  int sum_bf16;
   const unsigned char* chains;   // [B][H][n_chunks][chain_stride(KP)] chain plans of the writes (chain_plan_kernel)
   int B, T, H, dh, M, kk, n_chunks;
 };
@@ -698,7 +700,9 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
         dot_out[static_cast<int64_t>(t) * KP + i] = i < kk ? dot[o] : 0.f;
       }
       if (a.sum_out) {
-        store_vals<CPL, float>(a.sum_out + n * a.sum_stride + static_cast<int64_t>(h) * a.dh + col0 + CPL * l8, sum);
+        const int64_t at = n * a.sum_stride + static_cast<int64_t>(h) * a.dh + col0 + CPL * l8;
+        if (a.sum_bf16) store_vals<CPL, bf16_t>(static_cast<bf16_t*>(a.sum_out) + at, sum);
+        else store_vals<CPL, float>(static_cast<float*>(a.sum_out) + at, sum);
       }
     }
     lds_barrier();
@@ -814,10 +818,11 @@ struct AddrGradArgs {
   const float* score[2];
   const float* dot[2];       // [CG][B][H][T][KP] per-pick gradient partials: dww, dwr
   int n_cg;
-  float* dz[2];              // rows of H * d_a float32: d kz, d qz
+  void* dz[2];               // rows of H * d_a: d kz, d qz (float32; bfloat16 with out_bf16, as dgl)
   int64_t dz_stride[2];
-  float* dgl;                // rows of H float32 or nullptr
+  void* dgl;                 // rows of H or nullptr
   int64_t dgl_stride;
+  int out_bf16;
   float* part_f;             // [n_blk][2][H][2 + d_a]: dtau, d gate bias, d addr_b
   double* part_d;            // [n_blk][2][H]: lam dL/dlam
   float* part_k;             // [n_blk][2][H][2][n_sub][HALF]: d unit sub-keys
@@ -826,6 +831,12 @@ struct AddrGradArgs {
   int wave_tokens;           // tokens per wave (addr_grad_tile_kernel: a multiple of its 32-token tile)
 };
 
+
+// an input gradient in the caller's type
+__device__ __forceinline__ void store_grad(void* p, int64_t i, float v, int as_bf16) {
+  if (as_bf16) static_cast<bf16_t*>(p)[i] = from_f32<bf16_t>(v);
+  else static_cast<float*>(p)[i] = v;
+}
 
 __device__ __forceinline__ float lane_f(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
@@ -941,7 +952,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
   const float* wtp = a.wt[set];
   const float* scp = a.score[set];
   const float* dotp = a.dot[set];
-  float* dzp = a.dz[set];
+  void* dzp = a.dz[set];
   const int64_t dzs = a.dz_stride[set];
   const bool pl = e < kk;                 // the lane holds a live pick
   float acc_tau = 0.f, acc_gb = 0.f, acc_ab = 0.f;
@@ -1010,7 +1021,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
       dx = pj * (gt * dw - S);
       if (gated) {
         const float dlogit = dg * gt * (1.f - gt);
-        if (e == 0 && a.dgl) a.dgl[n * a.dgl_stride + h] = dlogit;
+        if (e == 0 && a.dgl) store_grad(a.dgl, n * a.dgl_stride + h, dlogit, a.out_bf16);
         acc_gb += e == 0 ? dlogit : 0.f;
       }
     }
@@ -1042,7 +1053,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
     }
     const float ud = half_sum<HALF>(u * du, e);
     const float dz = nz > 1e-12f ? (du - u * ud) * inz : du * 1e12f;
-    if (e < DA) dzp[n * dzs + static_cast<int64_t>(h) * DA + e] = dz;
+    if (e < DA) store_grad(dzp, n * dzs + static_cast<int64_t>(h) * DA + e, dz, a.out_bf16);
     acc_ab += dz;
     cur = nxt;
     n = n2;
@@ -1193,7 +1204,6 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
   const float* wtp = a.wt[set];
   const float* scp = a.score[set];
   const float* dotp = a.dot[set];
-  float* dzp = a.dz[set] + static_cast<int64_t>(h) * DA;
   const int dzs = static_cast<int>(a.dz_stride[set]);
   const bool live_col = NT == 2 ? col < HALF : col < DA;
   const int64_t N = static_cast<int64_t>(a.B) * a.T;   // below 2^31: each token has picks of 4 * 32 bytes and more
@@ -1241,7 +1251,9 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
         const int row = 8 * (r / 4) + 4 * hw + r % 4;
         zr[p][r] = zt[(row < left ? row : 0) * zs + (live_col ? p * HALF + col : 0)];
       }
-    float* dzt = dzp + n0 * dzs;
+    const int64_t dz0 = n0 * a.dz_stride[set] + static_cast<int64_t>(h) * DA;   // the tile's first output value
+    float* dzt = static_cast<float*>(a.dz[set]) + dz0;
+    bf16_t* dzb = static_cast<bf16_t*>(a.dz[set]) + dz0;
     // G to zero, then the picks' gradients
 #pragma unroll
     for (int k = 0; k < (kAddrTile * GP + 255) / 256; ++k) {
@@ -1276,7 +1288,7 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
         dx = pr * (gt * dw - S);
         if (gated && valid && pj == 0) {
           const float dlogit = dg * gt * (1.f - gt);
-          if (a.dgl) a.dgl[(n0 + it * TPI + lane / KP) * a.dgl_stride + h] = dlogit;
+          if (a.dgl) store_grad(a.dgl, (n0 + it * TPI + lane / KP) * a.dgl_stride + h, dlogit, a.out_bf16);
           acc_gb += dlogit;
         }
       }
@@ -1355,7 +1367,9 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
         const float ud = col_sum<HALF>(u[r] * du[r], col);
         const float dz = nz[r] > 1e-12f ? (du[r] - u[r] * ud) * inz[r] : du[r] * 1e12f;
         if (live_col && row < left) {
-          dzt[row * dzs + p * HALF + col] = dz;
+          const int at = row * dzs + p * HALF + col;
+          if (a.out_bf16) dzb[at] = from_f32<bf16_t>(dz);
+          else dzt[at] = dz;
           acc_ab[p] += dz;
         }
       }
@@ -1415,42 +1429,6 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
     float s = 0.f;
     for (int q = 0; q < kAddrTileWaves; ++q) s += dkb[q * KS + i];
     a.part_k[pid * KS + i] = s;
-  }
-}
-
-// Sums over records: out[i] = sum_r part[r * rec_stride + i] (r < n_rec) in float64 for n_items items.  Block of
-// 64 x 16 threads: lane i of group rg sums records rg, rg + 16, ... (loads issued together), then the 16 group sums
-// are added in group order: a fixed order, so the result is deterministic.
-constexpr int kRedGroups = 16;
-
-template <typename T>
-__global__ void __launch_bounds__(64 * kRedGroups) reduce_records_kernel(const T* __restrict__ part, int n_rec,
-                                                                        int64_t rec_stride, int64_t n_items,
-                                                                        double* __restrict__ out) {
-  __shared__ double red[kRedGroups][64];
-  const int l = threadIdx.x & 63;
-  const int rg = threadIdx.x >> 6;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + l;
-  double s = 0.0;
-  if (i < n_items) {
-    constexpr int kBatch = 16;
-    for (int r0 = rg; r0 < n_rec; r0 += kRedGroups * kBatch) {
-      T v[kBatch];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int r = r0 + q * kRedGroups;
-        v[q] = r < n_rec ? part[static_cast<int64_t>(r) * rec_stride + i] : T(0);
-      }
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) s += static_cast<double>(v[q]);
-    }
-  }
-  red[rg][l] = s;
-  __syncthreads();
-  if (rg == 0 && i < n_items) {
-    double t = 0.0;
-    for (int q = 0; q < kRedGroups; ++q) t += red[q][l];
-    out[i] = t;
   }
 }
 
@@ -1947,6 +1925,17 @@ int sdm_rt_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, const 
                     const void* gate_logits, int64_t gate_row_stride, sdm_rt_dtype in_dtype, const uint8_t* reset,
                     const sdm_rt_saved* saved, const void* dy, int64_t dy_row_stride, sdm_rt_dtype dy_dtype,
                     const sdm_rt_grads* grads, void* workspace, size_t workspace_bytes, void* stream) {
+  return sdm_rt_backward_typed(dims, params, kz, kz_row_stride, qz, qz_row_stride, v, v_row_stride, gate_logits,
+                               gate_row_stride, in_dtype, reset, saved, dy, dy_row_stride, dy_dtype, grads, SDM_RT_F32,
+                               workspace, workspace_bytes, stream);
+}
+
+int sdm_rt_backward_typed(const sdm_rt_dims* dims, const sdm_rt_params* params, const void* kz, int64_t kz_row_stride,
+                          const void* qz, int64_t qz_row_stride, const void* v, int64_t v_row_stride,
+                          const void* gate_logits, int64_t gate_row_stride, sdm_rt_dtype in_dtype,
+                          const uint8_t* reset, const sdm_rt_saved* saved, const void* dy, int64_t dy_row_stride,
+                          sdm_rt_dtype dy_dtype, const sdm_rt_grads* grads, sdm_rt_dtype grad_dtype, void* workspace,
+                          size_t workspace_bytes, void* stream) {
   g_err[0] = 0;
   GradPlan g;
   int rc = make_grad_plan(dims, &g);
@@ -1955,6 +1944,7 @@ int sdm_rt_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, const 
   if ((rc = check_params(params, dims->out_norm != 0))) return rc;
   if ((rc = check_dtype(in_dtype, "in_dtype"))) return rc;
   if ((rc = check_dtype(dy_dtype, "dy_dtype"))) return rc;
+  if ((rc = check_dtype(grad_dtype, "grad_dtype"))) return rc;
   if (!grads) return set_err(SDM_RT_EINVAL, "grads is NULL");
   if (p.B == 0 || p.T == 0) return SDM_RT_OK;
   if ((rc = check_saved(saved, dims->read_mean != 0))) return rc;
@@ -2050,6 +2040,7 @@ int sdm_rt_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, const 
     a.dot_out = dotw;
     a.sum_out = grads->d_v;
     a.sum_stride = grads->d_v_row_stride;
+    a.sum_bf16 = grad_dtype == SDM_RT_BF16;
     a.B = p.B;
     a.T = p.T;
     a.H = p.H;
@@ -2091,6 +2082,7 @@ int sdm_rt_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, const 
     a.dz_stride[1] = grads->d_qz_row_stride;
     a.dgl = dims->write_gate ? grads->d_gate_logits : nullptr;
     a.dgl_stride = grads->d_gate_row_stride;
+    a.out_bf16 = grad_dtype == SDM_RT_BF16;
     a.part_f = pf;
     a.part_d = pd;
     a.part_k = pk;

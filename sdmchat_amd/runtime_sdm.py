@@ -208,15 +208,26 @@ class RunTimeSdm(nn.Module):
         return pa[..., :o_q], pa[..., o_q:o_g], V, g
 
     def _forward_train(self, x, reset):
-        """The differentiable forward: _project_train, the core through SdmCoreFunction, finish's wo (:247)."""
+        """The differentiable forward: the norm, the projections and the core through MixerFunction (or, where it does
+        not serve the types, _project_train and SdmCoreFunction), then finish's wo (:247)."""
         B, T, _ = x.shape
         H = self.h
-        kz, qz, V, g = self._project_train(x)
         cfg = dict(k=self.k, read_mode=self.read_mode, out_norm=self.out_norm, read_eps=self.read_eps,
                    out_norm_eps=self.out_norm_eps, reset=reset, workspace=self._ws)
-        r = core.SdmCoreFunction.apply(kz, qz, V, g, self.keys1, self.keys2, self.addr_b, self.log_scale,
-                                       self.decay(), self.onorm_w if self.out_norm else None, None, cfg)
-        y = self.wo(r).to(x.dtype)
+        onorm_w = self.onorm_w if self.out_norm else None
+        gate = (self.wg.weight, self.wg.bias) if self.write_gate else (None, None)
+        weights = [self.wk.weight, self.wq.weight, self.wv.weight] + ([gate[0]] if self.write_gate else [])
+        dt = core.mixer_train_fits(x, weights)
+        if dt is not None:
+            cfg.update(dtype=dt, eps=self.norm.eps, first_rows=self._rows_a())
+            r = core.MixerFunction.apply(grad_scale(x, self.mem_in_grad), self.norm.w, *weights[:3], *gate, self.keys1,
+                                         self.keys2, self.addr_b, self.log_scale, self.decay(), onorm_w, cfg)
+            g = cfg["gate_logits"]
+        else:
+            kz, qz, V, g = self._project_train(x)
+            r = core.SdmCoreFunction.apply(kz, qz, V, g, self.keys1, self.keys2, self.addr_b, self.log_scale,
+                                           self.decay(), onorm_w, None, cfg)
+        y = core.train_linear(self.wo, r, x.dtype)
         self._gate_src = (g.detach().contiguous() if g is not None else None, None, (B, T, H), x.device)
         self._last_gate = None
         self._last_state, self._state_skipped = None, False

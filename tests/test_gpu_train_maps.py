@@ -1,0 +1,127 @@
+"""GPU parity of the dense parts of a training step: sdm_rt_weight_grad, sdm_rt_rms_norm_backward and
+core.MixerFunction, against float64 on the same values and against the op-by-op training path.
+"""
+import math
+
+import pytest
+import torch
+
+from sdmchat_amd import RunTimeSdm, TrainedSdm, core
+from tests._gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (1, 8, 8), (63, 136, 24), (64, 128, 128), (65, 40, 264),        # a step's edge, narrow tiles
+    (255, 256, 256), (257, 264, 256), (12289, 264, 512),            # 256-wide tiles, their remainders, several splits
+    (16384, 768, 768), (4000, 32, 768),
+])
+def test_weight_grad_matches_float64(rows, n, k):
+    """Every output within the bound of a float32 sum of its products in any order: rows * 2^-24 times the sum of their
+    magnitudes."""
+    say(f"[weight grad] rows={rows} n={n} k={k}")
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    wide = torch.randn(rows, n + 8, generator=g, device="cuda").bfloat16()   # a row stride of its own
+    dy, x = wide[:, 8:], torch.randn(rows, k, generator=g, device="cuda").bfloat16()
+    got = core.weight_grad(dy, x).double()
+    ref = dy.double().t() @ x.double()
+    bound = (rows + 1) * 2.0 ** -24 * (dy.double().abs().t() @ x.double().abs())
+    assert bool(((got - ref).abs() <= bound).all())
+    assert torch.equal(core.weight_grad(dy, x).double(), got)
+
+
+def test_weight_grad_takes_unaligned_rows():
+    g = torch.Generator(device="cuda").manual_seed(1)
+    dy = torch.randn(70, 41, generator=g, device="cuda").bfloat16()[:, 1:]
+    x = torch.randn(70, 24, generator=g, device="cuda").bfloat16()
+    assert torch.equal(core.weight_grad(dy, x), core.weight_grad(dy.contiguous(), x))
+
+
+@pytest.mark.parametrize("rows,d", [(1, 8), (7, 64), (9, 256), (33, 264), (4100, 768), (5, 1160), (3, 2048), (2, 2056)])
+@pytest.mark.parametrize("xt,yt", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                   (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+def test_rms_norm_backward_matches_float64(rows, d, xt, yt):
+    """float32 arithmetic on up to 2,048 values a row: 1e-5 of the largest entry (d * 2^-24 = 1.2e-4 would be the worst
+    case of every rounding alike), dx in bfloat16 plus half its ulp."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x = torch.randn(rows, d, generator=g, device="cuda").to(xt)
+    w = 1 + 0.3 * torch.randn(d, generator=g, device="cuda")
+    dy = torch.randn(rows, d, generator=g, device="cuda").to(yt)
+    dx, dw = core.rms_norm_backward(x, w, dy, 1e-6)
+    x64, w64 = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    (x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + 1e-6) * w64).backward(dy.double())
+    tol = 1e-5 * x64.grad.abs().max() + (2.0 ** -8 * x64.grad.abs() if xt == torch.bfloat16 else 0.0)
+    assert dx.dtype == xt and bool(((dx.double() - x64.grad).abs() <= tol).all())
+    assert (dw.double() - w64.grad).abs().max() <= 1e-5 * w64.grad.abs().max()
+    assert core.rms_norm_backward(x, w, dy, 1e-6, need_w=False)[1] is None
+    assert torch.equal(core.rms_norm_backward(x, w, dy, 1e-6, need_x=False)[1], dw)
+
+
+@pytest.mark.parametrize("amp,gate,reset,frozen", [
+    (True, True, False, ()), (False, True, True, ()), (True, False, True, ("wk", "norm")), (False, False, False, ("wv",)),
+])
+def test_mixer_function_equals_the_op_by_op_path(amp, gate, reset, frozen):
+    """The same forward bits; gradients within the compute type's rounding: each side rounds the projections' input
+    gradient (and, op by op, each weight gradient) once or twice more, 2^-8 of a value in bfloat16, so 2e-2 of the
+    largest entry there and 1e-5 in float32."""
+    torch.manual_seed(3)
+    B, T, d, H = 3, 130, 96, 4
+    m = RunTimeSdm(d, heads=H, n_sub=8, d_a=16, k=8, decays=(0.6, 0.8, 0.95, 0.99), learn_decay=True, write_gate=gate,
+                   addr_bias=0.2, mem_in_grad=0.5).to("cuda").train()
+    for n, p in m.named_parameters():
+        if n.split(".")[0] in frozen:
+            p.requires_grad_(False)
+    x = torch.randn(B, d, T, device="cuda").transpose(1, 2)   # not contiguous
+    rs = torch.rand(B, T, device="cuda") < 0.05 if reset else None
+    dy = torch.randn(B, T, d, device="cuda")
+
+    def step(fits):
+        keep, core.mixer_train_fits = core.mixer_train_fits, fits or core.mixer_train_fits
+        try:
+            xg = x.detach().clone().requires_grad_(True)
+            with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+                y = m(xg, rs)
+            ps = {n: p for n, p in m.named_parameters() if p.requires_grad}
+            gs = torch.autograd.grad(y, [xg] + list(ps.values()), dy, allow_unused=True)
+            return y, dict(zip(["x"] + list(ps), gs)), m.last_gate
+        finally:
+            core.mixer_train_fits = keep
+    y1, g1, gate1 = step(None)
+    y0, g0, gate0 = step(lambda *a: None)
+    assert torch.equal(y1, y0) and torch.equal(gate1, gate0)
+    for n in g0:
+        assert (g0[n] is None) == (g1[n] is None), n
+        if g0[n] is None:
+            continue
+        assert g1[n].dtype == g0[n].dtype and g1[n].shape == g0[n].shape, n
+        err = (g1[n] - g0[n]).abs().max().item()
+        scale = g0[n].abs().max().item()
+        say(f"  d{n}: {err:.2e} of {scale:.2e}")
+        assert err <= (2e-2 if amp else 1e-5) * max(scale, 1e-2), n
+
+
+def test_hooks_on_the_output_map_still_run():
+    m = RunTimeSdm(64, heads=2, n_sub=8, d_a=16, k=4, decays=(0.5, 0.9)).to("cuda").train()
+    t = TrainedSdm(64, 8, heads=2, d_a=8, k=4).to("cuda").train()
+    seen = []
+    hooks = [mod.wo.register_forward_hook(lambda *a: seen.append(1)) for mod in (m, t)]
+    x = torch.randn(2, 40, 64, device="cuda", requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        (m(x) + t(x)).float().sum().backward()
+    assert len(seen) == 2 and bool(torch.isfinite(x.grad).all())
+    for h in hooks:
+        h.remove()
+
+
+def test_offloaded_saved_tensors_give_the_same_gradients():
+    """Saved-tensor hooks see every tensor the mixer keeps: gradients from tensors offloaded to the host and back."""
+    m = RunTimeSdm(64, heads=2, n_sub=8, d_a=16, k=4, decays=(0.5, 0.9)).to("cuda").train()
+    x = torch.randn(2, 70, 64, device="cuda", requires_grad=True)
+    torch.nn.init.xavier_uniform_(m.wo.weight)
+    grads = []
+    for off in (False, True):
+        with torch.autograd.graph.saved_tensors_hooks(lambda v: v.cpu() if off else v, lambda v: v.cuda()):
+            y = m(x)
+        grads.append(torch.autograd.grad(y.square().sum(), [x] + list(m.parameters())))
+    assert all(torch.equal(a, b) for a, b in zip(*grads)) and math.isfinite(grads[0][0].sum().item())
