@@ -168,13 +168,26 @@ __global__ void __launch_bounds__(256) read_grad_kernel(const DyT* __restrict__ 
 // ---------------------------------------------------------------------------------------------------------------
 // chain plan: the write side of one chunk of a grad scan, built in parallel before the scan (the write records of the
 // forward plan, for the picks the forward kept).  Per (chunk, head, batch row), stride chain_stride(KP) bytes:
-//   u32 {n_rec, n_ext, 0, 0}
+//   u32 {n_rec, n_ext, reset mask lo, hi}   (the mask of the chunk's positions that empty the memory before they read)
 //   wrec[64][KP]   uint2 {slot | q0 << 16 | xo << 22, c0 | more << 31}: the distinct slots the chunk's kept writers
 //                  write, record u at [u % 64][u / 64] (group g applies records g, g + 64, ...); q0 the slot's first
 //                  kept writer, c0 = lam^(L-1-q0) w; with more, its later writers are ext[xo], ext[xo + 1], ... up to
 //                  the one flagged last.  Unused entries are null records {M, 0}.
 //   ext[64 * KP]   uint2 {c = lam^(L-1-q) w, q | last << 31}
 __host__ __device__ constexpr int chain_stride(int KP) { return (16 + 2 * 64 * KP * 8 + 255) / 256 * 256; }
+
+// Position p of chunk c of a scan in either direction: the chunks are those of 64 tokens from the sequence's start, the
+// reverse scan takes them from the last (which may be short) and each from its last token, so both directions agree
+// on which pairs of positions share a chunk.
+template <bool REV>
+struct ChunkSpan {
+  int L, base;   // live positions; the chunk's first token
+  __device__ __forceinline__ ChunkSpan(int c, int T, int n_chunks) {
+    base = (REV ? n_chunks - 1 - c : c) * kChunk;
+    L = min(kChunk, T - base);
+  }
+  __device__ __forceinline__ int token(int p) const { return base + (p < L ? (REV ? L - 1 - p : p) : 0); }
+};
 
 struct ChainArgs {
   const int32_t* w_slot;   // [B][H][T][KP] write picks
@@ -199,10 +212,10 @@ __global__ void __launch_bounds__(64) chain_plan_kernel(ChainArgs a) {
   const int M = a.M;
   const int kk = a.kk;
   const int T = a.T;
-  const int u0 = c * kChunk;
-  const int L = min(kChunk, T - u0);
+  const ChunkSpan<REV> span(c, T, a.n_chunks);
+  const int L = span.L;
   const bool valid = p < L;
-  const int t = valid ? (REV ? T - 1 - (u0 + p) : u0 + p) : 0;
+  const int t = span.token(p);
   const int64_t prow = ((static_cast<int64_t>(b) * a.H + h) * T + t) * KP;
   const float lam = a.decay[h];
   {
@@ -223,7 +236,8 @@ __global__ void __launch_bounds__(64) chain_plan_kernel(ChainArgs a) {
     slr[j] = a.w_slot[prow + j];
     wr[j] = a.w_wt[prow + j];
   }
-  const int64_t ri = static_cast<int64_t>(b) * T + (REV ? (valid && u0 + p >= 1 ? T - (u0 + p) : 0) : t);
+  const bool has = valid && a.reset && (REV ? t + 1 < T : true);   // backwards, a reset at t + 1 separates t from it
+  const int64_t ri = static_cast<int64_t>(b) * T + (has ? (REV ? t + 1 : t) : 0);
   const uint8_t rv8 = *(a.reset ? a.reset + ri : reinterpret_cast<const uint8_t*>(a.decay));
 #pragma unroll
   for (int j = 0; j < KP; ++j) {
@@ -231,7 +245,7 @@ __global__ void __launch_bounds__(64) chain_plan_kernel(ChainArgs a) {
     s_sl[p][j] = live ? ((slr[j] >= 0 && slr[j] < M) ? slr[j] : 0) : -1;
     s_w[p][j] = live ? wr[j] : 0.f;
   }
-  const bool rf = valid && a.reset && (REV ? u0 + p >= 1 : true) && rv8 != 0;
+  const bool rf = has && rv8 != 0;
   const unsigned long long rmask = __ballot(rf);
   const int last = rmask ? 63 - __builtin_clzll(rmask) : -1;   // writers before the chunk's last reset do not reach
   const unsigned long long keep = last >= 0 ? ~((1ull << last) - 1ull) : ~0ull;   // the state
@@ -283,7 +297,9 @@ __global__ void __launch_bounds__(64) chain_plan_kernel(ChainArgs a) {
   unsigned char* plan = a.chains + ((static_cast<int64_t>(b) * a.H + h) * a.n_chunks + c) * chain_stride(KP);
   uint2* wrec = reinterpret_cast<uint2*>(plan + 16);
   uint2* ext = wrec + kChunk * KP;
-  if (p == 0) *reinterpret_cast<uint4*>(plan) = make_uint4(n_rec, n_ext, 0u, 0u);
+  if (p == 0)
+    *reinterpret_cast<uint4*>(plan) =
+        make_uint4(n_rec, n_ext, static_cast<uint32_t>(rmask), static_cast<uint32_t>(rmask >> 32));
 #pragma unroll
   for (int k = 0; k < KP; ++k)
     if (p + kChunk * k >= n_rec) wrec[p * KP + k] = make_uint2(static_cast<uint32_t>(M), 0u);
@@ -314,26 +330,32 @@ __global__ void __launch_bounds__(64) chain_plan_kernel(ChainArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// grad_scan_kernel: the per-pick scan (see the top of this file)
+// grad_scan_kernel: the per-pick scan over the carried memory (see the top of this file); what a chunk's positions
+// read of the chunk's own writes is chunk_grad_kernel's
 struct GradScanArgs {
-  const int32_t* w_slot;   // [B][H][T][KP] write picks (entries >= kk ignored)
-  const float* w_wt;       //   and weights
-  const int32_t* r_slot;   // [B][H][T][KP] read picks
-  const float* r_wt;
+  const int32_t* r_slot;   // [B][H][T][KP] read picks (entries >= kk ignored)
+  const float* r_wt;       //   and weights
   const void* wv;          // write value rows (H * dh per row), type WT
   int64_t wv_stride;
   const float* wc;         // [B*T][H] write count factors, or nullptr for 1
   const void* rv;          // read vector rows, type RT
   int64_t rv_stride;
   const float* rc;         // [B*T][H] read count factors, or nullptr for 1
-  const uint8_t* reset;    // [B*T] or nullptr
   const float* decay;      // [H]
   float* dot_out;          // [dh / CW][B][H][T][KP] per-pick dots of this column group (count term in group 0)
+  const float* sum_in;     // rows of H * dh added to the sums (chunk_grad_kernel's part); with sum_out
   void* sum_out;           // rows of H * dh (weighted sums of the rows read; float32, bfloat16 with sum_bf16), or nullptr
   int64_t sum_stride;
   int sum_bf16;
   const unsigned char* chains;   // [B][H][n_chunks][chain_stride(KP)] chain plans of the writes (chain_plan_kernel)
   int B, T, H, dh, M, kk, n_chunks;
+  int vec;                 // the picks, rows and sums are aligned for one load per lane's piece
+};
+
+// CPL elements of a row as one load brings them
+template <typename T, int CPL>
+struct alignas(sizeof(T) * CPL) RawSeg {
+  T e[CPL];
 };
 
 // chain entries a grad_scan stages in LDS (the rest are read from the chain plan in global memory); typical chunks
@@ -342,23 +364,19 @@ __host__ __device__ constexpr int grad_ext_stage(int KP) { return KP <= 8 ? 64 *
 
 __host__ __device__ constexpr size_t align16(size_t x) { return (x + 15) / 16 * 16; }
 
-// LDS of one grad_scan workgroup: writer masks wmask[M] (u64), slab A[M + 1][CW] and counts cnt[M + 1] (row M stays
-// zero: null write records read it and write nothing), the chunk's write picks s_ws[64][KP] and weights
-// s_ww[64][KP], write values s_wv[64][CW], count factors s_wc[64], fade powers pw[68], the chunk's reset mask and its
-// staged chain entries
+// LDS of one grad_scan workgroup: slab A[M + 1][CW] and counts cnt[M + 1] (row M stays zero: null write records read
+// it and write nothing), the chunk's write values s_wv[64][CW], count factors s_wc[64], fade powers pw[68], write
+// records s_rec[64][KP] and staged chain entries
 struct GradScanLds {
-  size_t wmask, A, cnt, ws, ww, wv, wc, pw, rm, ext, total;
+  size_t A, cnt, wv, wc, pw, rec, ext, total;
   __host__ __device__ constexpr GradScanLds(int M, int KP, int CW)
-      : wmask(0),
-        A(align16(8 * static_cast<size_t>(M))),
-        cnt(A + align16(4 * static_cast<size_t>(M + 1) * CW)),
-        ws(cnt + align16(4 * static_cast<size_t>(M + 1))),
-        ww(ws + 4 * 64 * KP),
-        wv(ww + 4 * 64 * KP),
+      : A(0),
+        cnt(align16(4 * static_cast<size_t>(M + 1) * CW)),
+        wv(cnt + align16(4 * static_cast<size_t>(M + 1))),
         wc(wv + 4 * 64 * CW),
         pw(wc + 4 * 64),
-        rm(pw + 4 * 68),
-        ext(rm + 16),
+        rec(pw + 4 * 68),
+        ext(rec + 8 * 64 * KP),
         total(ext + grad_ext_stage(KP)) {}
 };
 
@@ -418,32 +436,219 @@ __device__ __forceinline__ unsigned long long group_or8(unsigned long long v) {
   return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
+// What a chunk's positions read of the chunk's own writes, for both directions at once: with X[t][s] = <dnum_t, V_s> +
+// dden_t and c[t][s] = lam^(t-1-s) for s < t of one chunk and one segment,
+//   dwr[t,i] += sum_s c ww[s,j] [match] X,  dww[s,j] += sum_t c wr[t,i] [match] X,
+//   dV_s      = sum_t c (sum_ij wr[t,i] ww[s,j] [match]) dnum_t
+// None of it needs the carried memory, so it runs over all chunks in parallel instead of inside the two scans, whose
+// chunks form a chain of 32 steps (B=8, T=2048) on 192 of the 256 compute units: there these loops were two fifths of
+// each scan.  B=8, T=2048, 12 heads, k=8, bfloat16: the scans 211 + 209 -> 132 + 143 us, this kernel 53 us; k=16
+// float32 (B=5, T=301, 4 heads): 114 + 116 -> 53 + 74, this kernel 19 us.
+// Block (chunk, head x group of 64 columns, batch row), 512 threads = 64 positions x 8 lanes of 8 columns.  Each slot's
+// writers (then its readers) of the chunk are a 64-bit mask in LDS; a position's lanes walk the union of their picks'
+// masks together, in position order (a fixed order), only over pairs that match.  A wave's positions are neighbours:
+// the last have the most writers before them and the fewest readers after them, so the two loops balance.
+struct ChunkGradArgs {
+  const int32_t* slot[2];   // write, read picks [B][H][T][KP] (entries >= kk ignored)
+  const float* wt[2];
+  const void* v;            // value rows (H * dh per row), type VT
+  int64_t v_stride;
+  const float* dnum;        // [B*T] rows of H * dh
+  const float* dden;        // [B*T][H]
+  const uint8_t* reset;     // [B*T] or nullptr
+  const float* decay;       // [H]
+  float* dot_w;             // [column group][B][H][T][KP] partial dww, dwr (dden term in group 0)
+  float* dot_r;
+  float* dv;                // rows of H * dh: partial dV
+  int B, T, H, dh, M, kk, n_xg;
+};
+
+struct ChunkGradLds {
+  size_t mask, v, dn, sl, wt, pw, dd, total;
+  __host__ __device__ constexpr ChunkGradLds(int M, int KP)
+      : mask(0),
+        v(align16(8 * static_cast<size_t>(M))),
+        dn(v + 4 * 64 * 64),
+        sl(dn + 4 * 64 * 64),
+        wt(sl + 2 * 4 * 64 * KP),
+        pw(wt + 2 * 4 * 64 * KP),
+        dd(pw + 4 * 64),
+        total(dd + 4 * 64) {}
+};
+
+template <int KP, typename VT>
+__global__ void __launch_bounds__(kGradScanThreads) chunk_grad_kernel(ChunkGradArgs a) {
+  constexpr int NO = KP / 8;   // picks per lane: l8, l8 + 8
+  extern __shared__ __attribute__((aligned(16))) unsigned char clds[];
+  const ChunkGradLds lay(a.M, KP);
+  unsigned long long* mask = reinterpret_cast<unsigned long long*>(clds + lay.mask);
+  float* sv = reinterpret_cast<float*>(clds + lay.v);
+  float* sdn = reinterpret_cast<float*>(clds + lay.dn);
+  int32_t* ssl = reinterpret_cast<int32_t*>(clds + lay.sl);   // [2][64][KP], pads -1
+  float* swt = reinterpret_cast<float*>(clds + lay.wt);
+  float* pw = reinterpret_cast<float*>(clds + lay.pw);
+  float* sdd = reinterpret_cast<float*>(clds + lay.dd);
+  const int u0 = blockIdx.x * kChunk;
+  const int h = blockIdx.y % a.H, xg = blockIdx.y / a.H;
+  const int b = blockIdx.z;
+  const int tid = threadIdx.x, p = tid >> 3, l8 = tid & 7, lane = tid & 63;
+  const int M = a.M, kk = a.kk, T = a.T;
+  const int L = min(kChunk, T - u0);
+  const bool valid = p < L;
+  const int t = u0 + (valid ? p : 0);
+  const int64_t n = static_cast<int64_t>(b) * T + t;
+  const int64_t prow = ((static_cast<int64_t>(b) * a.H + h) * T + t) * KP;
+  const float lam = a.decay[h];
+  // the lane's columns of the position's rows: 4 l8 .. + 3 and 32 + 4 l8 .. + 3 of the group's 64
+  float dn[8], v[8];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int c = 64 * xg + 32 * q + 4 * l8;
+    float x4[4] = {0.f, 0.f, 0.f, 0.f}, y4[4] = {0.f, 0.f, 0.f, 0.f};
+    if (valid && c < a.dh) {
+      load_vals<4, float>(a.dnum + n * a.H * a.dh + static_cast<int64_t>(h) * a.dh + c, x4);
+      load_vals<4, VT>(static_cast<const VT*>(a.v) + n * a.v_stride + static_cast<int64_t>(h) * a.dh + c, y4);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      dn[4 * q + e] = x4[e];
+      v[4 * q + e] = y4[e];
+    }
+    *reinterpret_cast<float4*>(&sdn[p * 64 + 32 * q + 4 * l8]) = make_float4(x4[0], x4[1], x4[2], x4[3]);
+    *reinterpret_cast<float4*>(&sv[p * 64 + 32 * q + 4 * l8]) = make_float4(y4[0], y4[1], y4[2], y4[3]);
+  }
+  const float dd = valid && xg == 0 ? a.dden[n * a.H + h] : 0.f;
+  if (l8 == 0) sdd[p] = dd;
+  int sl[2][NO];
+  float wt[2][NO];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      const int j = l8 + 8 * o;
+      const bool live = valid && j < kk;
+      const int s = live ? a.slot[k][prow + j] : 0;
+      sl[k][o] = live ? (s >= 0 && s < M ? s : 0) : -1;
+      wt[k][o] = live ? a.wt[k][prow + j] : 0.f;
+      ssl[(k * 64 + p) * KP + j] = sl[k][o];
+      swt[(k * 64 + p) * KP + j] = wt[k][o];
+    }
+  if (tid < 64) {
+    float f = 1.f, sq = lam;   // lam^tid by squaring (exact for lam = 0 and lam = 1)
+#pragma unroll
+    for (int bit = 0; bit < 6; ++bit) {
+      f = ((tid >> bit) & 1) ? f * sq : f;
+      sq *= sq;
+    }
+    pw[tid] = f;
+  }
+  // the chunk's resets, in every wave
+  const uint8_t rv8 = *(a.reset ? a.reset + static_cast<int64_t>(b) * T + u0 + min(lane, L - 1)
+                                : reinterpret_cast<const uint8_t*>(a.decay));
+  const unsigned long long rmask = __ballot(a.reset && lane < L && rv8 != 0);
+
+  float dot[2][NO], sum[8];
+#pragma unroll
+  for (int o = 0; o < NO; ++o) dot[0][o] = dot[1][o] = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+  const unsigned long long bit = 1ull << p, below = bit - 1ull, above = ~(below | bit);
+  // k = 0: position p reads the writers before it; k = 1: position p's writes are read by the readers after it
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (k == 1) lds_barrier();   // the writers' masks are done with
+    for (int i = tid; i < M; i += kGradScanThreads) mask[i] = 0ull;
+    lds_barrier();
+#pragma unroll
+    for (int o = 0; o < NO; ++o)
+      if (sl[k][o] >= 0) atomicOr(&mask[sl[k][o]], bit);
+    lds_barrier();
+    unsigned long long vis;   // the other side's positions of the segment
+    if (k == 0) {
+      const unsigned long long upto = rmask & (below | bit);
+      vis = below & (upto ? ~((1ull << (63 - __builtin_clzll(upto))) - 1ull) : ~0ull);
+    } else {
+      const unsigned long long after = rmask & above;
+      vis = above & (after ? (after & -after) - 1ull : ~0ull);
+    }
+    unsigned long long mk[NO], any = 0ull;
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      const int s = sl[1 - k][o];
+      mk[o] = s >= 0 ? mask[s] & vis : 0ull;
+      any |= mk[o];
+    }
+    unsigned long long U = group_or8(any);
+    const float* rows = k == 0 ? sv : sdn;
+    while (U) {
+      const int q = __builtin_ctzll(U);
+      U &= U - 1ull;
+      const float4 x0 = *reinterpret_cast<const float4*>(&rows[q * 64 + 4 * l8]);
+      const float4 x1 = *reinterpret_cast<const float4*>(&rows[q * 64 + 32 + 4 * l8]);
+      const float xr[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      const float f = pw[k == 0 ? p - 1 - q : q - 1 - p];
+      float X = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) X = fmaf(k == 0 ? dn[e] : v[e], xr[e], X);
+      X = sum8(X) + (k == 0 ? dd : sdd[q]);
+      float cs = 0.f;
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        const float wq = writer_weight<KP>(ssl + k * 64 * KP, swt + k * 64 * KP, q, sl[1 - k][o]);
+        const float co = ((mk[o] >> q) & 1ull) ? f * wq : 0.f;
+        dot[1 - k][o] = fmaf(co, X, dot[1 - k][o]);
+        cs = fmaf(wt[1 - k][o], co, cs);
+      }
+      if (k == 1) {
+        cs = sum8(cs);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] = fmaf(cs, xr[e], sum[e]);
+      }
+    }
+  }
+  if (!valid) return;
+  const int64_t cg = static_cast<int64_t>(xg) * a.B * a.H * T * KP;
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    const int j = l8 + 8 * o;
+    a.dot_w[cg + prow + j] = dot[0][o];
+    a.dot_r[cg + prow + j] = dot[1][o];
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int c = 64 * xg + 32 * q + 4 * l8;
+    if (c < a.dh) {
+      float o4[4] = {sum[4 * q], sum[4 * q + 1], sum[4 * q + 2], sum[4 * q + 3]};
+      store_vals<4, float>(a.dv + n * a.H * a.dh + static_cast<int64_t>(h) * a.dh + c, o4);
+    }
+  }
+}
+
 // One workgroup per (column group, head, batch row): 512 threads = 64 positions x 8 lanes of CW/8 columns; the
-// slab A (true state mu * A) and the counts stay in LDS.  REV runs the sequence backwards (position u is t = T-1-u);
-// a reset at t then separates u = T-t and later from what came before.  Per chunk of 64 positions:
-//   stage   the chunk's write picks, weights, values and count factors into LDS; mark each slot's writers in wmask
-//   read    group = position: the carried rows of its picks (scaled by mu lam^p; none after a reset in the chunk)
-//           and the in-chunk writes of earlier positions of its segment; per pick the dot with the position's read
-//           vector (+ the read count factor times the count, in column group 0) and, with sum_out, the pick-weighted
-//           sum of the rows
-//   write   fade (mu <- mu lam^L; a chunk with a reset empties the slab), then group g applies the chain plan's
-//           write records g + 64 k: each written slot's kept writers' faded values / mu, added to the slot's row in
-//           one pass (one owner per row: no atomics), lane l8 the count of record l8 + 8 b
+// slab A (true state mu * A) and the counts stay in LDS.  REV runs the sequence backwards (ChunkSpan); a reset at t
+// then separates t - 1 and earlier from what came before it.  Per chunk of 64 positions:
+//   read    group = position: the carried rows of its picks (scaled by mu lam^p; none after a reset in the chunk); per
+//           pick the dot with the position's read vector (+ the read count factor times the count, in column group 0)
+//           and, with sum_out, the pick-weighted sum of the rows
+//   sums    group g takes the chain plan's write records g + 64 k: each written slot's old row plus its kept writers'
+//           faded values / mu (mu <- mu lam^L; a chunk with a reset empties the slab), one owner per row, lane l8 the
+//           count of record l8 + 8 b
+//   store   the rows and counts back, the next chunk's write values, records and chain entries into LDS
+// with a barrier before and after the stores.  Bound: the chain of chunks on one compute unit per slab and column
+// group (192 of 256 at B=8, 12 heads), 8,500 cycles each: 3,900 of VALU, 2,900 of LDS (a quarter of it bank conflicts of
+// the random rows), the rest waits; neither fewer vector-memory instructions nor shorter walks of the chains moved it.
 template <int CW, int KP, bool REV, typename WT, typename RT>
 __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArgs a) {
   constexpr int CPL = CW / 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char glds[];
   const int M = a.M;
   const GradScanLds lay(M, KP, CW);
-  unsigned long long* wmask = reinterpret_cast<unsigned long long*>(glds + lay.wmask);
   float* A = reinterpret_cast<float*>(glds + lay.A);
   float* cnt = reinterpret_cast<float*>(glds + lay.cnt);
-  int32_t* s_ws = reinterpret_cast<int32_t*>(glds + lay.ws);
-  float* s_ww = reinterpret_cast<float*>(glds + lay.ww);
   float* s_wv = reinterpret_cast<float*>(glds + lay.wv);
   float* s_wc = reinterpret_cast<float*>(glds + lay.wc);
   float* pw = reinterpret_cast<float*>(glds + lay.pw);
-  unsigned char* s_rm = glds + lay.rm;
+  uint2* s_rec = reinterpret_cast<uint2*>(glds + lay.rec);
   unsigned char* s_ext = glds + lay.ext;
   constexpr int XS = grad_ext_stage(KP);
   constexpr int NX = (XS / 16 + kGradScanThreads - 1) / kGradScanThreads;   // staged chain pieces per thread
@@ -454,7 +659,6 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
   const int tid = threadIdx.x;
   const int g = tid >> 3;
   const int l8 = tid & 7;
-  const int lane = tid & 63;
   const int col0 = cg * CW;
   const int kk = a.kk;
   const int T = a.T;
@@ -472,60 +676,59 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
   float mu = 1.f;
   __syncthreads();
 
-  // one chunk's global inputs, loaded a chunk ahead into registers (raw element types, converted when staged)
+  // one chunk's global inputs, loaded a chunk ahead into registers (raw element types, converted when used)
   struct In {
-    int ws[KP / 8];
-    float ww[KP / 8];
-    WT wv[CPL];
+    RawSeg<WT, CPL> wv;
     float wc;
-    bool rf;
-    int rs[KP];
-    float rw[KP];
-    RT rv[CPL];
+    RawSeg<int, 4> rs[KP / 4];
+    RawSeg<float, 4> rw[KP / 4];
+    RawSeg<RT, CPL> rv;
     float rcf;
-    uint4 wrec[KP / 2];   // the group's write records
-    uint2 own_w[KP / 8];  // write records k = l8 + 8 b (the lane's count updates)
+    RawSeg<float, CPL> sum;
+    uint2 own_w[KP / 8];  // write records k = l8 + 8 b of the group (the lane's count updates; staged for the group)
     uint4 xp[NX];         // chain pieces to stage
+    uint2 rm;             // the chunk's reset mask
   };
   const unsigned char* chains = a.chains + bh * a.n_chunks * chain_stride(KP);
   auto fetch = [&](int c, In& x) {
-    const int u0 = c * kChunk;
-    const bool valid = g < min(kChunk, T - u0);
-    const int t = valid ? (REV ? T - 1 - (u0 + g) : u0 + g) : 0;   // row 0 stands in for a missing position
+    const ChunkSpan<REV> span(c, T, a.n_chunks);
+    const bool valid = g < span.L;
+    const int t = span.token(g);   // the chunk's first token stands in for a missing position
     const int64_t n = static_cast<int64_t>(b) * T + t;
     const int64_t prow = (bh * T + t) * KP;
+    const int64_t vcol = static_cast<int64_t>(h) * a.dh + col0 + CPL * l8;
+    // one load per lane's piece where everything is aligned: 9 loads per wave and chunk instead of 25 to 38
+    const WT* wvp = static_cast<const WT*>(a.wv) + n * a.wv_stride + vcol;
+    const RT* rvp = static_cast<const RT*>(a.rv) + n * a.rv_stride + vcol;
+    const float* sip = REV ? a.sum_in + n * a.H * a.dh + vcol : nullptr;
+    if (a.vec) {
+      x.wv = *reinterpret_cast<const RawSeg<WT, CPL>*>(wvp);
+      x.rv = *reinterpret_cast<const RawSeg<RT, CPL>*>(rvp);
+      if constexpr (REV) x.sum = *reinterpret_cast<const RawSeg<float, CPL>*>(sip);
 #pragma unroll
-    for (int o = 0; o < KP / 8; ++o) {
-      const bool live = valid && l8 + 8 * o < kk;
-      x.ws[o] = live ? a.w_slot[prow + l8 + 8 * o] : -1;
-      x.ww[o] = live ? a.w_wt[prow + l8 + 8 * o] : 0.f;
-    }
-    const WT* wvp = static_cast<const WT*>(a.wv) + n * a.wv_stride + static_cast<int64_t>(h) * a.dh + col0 + CPL * l8;
+      for (int i = 0; i < KP / 4; ++i) {
+        x.rs[i] = *reinterpret_cast<const RawSeg<int, 4>*>(a.r_slot + prow + 4 * i);
+        x.rw[i] = *reinterpret_cast<const RawSeg<float, 4>*>(a.r_wt + prow + 4 * i);
+      }
+    } else {
+      asm volatile("" ::: "memory");   // keeps the compiler from merging the branches' loads into element loads
 #pragma unroll
-    for (int k = 0; k < CPL; ++k) x.wv[k] = wvp[k];
-    x.wc = valid ? (a.wc ? a.wc[n * a.H + h] : 1.f) : 0.f;
-    x.rf = false;
-    if (valid && a.reset) {
-      if constexpr (REV) {
-        x.rf = (u0 + g >= 1) && a.reset[static_cast<int64_t>(b) * T + (T - (u0 + g))];
-      } else {
-        x.rf = a.reset[n] != 0;
+      for (int k = 0; k < CPL; ++k) {
+        x.wv.e[k] = wvp[k];
+        x.rv.e[k] = rvp[k];
+        if constexpr (REV) x.sum.e[k] = sip[k];
+      }
+#pragma unroll
+      for (int i = 0; i < KP; ++i) {
+        x.rs[i / 4].e[i % 4] = a.r_slot[prow + i];
+        x.rw[i / 4].e[i % 4] = a.r_wt[prow + i];
       }
     }
-#pragma unroll
-    for (int i = 0; i < KP; ++i) {
-      const bool live = valid && i < kk;
-      x.rs[i] = live ? a.r_slot[prow + i] : 0;
-      x.rw[i] = live ? a.r_wt[prow + i] : 0.f;
-    }
-    const RT* rvp = static_cast<const RT*>(a.rv) + n * a.rv_stride + static_cast<int64_t>(h) * a.dh + col0 + CPL * l8;
-#pragma unroll
-    for (int k = 0; k < CPL; ++k) x.rv[k] = rvp[k];
+    x.wc = valid ? (a.wc ? a.wc[n * a.H + h] : 1.f) : 0.f;
     x.rcf = (valid && a.rc) ? a.rc[n * a.H + h] : 1.f;
     const unsigned char* cp = chains + static_cast<int64_t>(c) * chain_stride(KP);
+    x.rm = reinterpret_cast<const uint2*>(cp)[1];
     const uint2* wrow = reinterpret_cast<const uint2*>(cp + 16) + g * KP;
-#pragma unroll
-    for (int k = 0; k < KP / 2; ++k) x.wrec[k] = reinterpret_cast<const uint4*>(wrow)[k];
 #pragma unroll
     for (int k = 0; k < KP / 8; ++k) x.own_w[k] = wrow[l8 + 8 * k];
     // the first chain entries (the whole staged span: loads past n_ext stay inside the plan)
@@ -537,69 +740,56 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
     }
   };
 
-  In cur;
-  fetch(0, cur);
-  for (int c = 0; c < a.n_chunks; ++c) {
-    const int u0 = c * kChunk;
-    const int L = min(kChunk, T - u0);
-    const bool valid = g < L;
-    const int t = valid ? (REV ? T - 1 - (u0 + g) : u0 + g) : 0;
-    const int64_t n = static_cast<int64_t>(b) * T + t;
-    // stage the writes
+  // a chunk's write values, count factors, records and chain entries into LDS
+  auto stage = [&](const In& x, bool valid) {
+    float vv[CPL];
 #pragma unroll
-    for (int o = 0; o < KP / 8; ++o) {
-      const int s = cur.ws[o];
-      s_ws[g * KP + l8 + 8 * o] = s < 0 ? -1 : min(s, M - 1);   // pads -1
-      s_ww[g * KP + l8 + 8 * o] = cur.ww[o];
-    }
-    {
-      float vv[CPL];
+    for (int k = 0; k < CPL; ++k) vv[k] = valid ? to_f32(x.wv.e[k]) : 0.f;
+    lds_seg_store<CPL>(&s_wv[g * CW + CPL * l8], *reinterpret_cast<const Seg<CPL>*>(vv));
+    if (l8 == 0) s_wc[g] = x.wc;
 #pragma unroll
-      for (int k = 0; k < CPL; ++k) vv[k] = valid ? to_f32(cur.wv[k]) : 0.f;
-      lds_seg_store<CPL>(&s_wv[g * CW + CPL * l8], *reinterpret_cast<const Seg<CPL>*>(vv));
-    }
-    if (l8 == 0) s_wc[g] = cur.wc;
+    for (int k = 0; k < KP / 8; ++k) s_rec[g * KP + l8 + 8 * k] = x.own_w[k];
 #pragma unroll
     for (int k = 0; k < NX; ++k) {
       const int piece = tid + k * kGradScanThreads;
-      if (piece < XS / 16) reinterpret_cast<uint4*>(s_ext)[piece] = cur.xp[k];
+      if (piece < XS / 16) reinterpret_cast<uint4*>(s_ext)[piece] = x.xp[k];
     }
-    {
-      const unsigned long long bal = __ballot(cur.rf && l8 == 0);   // bits 0, 8, ..., 56: the wave's 8 positions
-      if (lane == 0) {
-        unsigned v8 = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v8 |= static_cast<unsigned>((bal >> (8 * k)) & 1ull) << k;
-        s_rm[tid >> 6] = static_cast<unsigned char>(v8);
-      }
-    }
+  };
+
+  In cur;
+  fetch(0, cur);
+  stage(cur, g < ChunkSpan<REV>(0, T, a.n_chunks).L);
+  lds_barrier();
+  for (int c = 0; c < a.n_chunks; ++c) {
+    const ChunkSpan<REV> span(c, T, a.n_chunks);
+    const int L = span.L;
+    const bool valid = g < L;
+    const int t = span.token(g);
+    const int64_t n = static_cast<int64_t>(b) * T + t;
+    const unsigned long long rmask = (static_cast<unsigned long long>(cur.rm.y) << 32) | cur.rm.x;
     // the read side of this position, in registers: all picks (every lane), the lane's vector columns
     int rs[KP];
     float rw[KP];
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
-      rs[i] = (cur.rs[i] >= 0 && cur.rs[i] < M) ? cur.rs[i] : 0;
-      rw[i] = cur.rw[i];
+      rs[i] = static_cast<int>(min(static_cast<uint32_t>(cur.rs[i / 4].e[i % 4]), static_cast<uint32_t>(M)));
+      rw[i] = cur.rw[i / 4].e[i % 4];
+    }
+    if (kk < KP) {   // pads, as stray slots, read row M, which is zero
+#pragma unroll
+      for (int i = 0; i < KP; ++i)
+        if (i >= kk) {
+          rs[i] = M;
+          rw[i] = 0.f;
+        }
     }
     float rv[CPL];
 #pragma unroll
-    for (int k = 0; k < CPL; ++k) rv[k] = valid ? to_f32(cur.rv[k]) : 0.f;
+    for (int k = 0; k < CPL; ++k) rv[k] = valid ? to_f32(cur.rv.e[k]) : 0.f;
     const float rcf = cur.rcf;
-    for (int i = tid; i < M; i += kGradScanThreads) wmask[i] = 0ull;
     In nxt;
     const bool more = c + 1 < a.n_chunks;
-    if (more) fetch(c + 1, nxt);   // in flight across the barriers below (they order LDS only)
-    lds_barrier();
-    if (valid) {
-#pragma unroll
-      for (int j = l8; j < KP; j += 8)
-        if (j < kk) {
-          const int m = s_ws[g * KP + j];
-          if (m >= 0) atomicOr(&wmask[m], 1ull << g);
-        }
-    }
-    const unsigned long long rmask = *reinterpret_cast<const unsigned long long*>(s_rm);
-    lds_barrier();
+    if (more) fetch(c + 1, nxt);   // in flight across the barrier below (it orders LDS only)
 
     // read
     constexpr int NO = KP / 8;   // picks owned per lane: l8, l8 + 8
@@ -611,9 +801,7 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
     for (int k = 0; k < CPL; ++k) sum[k] = 0.f;
     if (valid) {
       const int p = g;
-      const unsigned long long upto = rmask & (p == 63 ? ~0ull : (2ull << p) - 1ull);
-      const int seg0 = upto ? 63 - __builtin_clzll(upto) : -1;
-      if (seg0 < 0) {   // the carried state
+      if (!(rmask & (p == 63 ? ~0ull : (2ull << p) - 1ull))) {   // the carried state
         const float fin = mu * pw[p];
         float part[KP];
 #pragma unroll
@@ -647,141 +835,110 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
 #pragma unroll
         for (int k = 0; k < CPL; ++k) sum[k] *= fin;
       }
-      // in-chunk writes of earlier positions of the segment
-      const unsigned long long below = (1ull << p) - 1ull;
-      const unsigned long long vis = below & (seg0 >= 0 ? ~((1ull << seg0) - 1ull) : ~0ull);
-      int so[NO];
-      float wo[NO];
-      unsigned long long mk[NO];
-      unsigned long long any = 0ull;
-#pragma unroll
-      for (int o = 0; o < NO; ++o) {
-        so[o] = 0;
-        wo[o] = 0.f;
-#pragma unroll
-        for (int i = 0; i < KP; ++i)
-          if (i == l8 + 8 * o) {
-            so[o] = rs[i];
-            wo[o] = rw[i];
-          }
-        mk[o] = (l8 + 8 * o < kk) ? (wmask[so[o]] & vis) : 0ull;
-        any |= mk[o];
-      }
-      unsigned long long U = group_or8(any);
-      while (U) {
-        const int q = __builtin_ctzll(U);
-        U &= U - 1ull;
-        const Seg<CPL> x = lds_seg<CPL>(&s_wv[q * CW + CPL * l8]);
-        float d = 0.f;
-#pragma unroll
-        for (int k = 0; k < CPL; ++k) d = fmaf(rv[k], x.v[k], d);
-        d = sum8(d);
-        const float fq = pw[p - 1 - q];
-        const float wcq = s_wc[q];
-        float cs = 0.f;
-#pragma unroll
-        for (int o = 0; o < NO; ++o) {
-          const float wq = writer_weight<KP>(s_ws, s_ww, q, so[o]);   // loaded with the row: no branch
-          const float co = ((mk[o] >> q) & 1ull) ? fq * wq : 0.f;
-          dot[o] = fmaf(co, d, dot[o]);
-          if (cg == 0) dot[o] = fmaf(co * rcf, wcq, dot[o]);
-          cs = fmaf(wo[o], co, cs);
-        }
-        if (a.sum_out) {
-          cs = sum8(cs);
-#pragma unroll
-          for (int k = 0; k < CPL; ++k) sum[k] = fmaf(cs, x.v[k], sum[k]);
-        }
-      }
       // outputs
 #pragma unroll
       for (int o = 0; o < NO; ++o) {
         const int i = l8 + 8 * o;
         dot_out[static_cast<int64_t>(t) * KP + i] = i < kk ? dot[o] : 0.f;
       }
-      if (a.sum_out) {
+      if (REV) {
+#pragma unroll
+        for (int k = 0; k < CPL; ++k) sum[k] += cur.sum.e[k];
         const int64_t at = n * a.sum_stride + static_cast<int64_t>(h) * a.dh + col0 + CPL * l8;
         if (a.sum_bf16) store_vals<CPL, bf16_t>(static_cast<bf16_t*>(a.sum_out) + at, sum);
         else store_vals<CPL, float>(static_cast<float*>(a.sum_out) + at, sum);
       }
     }
-    lds_barrier();
 
-    // write: fade (an emptied slab for a chunk with a reset), then the kept writers of each slot
-    float mu_new = mu * pw[L];
-    if (rmask) {
-      for (int i = tid; i < M * CW; i += kGradScanThreads) A[i] = 0.f;
-      for (int i = tid; i < M; i += kGradScanThreads) cnt[i] = 0.f;
-      mu_new = 1.f;
-      lds_barrier();
-    } else if (!(mu_new >= kMuFloor)) {
-      for (int i = tid; i < M * CW; i += kGradScanThreads) A[i] *= mu_new;
-      for (int i = tid; i < M; i += kGradScanThreads) cnt[i] *= mu_new;
-      mu_new = 1.f;
-      lds_barrier();
-    }
-    // group g applies records g + 64 k of the chain plan, 8 at a time (distinct slots; null records write nothing)
-    {
-      const float inv_mu = fast_rcp(mu_new);
-      const unsigned char* gext = chains + static_cast<int64_t>(c) * chain_stride(KP) + 16 + 8 * kChunk * KP;
-      auto ext_at = [&](int e) {
-        return 8 * e + 8 <= XS ? reinterpret_cast<const uint2*>(s_ext)[e] : reinterpret_cast<const uint2*>(gext)[e];
-      };
-      uint2 wr[KP];
+    // the written rows' new values (no other group writes them, so they can be summed before the reads are done):
+    // the old row faded by the chunk (as mu; by `keep` itself where the slab is emptied or rescaled), the slot's first
+    // writer and its later ones from the chain.  Group g takes records g + 64 k; null records (row M) write nothing
+    const float mu_all = mu * pw[L];
+    const bool fold = rmask != 0 || !(mu_all >= kMuFloor);   // the slab takes the scale in: mu restarts at 1
+    const float keep = rmask ? 0.f : fold ? mu_all : 1.f;
+    const float inv_mu = fold ? 1.f : fast_rcp(mu_all);
+    const unsigned char* gext = chains + static_cast<int64_t>(c) * chain_stride(KP) + 16 + 8 * kChunk * KP;
+    auto ext_at = [&](int e) {
+      return 8 * e + 8 <= XS ? reinterpret_cast<const uint2*>(s_ext)[e] : reinterpret_cast<const uint2*>(gext)[e];
+    };
+    auto row_of = [&](int q) { return lds_seg<CPL>(&s_wv[(q & 63) * CW + CPL * l8]); };
+    Seg<CPL> x[KP];
+    int slot_of[KP], own_slot[NO];
+    float own_cnt[NO];
 #pragma unroll
-      for (int k = 0; k < KP; ++k)
-        wr[k] = make_uint2(u4_word(cur.wrec[k / 2], 2 * (k % 2)), u4_word(cur.wrec[k / 2], 2 * (k % 2) + 1));
+    for (int k0 = 0; k0 < KP; k0 += 8) {
+      uint2 wr[8];
 #pragma unroll
-      for (int k0 = 0; k0 < KP; k0 += 8) {
-        Seg<CPL> x[8], vq[8];
-        float dc[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t rx = wr[k0 + j].x;
-          dc[j] = __uint_as_float(wr[k0 + j].y & 0x7fffffffu) * inv_mu;
-          x[j] = lds_seg<CPL>(&A[(rx & 0xffffu) * CW + CPL * l8]);
-          vq[j] = lds_seg<CPL>(&s_wv[((rx >> 16) & 63u) * CW + CPL * l8]);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-#pragma unroll
-          for (int k = 0; k < CPL; ++k) x[j].v[k] = fmaf(dc[j], vq[j].v[k], x[j].v[k]);
-          if (wr[k0 + j].y & 0x80000000u) {   // later writers of the slot in this chunk
-            int e = wr[k0 + j].x >> 22;
-            uint2 t;
-            do {
-              t = ext_at(e++);
-              const float cf = __uint_as_float(t.x) * inv_mu;
-              const Seg<CPL> vx = lds_seg<CPL>(&s_wv[(t.y & 63u) * CW + CPL * l8]);
-#pragma unroll
-              for (int k = 0; k < CPL; ++k) x[j].v[k] = fmaf(cf, vx.v[k], x[j].v[k]);
-            } while (!(t.y & 0x80000000u));
-          }
-        }
-        // lane l8's count update for record k0 + l8: the writers' coefficients times their count factors
-        const uint2 ow = cur.own_w[k0 / 8];
-        const int mc = static_cast<int>(ow.x & 0xffffu);
-        float dcc = __uint_as_float(ow.y & 0x7fffffffu) * s_wc[(ow.x >> 16) & 63u];
-        if (ow.y & 0x80000000u) {
-          int e = ow.x >> 22;
-          uint2 t;
-          do {
-            t = ext_at(e++);
-            dcc = fmaf(__uint_as_float(t.x), s_wc[t.y & 63u], dcc);
-          } while (!(t.y & 0x80000000u));
-        }
-        const float cold = cnt[mc];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {   // null records (row M) write nothing: no same-row write conflicts
-          const int mj = static_cast<int>(wr[k0 + j].x & 0xffffu);
-          if (mj != M) lds_seg_store<CPL>(&A[mj * CW + CPL * l8], x[j]);
-        }
-        if (mc != M) cnt[mc] = fmaf(dcc, inv_mu, cold);
+      for (int j = 0; j < 8; j += 2) {
+        const uint4 r2 = *reinterpret_cast<const uint4*>(&s_rec[g * KP + k0 + j]);
+        wr[j] = make_uint2(r2.x, r2.y);
+        wr[j + 1] = make_uint2(r2.z, r2.w);
       }
+      Seg<CPL> vq[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        slot_of[k0 + j] = static_cast<int>(wr[j].x & 0xffffu);
+        x[k0 + j] = lds_seg<CPL>(&A[slot_of[k0 + j] * CW + CPL * l8]);
+        vq[j] = row_of(wr[j].x >> 16);
+      }
+      const uint2 ow = cur.own_w[k0 / 8];   // the lane's count: record k0 + l8
+      own_slot[k0 / 8] = static_cast<int>(ow.x & 0xffffu);
+      const float cold = cnt[own_slot[k0 / 8]] * keep;
+      float dcc = __uint_as_float(ow.y & 0x7fffffffu) * s_wc[(ow.x >> 16) & 63u];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float dc = __uint_as_float(wr[j].y & 0x7fffffffu) * inv_mu;
+#pragma unroll
+        for (int k = 0; k < CPL; ++k) x[k0 + j].v[k] = fmaf(dc, vq[j].v[k], x[k0 + j].v[k] * keep);
+      }
+      // the later writers of two records at a time, the next entries loaded ahead: a chain costs one LDS round trip a
+      // writer, and the two records' overlap
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) {
+        bool l0 = wr[j].y >> 31, l1 = wr[j + 1].y >> 31;
+        if (l0 || l1) {
+          int e0 = wr[j].x >> 22, e1 = wr[j + 1].x >> 22;
+          uint2 t0 = ext_at(min(e0, kChunk * KP - 1)), t1 = ext_at(min(e1, kChunk * KP - 1));
+          do {
+            const Seg<CPL> v0 = row_of(t0.y), v1 = row_of(t1.y);
+            const float w0 = s_wc[t0.y & 63u], w1 = s_wc[t1.y & 63u];
+            const uint2 n0 = ext_at(min(++e0, kChunk * KP - 1)), n1 = ext_at(min(++e1, kChunk * KP - 1));
+            const float c0 = __uint_as_float(t0.x), c1 = __uint_as_float(t1.x);
+#pragma unroll
+            for (int k = 0; k < CPL; ++k) {
+              x[k0 + j].v[k] = l0 ? fmaf(c0 * inv_mu, v0.v[k], x[k0 + j].v[k]) : x[k0 + j].v[k];
+              x[k0 + j + 1].v[k] = l1 ? fmaf(c1 * inv_mu, v1.v[k], x[k0 + j + 1].v[k]) : x[k0 + j + 1].v[k];
+            }
+            dcc = l0 && l8 == j ? fmaf(c0, w0, dcc) : dcc;
+            dcc = l1 && l8 == j + 1 ? fmaf(c1, w1, dcc) : dcc;
+            l0 = l0 && !(t0.y >> 31);
+            l1 = l1 && !(t1.y >> 31);
+            t0 = n0;
+            t1 = n1;
+          } while (l0 || l1);
+        }
+      }
+      own_cnt[k0 / 8] = fmaf(dcc, inv_mu, cold);
     }
-    mu = mu_new;
+    lds_barrier();   // every read of the slab and of the staged chunk is done
+
+    if (fold) {
+      for (int i = tid; i < M * CW; i += kGradScanThreads) A[i] = rmask ? 0.f : A[i] * mu_all;
+      for (int i = tid; i < M; i += kGradScanThreads) cnt[i] = rmask ? 0.f : cnt[i] * mu_all;
+      lds_barrier();
+    }
+#pragma unroll
+    for (int j = 0; j < KP; ++j)
+      if (slot_of[j] != M) lds_seg_store<CPL>(&A[slot_of[j] * CW + CPL * l8], x[j]);
+#pragma unroll
+    for (int o = 0; o < NO; ++o)
+      if (own_slot[o] != M) cnt[own_slot[o]] = own_cnt[o];
+    mu = fold ? 1.f : mu_all;
+    if (more) {
+      stage(nxt, g < ChunkSpan<REV>(c + 1, T, a.n_chunks).L);
+      cur = nxt;
+    }
     lds_barrier();
-    if (more) cur = nxt;
   }
 }
 
@@ -1208,8 +1365,8 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
   const bool live_col = NT == 2 ? col < HALF : col < DA;
   const int64_t N = static_cast<int64_t>(a.B) * a.T;   // below 2^31: each token has picks of 4 * 32 bytes and more
   const int64_t cg_stride = N * a.H * KP;
-  float acc_tau = 0.f, acc_gb = 0.f, acc_ab[NT];
-  double acc_lam = 0.0;
+  float acc_ab[NT];
+  double acc_lam = 0.0, acc_tau = 0.0, acc_gb = 0.0;
   floatx16 dk[2][NSB];
 #pragma unroll
   for (int p = 0; p < NT; ++p) acc_ab[p] = 0.f;
@@ -1237,8 +1394,10 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
       slr[it] = slot[e];
       svr[it] = scp[e];
       wtr[it] = wtp[e];
-      dwr[it] = dotp[e];
-      for (int c = 1; c < a.n_cg; ++c) dwr[it] += dotp[c * cg_stride + e];
+      // up to three partials (a head of 64 columns) in straight code: their loads issue with the others
+      const float d1 = dotp[(a.n_cg > 1 ? cg_stride : 0) + e], d2 = dotp[(a.n_cg > 2 ? 2 * cg_stride : 0) + e];
+      dwr[it] = dotp[e] + (a.n_cg > 1 ? d1 : 0.f) + (a.n_cg > 2 ? d2 : 0.f);
+      for (int c = 3; c < a.n_cg; ++c) dwr[it] += dotp[c * cg_stride + e];
       glr[it] = gated ? static_cast<const InT*>(a.gl)[n * a.g_stride + h] : zb[0];
     }
     const InT* zt = zb + n0 * zs;   // the tile's rows: offsets from here in 32 bits
@@ -1272,14 +1431,14 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
       const float wt = pl ? wtr[it] : 0.f;
       const float dw = pl ? dwr[it] : 0.f;
       const float P = pick_sum<KP>(wt * dw);
+      const float sv0 = __shfl(sv, lane & ~(KP - 1));   // the token's best score
       float dx;
       if (set == 1) {   // read: softmax
         dx = wt * (dw - P);
         if (pj == 0) acc_lam += static_cast<double>(tr[it]) * static_cast<double>(P);
       } else {          // write: gated softmax
         if (pj == 0) acc_lam -= static_cast<double>(tr[it] + 1) * static_cast<double>(P);
-        const float x0 = __shfl(sv, lane & ~(KP - 1)) * tau;
-        float pr = pl ? __expf(sv * tau - x0) : 0.f;
+        float pr = pl ? __expf(sv * tau - sv0 * tau) : 0.f;
         const float ps = pick_sum<KP>(pr);
         pr *= fast_rcp(valid ? ps : 1.f);
         const float gt = gated ? fast_rcp(1.f + __expf(-(to_f32(glr[it]) + gb))) : 1.f;
@@ -1293,7 +1452,8 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
         }
       }
       if (!pl) dx = 0.f;
-      acc_tau = fmaf(sv, dx, acc_tau);
+      // a token's dx sum to zero, so its scores count from the best one: small terms instead of large ones that cancel
+      acc_tau += static_cast<double>((sv - sv0) * dx);
       hs[it] = 0.5f * tau * dx;
       const int i1 = n_sub > 1 ? static_cast<int>(__umulhi(static_cast<uint32_t>(sl), magic)) : sl;
       const int row = (it * TPI + lane / KP) * GP;
@@ -1377,10 +1537,12 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
     wave_lds_fence();
   }
   // block sums in a fixed order: waves -> LDS -> threads
-  acc_tau = wave_sum(acc_tau);
-  acc_gb = wave_sum(acc_gb);
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) acc_lam += __shfl_xor(acc_lam, off);
+  for (int off = 1; off < 64; off <<= 1) {
+    acc_gb += __shfl_xor(acc_gb, off);
+    acc_lam += __shfl_xor(acc_lam, off);
+    acc_tau += __shfl_xor(acc_tau, off);
+  }
 #pragma unroll
   for (int p = 0; p < NT; ++p) acc_ab[p] += __shfl_xor(acc_ab[p], 32);
   __syncthreads();   // every wave's G is done with
@@ -1407,8 +1569,8 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
       if (NT == 2 ? col < HALF : col < DA) red[w * (DA + 2) + p * HALF + col] = acc_ab[p];
   }
   if (lane == 0) {
-    red[w * (DA + 2) + DA] = acc_tau;
-    red[w * (DA + 2) + DA + 1] = acc_gb;
+    red[w * (DA + 2) + DA] = static_cast<float>(acc_tau);
+    red[w * (DA + 2) + DA + 1] = static_cast<float>(acc_gb);
     redd[w] = acc_lam;
   }
   __syncthreads();
@@ -1641,8 +1803,8 @@ int64_t addr_block_tokens(int tiles, int waves) {
 
 struct GradPlan {
   Plan p;
-  int cw, n_cg, n_rb, n_blk, addr_waves, tiles;
-  size_t off_dnum, off_dden, off_dotw, off_dotr, off_p1, off_pf, off_pd, off_pk, off_sums, off_chains, total;
+  int cw, n_cg, n_xg, n_rb, n_blk, addr_waves, tiles;   // n_xg: column groups of chunk_grad_kernel
+  size_t off_dnum, off_dden, off_dv, off_dotw, off_dotr, off_p1, off_pf, off_pd, off_pk, off_sums, off_chains, total;
 };
 
 // widest column group (32, 16, 8) whose grad_scan slab fits in LDS
@@ -1662,6 +1824,7 @@ int make_grad_plan(const sdm_rt_dims* d, GradPlan* g) {
   g->addr_waves = addr_grad_waves(p.n_sub, p.half, p.pitch);
   if (!g->addr_waves) return set_err(SDM_RT_EUNSUPPORTED, "backward: n_sub = %d sub-keys do not fit in LDS", p.n_sub);
   g->n_cg = p.dh / g->cw;
+  g->n_xg = (p.dh + 63) / 64;
   const int64_t N = static_cast<int64_t>(p.B) * p.T;
   g->n_rb = static_cast<int>((N + kReadGradRows - 1) / kReadGradRows);
   g->tiles = addr_tiles(p, 2);
@@ -1674,10 +1837,12 @@ int make_grad_plan(const sdm_rt_dims* d, GradPlan* g) {
   o = align_up(o + sizeof(float) * N * hd, 256);
   g->off_dden = o;
   o = align_up(o + sizeof(float) * N * p.H, 256);
-  g->off_dotw = o;
-  o = align_up(o + sizeof(float) * g->n_cg * picks, 256);
+  g->off_dv = o;
+  o = align_up(o + sizeof(float) * N * hd, 256);
+  g->off_dotw = o;   // the scans' column groups, then chunk_grad_kernel's
+  o = align_up(o + sizeof(float) * (g->n_cg + g->n_xg) * picks, 256);
   g->off_dotr = o;
-  o = align_up(o + sizeof(float) * g->n_cg * picks, 256);
+  o = align_up(o + sizeof(float) * (g->n_cg + g->n_xg) * picks, 256);
   g->off_p1 = o;
   o = align_up(o + sizeof(float) * g->n_rb * hd, 256);
   g->off_pf = o;
@@ -1696,20 +1861,8 @@ int make_grad_plan(const sdm_rt_dims* d, GradPlan* g) {
 }
 
 template <int CW, int KP, bool REV, typename WT, typename RT>
-int launch_grad_scan_t(const GradPlan& g, const GradScanArgs& a, hipStream_t st) {
+int launch_grad_scan_t(const GradPlan& g, const GradScanArgs& a, const ChainArgs& c, hipStream_t st) {
   {
-    ChainArgs c{};
-    c.w_slot = a.w_slot;
-    c.w_wt = a.w_wt;
-    c.reset = a.reset;
-    c.decay = a.decay;
-    c.chains = const_cast<unsigned char*>(a.chains);
-    c.B = a.B;
-    c.T = a.T;
-    c.H = a.H;
-    c.M = a.M;
-    c.kk = a.kk;
-    c.n_chunks = a.n_chunks;
     hipLaunchKernelGGL((chain_plan_kernel<KP, REV>), dim3(a.n_chunks, a.H, a.B), dim3(64),
                        sizeof(unsigned long long) * a.M, st, c);
     if (int rc = check_launch("chain plan")) return rc;
@@ -1725,13 +1878,30 @@ int launch_grad_scan_t(const GradPlan& g, const GradScanArgs& a, hipStream_t st)
 }
 
 template <bool REV, typename WT, typename RT>
-int launch_grad_scan(const GradPlan& g, const GradScanArgs& a, hipStream_t st) {
+int launch_grad_scan(const GradPlan& g, const GradScanArgs& a, const ChainArgs& ch, hipStream_t st) {
   const bool k8 = g.p.pitch == 8;
   switch (g.cw) {
-    case 32: return k8 ? launch_grad_scan_t<32, 8, REV, WT, RT>(g, a, st) : launch_grad_scan_t<32, 16, REV, WT, RT>(g, a, st);
-    case 16: return k8 ? launch_grad_scan_t<16, 8, REV, WT, RT>(g, a, st) : launch_grad_scan_t<16, 16, REV, WT, RT>(g, a, st);
-    default: return k8 ? launch_grad_scan_t<8, 8, REV, WT, RT>(g, a, st) : launch_grad_scan_t<8, 16, REV, WT, RT>(g, a, st);
+    case 32: return k8 ? launch_grad_scan_t<32, 8, REV, WT, RT>(g, a, ch, st) : launch_grad_scan_t<32, 16, REV, WT, RT>(g, a, ch, st);
+    case 16: return k8 ? launch_grad_scan_t<16, 8, REV, WT, RT>(g, a, ch, st) : launch_grad_scan_t<16, 16, REV, WT, RT>(g, a, ch, st);
+    default: return k8 ? launch_grad_scan_t<8, 8, REV, WT, RT>(g, a, ch, st) : launch_grad_scan_t<8, 16, REV, WT, RT>(g, a, ch, st);
   }
+}
+
+template <typename VT>
+int launch_chunk_grad(const GradPlan& g, const ChunkGradArgs& a, hipStream_t st) {
+  const Plan& p = g.p;
+  const dim3 grid(p.n_chunks, p.H * g.n_xg, p.B);
+  const size_t lds = ChunkGradLds(p.M, p.pitch).total;
+  if (p.pitch == 8) {
+    static const bool ok = allow_lds(reinterpret_cast<const void*>(&chunk_grad_kernel<8, VT>));
+    if (!ok) return lds_err("chunk grad");
+    hipLaunchKernelGGL((chunk_grad_kernel<8, VT>), grid, dim3(kGradScanThreads), lds, st, a);
+  } else {
+    static const bool ok = allow_lds(reinterpret_cast<const void*>(&chunk_grad_kernel<16, VT>));
+    if (!ok) return lds_err("chunk grad");
+    hipLaunchKernelGGL((chunk_grad_kernel<16, VT>), grid, dim3(kGradScanThreads), lds, st, a);
+  }
+  return check_launch("chunk grad");
 }
 
 template <int HALF, typename InT>
@@ -1993,54 +2163,65 @@ int sdm_rt_backward_typed(const sdm_rt_dims* dims, const sdm_rt_params* params, 
     }
     if ((rc = check_launch("read grad"))) return rc;
   }
-  // 2. forward replay: dwr
+  // 2. the chunks' own writes: parts of dwr, dww and dV
+  float* dv_in = reinterpret_cast<float*>(ws + g.off_dv);
   {
-    GradScanArgs a{};
-    a.w_slot = saved->slots_w;
-    a.w_wt = saved->weights_w;
-    a.r_slot = saved->slots_r;
-    a.r_wt = saved->weights_r;
-    a.wv = v;
-    a.wv_stride = v_row_stride;
-    a.wc = nullptr;
-    a.rv = dnum;
-    a.rv_stride = wv;
-    a.rc = dden;
+    ChunkGradArgs a{};
+    a.slot[0] = saved->slots_w;
+    a.slot[1] = saved->slots_r;
+    a.wt[0] = saved->weights_w;
+    a.wt[1] = saved->weights_r;
+    a.v = v;
+    a.v_stride = v_row_stride;
+    a.dnum = dnum;
+    a.dden = dden;
     a.reset = reset;
     a.decay = params->decay;
-    a.dot_out = dotr;
-    a.sum_out = nullptr;
+    const int64_t picks = N * p.H * p.pitch;
+    a.dot_w = dotw + g.n_cg * picks;
+    a.dot_r = dotr + g.n_cg * picks;
+    a.dv = dv_in;
     a.B = p.B;
     a.T = p.T;
     a.H = p.H;
     a.dh = p.dh;
     a.M = p.M;
     a.kk = p.kk;
-    a.n_chunks = p.n_chunks;
-    a.chains = reinterpret_cast<const unsigned char*>(ws + g.off_chains);
-    rc = in_dtype == SDM_RT_BF16 ? launch_grad_scan<false, bf16_t, float>(g, a, st)
-                                 : launch_grad_scan<false, float, float>(g, a, st);
+    a.n_xg = g.n_xg;
+    rc = in_dtype == SDM_RT_BF16 ? launch_chunk_grad<bf16_t>(g, a, st) : launch_chunk_grad<float>(g, a, st);
     if (rc) return rc;
   }
-  // 3. reverse scan: dww and dV
-  {
+  // 3. the carried memory: forward replay (dwr), then the reverse scan (dww and dV)
+  for (int rev = 0; rev < 2; ++rev) {
+    ChainArgs c{};
+    c.w_slot = rev ? saved->slots_r : saved->slots_w;
+    c.w_wt = rev ? saved->weights_r : saved->weights_w;
+    c.reset = reset;
+    c.decay = params->decay;
+    c.chains = reinterpret_cast<unsigned char*>(ws + g.off_chains);
+    c.B = p.B;
+    c.T = p.T;
+    c.H = p.H;
+    c.M = p.M;
+    c.kk = p.kk;
+    c.n_chunks = p.n_chunks;
     GradScanArgs a{};
-    a.w_slot = saved->slots_r;
-    a.w_wt = saved->weights_r;
-    a.r_slot = saved->slots_w;
-    a.r_wt = saved->weights_w;
-    a.wv = dnum;
-    a.wv_stride = wv;
-    a.wc = dden;
-    a.rv = v;
-    a.rv_stride = v_row_stride;
-    a.rc = nullptr;
-    a.reset = reset;
+    a.r_slot = rev ? saved->slots_w : saved->slots_r;
+    a.r_wt = rev ? saved->weights_w : saved->weights_r;
+    a.wv = rev ? dnum : v;
+    a.wv_stride = rev ? wv : v_row_stride;
+    a.wc = rev ? dden : nullptr;
+    a.rv = rev ? v : dnum;
+    a.rv_stride = rev ? v_row_stride : wv;
+    a.rc = rev ? nullptr : dden;
     a.decay = params->decay;
-    a.dot_out = dotw;
-    a.sum_out = grads->d_v;
-    a.sum_stride = grads->d_v_row_stride;
-    a.sum_bf16 = grad_dtype == SDM_RT_BF16;
+    a.dot_out = rev ? dotw : dotr;
+    if (rev) {
+      a.sum_in = dv_in;
+      a.sum_out = grads->d_v;
+      a.sum_stride = grads->d_v_row_stride;
+      a.sum_bf16 = grad_dtype == SDM_RT_BF16;
+    }
     a.B = p.B;
     a.T = p.T;
     a.H = p.H;
@@ -2048,9 +2229,17 @@ int sdm_rt_backward_typed(const sdm_rt_dims* dims, const sdm_rt_params* params, 
     a.M = p.M;
     a.kk = p.kk;
     a.n_chunks = p.n_chunks;
-    a.chains = reinterpret_cast<const unsigned char*>(ws + g.off_chains);
-    rc = in_dtype == SDM_RT_BF16 ? launch_grad_scan<true, float, bf16_t>(g, a, st)
-                                 : launch_grad_scan<true, float, float>(g, a, st);
+    a.chains = c.chains;
+    auto aligned = [](const void* p, int64_t stride, size_t piece) {   // every row's pieces start on their size
+      return reinterpret_cast<uintptr_t>(p) % piece == 0 && stride % static_cast<int64_t>(piece) == 0;
+    };
+    const size_t in_es = in_dtype == SDM_RT_BF16 ? 2 : 4, cpl = g.cw / 8;
+    a.vec = aligned(a.r_slot, 0, 16) && aligned(a.r_wt, 0, 16) &&
+            aligned(v, v_row_stride * static_cast<int64_t>(in_es), in_es * cpl);
+    const bool b16 = in_dtype == SDM_RT_BF16;
+    rc = rev ? (b16 ? launch_grad_scan<true, float, bf16_t>(g, a, c, st) : launch_grad_scan<true, float, float>(g, a, c, st))
+             : (b16 ? launch_grad_scan<false, bf16_t, float>(g, a, c, st)
+                    : launch_grad_scan<false, float, float>(g, a, c, st));
     if (rc) return rc;
   }
   // 4. softmax, gate and address backward
@@ -2075,7 +2264,7 @@ int sdm_rt_backward_typed(const sdm_rt_dims* dims, const sdm_rt_params* params, 
     a.score[1] = saved->scores_r;
     a.dot[0] = dotw;
     a.dot[1] = dotr;
-    a.n_cg = g.n_cg;
+    a.n_cg = g.n_cg + g.n_xg;
     a.dz[0] = grads->d_kz;
     a.dz[1] = grads->d_qz;
     a.dz_stride[0] = grads->d_kz_row_stride;

@@ -161,6 +161,18 @@ def test_address_gradients_at_tile_edges(B, T, H, dh, d_a, n_sub, k, dtype):
     check_case("tile", 31, B, T, H, dh, d_a, n_sub, k, dtype=dtype, overlap=0.8)
 
 
+@pytest.mark.parametrize("T,dh,k,reset_p,overlap,dtype", [
+    (1, 64, 8, 0.0, 0.8, torch.float32), (63, 64, 8, 0.1, 0.9, torch.float32), (64, 64, 8, 0.0, 0.9, torch.bfloat16),
+    (65, 72, 8, 0.1, 0.9, torch.float32), (127, 128, 16, 0.02, 0.9, torch.float32),
+    (193, 200, 8, 0.01, 0.7, torch.bfloat16),   # the reverse scan starts with a chunk of one token; 4 column groups
+    (200, 24, 4, 0.2, 0.9, torch.float32),
+])
+def test_in_chunk_and_carried_gradients_at_chunk_edges(T, dh, k, reset_p, overlap, dtype):
+    """chunk_grad_kernel's pairs of one chunk and the scans' carried part meet at chunk edges, resets and 64-column
+    groups."""
+    check_case("chunk", 41, 2, T, 2, dh, 16, 8, k, dtype=dtype, reset_p=reset_p, overlap=overlap)
+
+
 def test_backward_is_deterministic():
     t, reset = make(16, 1, 200, 4, 32, 16, 8, overlap=0.7)
     cfg = dict(k=8, read_mode="mean", out_norm=True, read_eps=1e-3, out_norm_eps=1e-2)
