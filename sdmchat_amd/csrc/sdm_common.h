@@ -1429,6 +1429,7 @@ struct CoreIO {
   float* state_out_cnt;
   float* read_out;
   float* den_out;
+  const sdm_rt_saved* saved;   // the training forward's picks, weights and scores, or nullptr
 };
 int run_core(const Plan& p, const sdm_rt_dims* dims, const sdm_rt_params* prm, const CoreIO& io, void* workspace,
              hipStream_t st);

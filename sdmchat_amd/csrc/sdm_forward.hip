@@ -69,6 +69,11 @@ int run_core(const Plan& p, const sdm_rt_dims* dims, const sdm_rt_params* prm, c
   pa.plans = plans;
   pa.sizes = sizes;
   pa.sync = sync;
+  for (int i = 0; i < 2 && io.saved; ++i) {
+    pa.slot_out[i] = i ? io.saved->slots_r : io.saved->slots_w;
+    pa.w_out[i] = i ? io.saved->weights_r : io.saved->weights_w;
+    pa.s_out[i] = i ? io.saved->scores_r : io.saved->scores_w;
+  }
   pa.groups = p.groups;
   pa.xch = pick && dims->out_norm && p.dh / cw > 1 ? reinterpret_cast<unsigned long long*>(xch) : nullptr;
   pa.xgroups = p.dh / cw;

@@ -1594,51 +1594,83 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
   }
 }
 
-// the per-head sums to the parameter gradients: sums[h][F] = (dtau, d gate bias, d addr_b[DA]) and lam dL/dlam
-__global__ void __launch_bounds__(128) addr_post_kernel(const double* __restrict__ sums, const double* __restrict__ lam,
-                                                        int DA, const float* __restrict__ log_scale, float* d_log_scale,
-                                                        float* d_gate_bias, float* d_addr_b, float* d_log_decay) {
-  const int h = blockIdx.x;
-  const int F = 2 + DA;
-  for (int f = threadIdx.x; f <= F; f += blockDim.x) {
-    if (f == F) {
-      if (d_log_decay) d_log_decay[h] = static_cast<float>(lam[h]);
-    } else if (f == 0) {
-      if (d_log_scale) d_log_scale[h] = static_cast<float>(sums[h * F] * static_cast<double>(expf(log_scale[h])));
-    } else if (f == 1) {
-      if (d_gate_bias) d_gate_bias[h] = static_cast<float>(sums[h * F + 1]);
-    } else if (d_addr_b) {
-      d_addr_b[h * DA + (f - 2)] = static_cast<float>(sums[h * F + f]);
+// The parameter gradients from the blocks' partial records, all in one launch (seven of them, each a few microseconds
+// of launch and round trips, took 34 us of a backward; this one takes 8): block ranges by what they sum, 64 items a
+// block (reduce_item), in float64.
+//   keys    whole sub-key rows, 64 / half a block; from the summed unit sub-key gradient dk^ the raw one (F.normalize
+//           backward): dK = (dk^ - k^ <k^, dk^>) / |K|   (dk^ / 1e-12 below the floor)
+//   fields  [H][2 + d_a]: dtau (times tau: the gradient with respect to log tau), the gate bias, addr_b
+//   fades   [H]: lam dL/dlam
+//   onorm   [H][dh]
+struct GradSumsArgs {
+  const float* pk;        // [n_rec][H][2][n_sub][half]
+  const float* pf;        // [n_rec][H][2 + DA]
+  const double* pd;       // [n_rec][H]
+  const float* p1;        // [n_rb][H * dh]
+  int n_rec, n_rb, H, DA, n_sub, half, n_onorm;
+  int key_blocks, field_blocks, fade_blocks;   // the onorm blocks follow
+  const float* keys[2];
+  const float* log_scale;
+  float* d_keys[2];
+  float* d_log_scale;
+  float* d_gate_bias;
+  float* d_addr_b;
+  float* d_log_decay;
+  float* d_onorm;
+};
+
+__global__ void __launch_bounds__(64 * kRedGroups) grad_sums_kernel(GradSumsArgs a) {
+  __shared__ double red[kRedGroups][64];
+  __shared__ float dkn[64], key[64];
+  const int l = threadIdx.x & 63;
+  const bool first = threadIdx.x < 64;   // the lanes that hold the sums
+  int blk = blockIdx.x;
+  if (blk < a.key_blocks) {
+    const int rows = 64 / a.half;
+    const int row = blk * rows + l / a.half;   // [H][2][n_sub]
+    const int n_rows = a.H * 2 * a.n_sub;
+    const bool live = l / a.half < rows && row < n_rows;
+    const int64_t i = static_cast<int64_t>(blk) * rows * a.half + l;
+    const double s = reduce_item(a.pk, a.n_rec, static_cast<int64_t>(n_rows) * a.half, i, live, red);
+    const int h = row / (2 * a.n_sub), part = (row / a.n_sub) & 1, sub = row % a.n_sub;
+    const int64_t at = (static_cast<int64_t>(h) * a.n_sub + sub) * a.half + l % a.half;
+    if (first) {
+      dkn[l] = static_cast<float>(s);
+      key[l] = live ? a.keys[part][at] : 0.f;
     }
+    __syncthreads();
+    if (!first || !live) return;
+    const int c0 = l / a.half * a.half;
+    float kk = 0.f;
+    for (int c = 0; c < a.half; ++c) kk = fmaf(key[c0 + c], key[c0 + c], kk);
+    const float nk = sqrtf(kk), inv = fmaxf(nk, 1e-12f);
+    float dot = 0.f;
+    for (int c = 0; c < a.half; ++c) dot = fmaf(key[c0 + c] / inv, dkn[c0 + c], dot);
+    a.d_keys[part][at] = nk > 1e-12f ? (dkn[l] - key[l] / inv * dot) / nk : dkn[l] * 1e12f;
+    return;
   }
-}
-
-// raw sub-key gradient from the summed unit sub-key gradient dk^ ([H][2][n_sub][half]; F.normalize backward):
-// one wave per sub-key row, dK = (dk^ - k^ <k^, dk^>) / |K|   (dk^ / 1e-12 below the floor)
-__global__ void __launch_bounds__(64) keys_grad_kernel(const double* __restrict__ dkn_sum, int n_sub, int half,
-                                                       const float* __restrict__ keys1,
-                                                       const float* __restrict__ keys2, float* d_keys1,
-                                                       float* d_keys2) {
-  const int row = blockIdx.x;                 // [H][2][n_sub]
-  const int h = row / (2 * n_sub);
-  const int part = (row / n_sub) & 1;
-  const int i = row % n_sub;
-  const int c = threadIdx.x;
-  const bool live = c < half;
-  const float* key = (part ? keys2 : keys1) + (static_cast<int64_t>(h) * n_sub + i) * half;
-  float* out = (part ? d_keys2 : d_keys1);
-  const float kv = live ? key[c] : 0.f;
-  const float dkn = live ? static_cast<float>(dkn_sum[static_cast<int64_t>(row) * half + c]) : 0.f;
-  const float nk = sqrtf(wave_sum(kv * kv));
-  const float kh = kv / fmaxf(nk, 1e-12f);
-  const float dot = wave_sum(kh * dkn);
-  const float d = nk > 1e-12f ? (dkn - kh * dot) / nk : dkn * 1e12f;
-  if (live && out) out[(static_cast<int64_t>(h) * n_sub + i) * half + c] = d;
-}
-
-__global__ void __launch_bounds__(256) to_float_kernel(const double* __restrict__ in, int64_t n, float* out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) out[i] = static_cast<float>(in[i]);
+  blk -= a.key_blocks;
+  if (blk < a.field_blocks) {
+    const int F = 2 + a.DA;
+    const int64_t i = static_cast<int64_t>(blk) * 64 + l, n = static_cast<int64_t>(a.H) * F;
+    const double s = reduce_item(a.pf, a.n_rec, n, i, i < n, red);
+    if (!first || i >= n) return;
+    const int h = static_cast<int>(i / F), f = static_cast<int>(i % F);
+    if (f == 0) {
+      if (a.d_log_scale) a.d_log_scale[h] = static_cast<float>(s * static_cast<double>(expf(a.log_scale[h])));
+    } else if (f == 1) {
+      if (a.d_gate_bias) a.d_gate_bias[h] = static_cast<float>(s);
+    } else if (a.d_addr_b) {
+      a.d_addr_b[h * a.DA + (f - 2)] = static_cast<float>(s);
+    }
+    return;
+  }
+  blk -= a.field_blocks;
+  const bool fade = blk < a.fade_blocks;
+  if (!fade) blk -= a.fade_blocks;
+  const int64_t i = static_cast<int64_t>(blk) * 64 + l, n = fade ? a.H : a.n_onorm;
+  const double s = fade ? reduce_item(a.pd, a.n_rec, n, i, i < n, red) : reduce_item(a.p1, a.n_rb, n, i, i < n, red);
+  if (first && i < n) (fade ? a.d_log_decay : a.d_onorm)[i] = static_cast<float>(s);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1804,7 +1836,7 @@ int64_t addr_block_tokens(int tiles, int waves) {
 struct GradPlan {
   Plan p;
   int cw, n_cg, n_xg, n_rb, n_blk, addr_waves, tiles;   // n_xg: column groups of chunk_grad_kernel
-  size_t off_dnum, off_dden, off_dv, off_dotw, off_dotr, off_p1, off_pf, off_pd, off_pk, off_sums, off_chains, total;
+  size_t off_dnum, off_dden, off_dv, off_dotw, off_dotr, off_p1, off_pf, off_pd, off_pk, off_chains, total;
 };
 
 // widest column group (32, 16, 8) whose grad_scan slab fits in LDS
@@ -1851,9 +1883,6 @@ int make_grad_plan(const sdm_rt_dims* d, GradPlan* g) {
   o = align_up(o + sizeof(double) * 2 * g->n_blk * p.H, 256);
   g->off_pk = o;
   o = align_up(o + sizeof(float) * 2 * g->n_blk * p.H * 2 * static_cast<size_t>(p.n_sub) * p.half, 256);
-  g->off_sums = o;   // float64 sums: addressing fields [H][2 + d_a], lam [H], unit sub-keys [H][2][n_sub][half], onorm
-  o = align_up(o + sizeof(double) * (static_cast<size_t>(p.H) * (2 + p.d_a) + p.H +
-                                     static_cast<size_t>(p.H) * 2 * p.n_sub * p.half + hd), 256);
   g->off_chains = o;   // the chain plans of one scan direction at a time
   o = align_up(o + static_cast<size_t>(p.B) * p.H * p.n_chunks * chain_stride(p.pitch), 256);
   g->total = o;
@@ -1885,6 +1914,17 @@ int launch_grad_scan(const GradPlan& g, const GradScanArgs& a, const ChainArgs& 
     case 16: return k8 ? launch_grad_scan_t<16, 8, REV, WT, RT>(g, a, ch, st) : launch_grad_scan_t<16, 16, REV, WT, RT>(g, a, ch, st);
     default: return k8 ? launch_grad_scan_t<8, 8, REV, WT, RT>(g, a, ch, st) : launch_grad_scan_t<8, 16, REV, WT, RT>(g, a, ch, st);
   }
+}
+
+// the parameter gradients asked for (null outputs are left out)
+int launch_grad_sums(GradSumsArgs a, hipStream_t st) {
+  const int rows = 64 / a.half;
+  a.key_blocks = a.d_keys[0] ? (a.H * 2 * a.n_sub + rows - 1) / rows : 0;
+  a.field_blocks = (a.H * (2 + a.DA) + 63) / 64;
+  a.fade_blocks = a.d_log_decay ? (a.H + 63) / 64 : 0;
+  const int blocks = a.key_blocks + a.field_blocks + a.fade_blocks + (a.d_onorm ? (a.n_onorm + 63) / 64 : 0);
+  hipLaunchKernelGGL(grad_sums_kernel, dim3(blocks), dim3(64 * kRedGroups), 0, st, a);
+  return check_launch("gradient sums");
 }
 
 template <typename VT>
@@ -1954,7 +1994,7 @@ struct TablePlan {
   Plan p;
   int n_blk, addr_waves, tiles, key_bits;
   int64_t n_entries;
-  size_t off_dw, off_pf, off_pd, off_pk, off_sums, off_keys, off_count, off_offsets, off_cub, cub_bytes, total;
+  size_t off_dw, off_pf, off_pd, off_pk, off_keys, off_count, off_offsets, off_cub, cub_bytes, total;
 };
 
 int make_table_plan(const sdm_rt_dims* d, TablePlan* g) {
@@ -1979,8 +2019,6 @@ int make_table_plan(const sdm_rt_dims* d, TablePlan* g) {
   o = align_up(o + sizeof(double) * g->n_blk * p.H, 256);
   g->off_pk = o;
   o = align_up(o + sizeof(float) * g->n_blk * KSH, 256);
-  g->off_sums = o;
-  o = align_up(o + sizeof(double) * (static_cast<size_t>(p.H) * (2 + p.d_a) + p.H + KSH), 256);
   // the value-table gradient: sort keys and values (in and out), per-row counts and offsets, hipCUB's scratch
   g->n_entries = N * p.H * p.pitch;
   if (g->n_entries > 0x7fffffffLL) return set_err(SDM_RT_EUNSUPPORTED, "table backward: too many picks");
@@ -2044,27 +2082,6 @@ int sdm_rt_forward_train(const sdm_rt_dims* dims, const sdm_rt_params* params, c
   hipStream_t st = static_cast<hipStream_t>(stream);
   const void* gl = dims->write_gate ? gate_logits : nullptr;
 
-  // both address sets: picks, weights (gate included) and scores
-  AddrArgs aa{};
-  aa.g = addr_geom(p, params);
-  aa.z = kz;
-  aa.z_stride = kz_row_stride;
-  aa.gl = gl;
-  aa.g_stride = gate_row_stride;
-  aa.B = p.B;
-  aa.T = p.T;
-  aa.pitch = p.pitch;
-  aa.slot_out = saved->slots_w;
-  aa.w_out = saved->weights_w;
-  aa.s_out = saved->scores_w;
-  aa.z2 = qz;
-  aa.z2_stride = qz_row_stride;
-  aa.slot_out2 = saved->slots_r;
-  aa.w_out2 = saved->weights_r;
-  aa.s_out2 = saved->scores_r;
-  rc = launch_address(p, aa, in_dtype, st);
-  if (rc) return rc;
-
   CoreIO io{};
   io.kz = kz;
   io.kz_stride = kz_row_stride;
@@ -2079,6 +2096,7 @@ int sdm_rt_forward_train(const sdm_rt_dims* dims, const sdm_rt_params* params, c
   io.r_out = r_out;
   io.r_stride = out_row_stride;
   io.out_dtype = out_dtype;
+  io.saved = saved;   // the plan kernel's picks, weights (gate included) and scores
   io.read_out = saved->read;
   io.den_out = dims->read_mean ? saved->den : nullptr;
   return run_core(p, dims, params, io, workspace, st);
@@ -2284,39 +2302,33 @@ int sdm_rt_backward_typed(const sdm_rt_dims* dims, const sdm_rt_params* params, 
                                  : by_half<AddrGradLaunch, float>(p.half, g, a, st);
     if (rc) return rc;
   }
-  // 5. parameter sums (fixed order, float64)
+  // 5. parameter sums
   {
-    double* sums_f = reinterpret_cast<double*>(ws + g.off_sums);
-    double* sums_d = sums_f + static_cast<size_t>(p.H) * (2 + p.d_a);
-    double* sums_k = sums_d + p.H;
-    double* sums_o = sums_k + static_cast<size_t>(p.H) * 2 * p.n_sub * p.half;
-    const int n_rec = 2 * g.n_blk;
-    auto reduce = [&](auto* part, int nr, int64_t items, double* out) {
-      using T = std::remove_const_t<std::remove_pointer_t<decltype(part)>>;
-      hipLaunchKernelGGL(reduce_records_kernel<T>, dim3(static_cast<unsigned>((items + 63) / 64)), dim3(64 * kRedGroups),
-                         0, st, part, nr, items, items, out);
-      return check_launch("reduce");
-    };
-    const int64_t F = 2 + p.d_a;
-    const int64_t KSH = static_cast<int64_t>(p.H) * 2 * p.n_sub * p.half;
-    if ((rc = reduce(static_cast<const float*>(pf), n_rec, p.H * F, sums_f))) return rc;
-    if ((rc = reduce(static_cast<const double*>(pd), n_rec, p.H, sums_d))) return rc;
-    hipLaunchKernelGGL(addr_post_kernel, dim3(p.H), dim3(128), 0, st, sums_f, sums_d, p.d_a, params->log_scale,
-                       grads->d_log_scale, grads->d_gate_bias, grads->d_addr_b, grads->d_log_decay);
-    if ((rc = check_launch("addr post"))) return rc;
-    if (grads->d_keys1 || grads->d_keys2) {
-      if (!grads->d_keys1 || !grads->d_keys2) return set_err(SDM_RT_EINVAL, "grads: give both d_keys1 and d_keys2");
-      if ((rc = reduce(static_cast<const float*>(pk), n_rec, KSH, sums_k))) return rc;
-      hipLaunchKernelGGL(keys_grad_kernel, dim3(p.H * 2 * p.n_sub), dim3(64), 0, st, sums_k, p.n_sub, p.half,
-                         params->keys1, params->keys2, grads->d_keys1, grads->d_keys2);
-      if ((rc = check_launch("keys grad"))) return rc;
-    }
-    if (grads->d_onorm_w && onw) {
-      if ((rc = reduce(static_cast<const float*>(p1), g.n_rb, wv, sums_o))) return rc;
-      hipLaunchKernelGGL(to_float_kernel, dim3(static_cast<unsigned>((wv + 255) / 256)), dim3(256), 0, st, sums_o, wv,
-                         grads->d_onorm_w);
-      if ((rc = check_launch("onorm"))) return rc;
-    }
+    if ((grads->d_keys1 == nullptr) != (grads->d_keys2 == nullptr))
+      return set_err(SDM_RT_EINVAL, "grads: give both d_keys1 and d_keys2");
+    GradSumsArgs a{};
+    a.pk = pk;
+    a.pf = pf;
+    a.pd = pd;
+    a.p1 = p1;
+    a.n_rec = 2 * g.n_blk;
+    a.n_rb = g.n_rb;
+    a.H = p.H;
+    a.DA = p.d_a;
+    a.n_sub = p.n_sub;
+    a.half = p.half;
+    a.n_onorm = static_cast<int>(wv);
+    a.keys[0] = params->keys1;
+    a.keys[1] = params->keys2;
+    a.log_scale = params->log_scale;
+    a.d_keys[0] = grads->d_keys1;
+    a.d_keys[1] = grads->d_keys2;
+    a.d_log_scale = grads->d_log_scale;
+    a.d_gate_bias = grads->d_gate_bias;
+    a.d_addr_b = grads->d_addr_b;
+    a.d_log_decay = grads->d_log_decay;
+    a.d_onorm = onw ? grads->d_onorm_w : nullptr;
+    if ((rc = launch_grad_sums(a, st))) return rc;
   }
   return SDM_RT_OK;
 }
@@ -2445,30 +2457,22 @@ int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, 
                                  : by_half<AddrGradLaunch, float>(p.half, gp, a, st);
     if (rc) return rc;
   }
-  // 4. parameter sums (fixed order, float64)
-  double* sums_f = reinterpret_cast<double*>(ws + g.off_sums);
-  double* sums_d = sums_f + static_cast<size_t>(p.H) * (2 + p.d_a);
-  double* sums_k = sums_d + p.H;
-  const int64_t F = 2 + p.d_a;
-  const int64_t KSH = static_cast<int64_t>(p.H) * 2 * p.n_sub * p.half;
-  hipLaunchKernelGGL(reduce_records_kernel<float>, dim3(static_cast<unsigned>((p.H * F + 63) / 64)),
-                     dim3(64 * kRedGroups), 0, st, static_cast<const float*>(pf), g.n_blk, p.H * F, p.H * F, sums_f);
-  if ((rc = check_launch("reduce"))) return rc;
-  hipLaunchKernelGGL(reduce_records_kernel<double>, dim3(static_cast<unsigned>((p.H + 63) / 64)),
-                     dim3(64 * kRedGroups), 0, st, static_cast<const double*>(pd), g.n_blk, p.H, p.H, sums_d);
-  if ((rc = check_launch("reduce"))) return rc;
-  hipLaunchKernelGGL(addr_post_kernel, dim3(p.H), dim3(128), 0, st, sums_f, sums_d, p.d_a, params->log_scale,
-                     d_log_scale, nullptr, nullptr, nullptr);
-  if ((rc = check_launch("addr post"))) return rc;
-  if (d_keys1) {
-    hipLaunchKernelGGL(reduce_records_kernel<float>, dim3(static_cast<unsigned>((KSH + 63) / 64)),
-                       dim3(64 * kRedGroups), 0, st, static_cast<const float*>(pk), g.n_blk, KSH, KSH, sums_k);
-    if ((rc = check_launch("reduce"))) return rc;
-    hipLaunchKernelGGL(keys_grad_kernel, dim3(p.H * 2 * p.n_sub), dim3(64), 0, st, sums_k, p.n_sub, p.half,
-                       params->keys1, params->keys2, d_keys1, d_keys2);
-    if ((rc = check_launch("keys grad"))) return rc;
-  }
-  return SDM_RT_OK;
+  // 4. parameter sums
+  GradSumsArgs a{};
+  a.pk = pk;
+  a.pf = pf;
+  a.n_rec = g.n_blk;
+  a.H = p.H;
+  a.DA = p.d_a;
+  a.n_sub = p.n_sub;
+  a.half = p.half;
+  a.keys[0] = params->keys1;
+  a.keys[1] = params->keys2;
+  a.log_scale = params->log_scale;
+  a.d_keys[0] = d_keys1;
+  a.d_keys[1] = d_keys2;
+  a.d_log_scale = d_log_scale;
+  return launch_grad_sums(a, st);
 }
 
 }  // extern "C"

@@ -44,6 +44,11 @@ struct PlanArgs {
   uint32_t* sync;          // [B*H][groups] scan progress counters, then a status word: zeroed here, or nullptr
   unsigned long long* xch; // pick plans: [B*H][n_chunks][xgroups][64] out-norm partial sums, cleared here, or nullptr
   void* gate_copy;         // [B*T][H] of the input type: the gate logits as read (rows of H), or nullptr
+  // the training forward's picks, weights (gate included) and scores of the write and read set, [B][H][T][KP] with pads
+  // slot -1, or all nullptr.  Addressing them again in a kernel of its own took 45 us at B=8, T=2048 (12 heads, k=8)
+  int32_t* slot_out[2];
+  float* w_out[2];
+  float* s_out[2];
   int groups;
   int xgroups;             // column groups of the pick scan
   int row_bytes;           // bytes of a slab row in the scan's LDS (its column group width * 4)
@@ -254,6 +259,15 @@ __global__ void __launch_bounds__(128, 3) plan_kernel(PlanArgs a) {
     } else if (p < L) {
       address_one<HALF, KP, InT>(a.g, h, kn, zb + (row0 + p) * zs + static_cast<int64_t>(h) * 2 * HALF, gate, slot, w,
                                  sc);
+    }
+    if (a.slot_out[0] && p < L) {
+      const int64_t at = ((static_cast<int64_t>(b) * a.g.H + h) * a.T + c0 + p) * KP;
+      float si[KP];
+#pragma unroll
+      for (int j = 0; j < KP; ++j) si[j] = __int_as_float(j < kk ? slot[j] : -1);
+      store_vals<KP, float>(reinterpret_cast<float*>(a.slot_out[set]) + at, si);
+      store_vals<KP, float>(a.w_out[set] + at, w);
+      store_vals<KP, float>(a.s_out[set] + at, sc);
     }
 #pragma unroll
     for (int j = 0; j < KP; ++j) {

@@ -4,21 +4,19 @@
 
 namespace sdmrt {
 
-// Sums over records: out[i] = sum_r part[r * rec_stride + i] (r < n_rec) in float64 for n_items items.  Block of
-// 64 x 16 threads: lane i of group rg sums records rg, rg + 16, ... (loads issued together), then the 16 group sums
-// are added in group order: a fixed order, so the result is deterministic.
+// The sum over n_rec records of part[r * rec_stride + i] for item i (nothing where !live), in float64: block of 64 x 16
+// threads, lane l of group rg sums records rg, rg + 16, ... of its item (loads issued together), then the 16 group
+// sums are added in group order: a fixed order, so the result is deterministic.  Every thread calls it; the sums are
+// returned in group 0's lanes.  red: 16 x 64 doubles of LDS, free again after the next __syncthreads
 constexpr int kRedGroups = 16;
 
-template <typename T, typename OutT = double>
-__global__ void __launch_bounds__(64 * kRedGroups) reduce_records_kernel(const T* __restrict__ part, int n_rec,
-                                                                        int64_t rec_stride, int64_t n_items,
-                                                                        OutT* __restrict__ out) {
-  __shared__ double red[kRedGroups][64];
+template <typename T>
+__device__ __forceinline__ double reduce_item(const T* __restrict__ part, int n_rec, int64_t rec_stride, int64_t i,
+                                              bool live, double (*red)[64]) {
   const int l = threadIdx.x & 63;
   const int rg = threadIdx.x >> 6;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + l;
   double s = 0.0;
-  if (i < n_items) {
+  if (live) {
     constexpr int kBatch = 16;
     for (int r0 = rg; r0 < n_rec; r0 += kRedGroups * kBatch) {
       T v[kBatch];
@@ -33,11 +31,21 @@ __global__ void __launch_bounds__(64 * kRedGroups) reduce_records_kernel(const T
   }
   red[rg][l] = s;
   __syncthreads();
-  if (rg == 0 && i < n_items) {
-    double t = 0.0;
+  double t = 0.0;
+  if (rg == 0)
     for (int q = 0; q < kRedGroups; ++q) t += red[q][l];
-    out[i] = static_cast<OutT>(t);
-  }
+  return t;
+}
+
+// out[i] = the sum over records of item i, for n_items items
+template <typename T>
+__global__ void __launch_bounds__(64 * kRedGroups) reduce_records_kernel(const T* __restrict__ part, int n_rec,
+                                                                        int64_t rec_stride, int64_t n_items,
+                                                                        float* __restrict__ out) {
+  __shared__ double red[kRedGroups][64];
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + (threadIdx.x & 63);
+  const double t = reduce_item(part, n_rec, rec_stride, i, i < n_items, red);
+  if (threadIdx.x < 64 && i < n_items) out[i] = static_cast<float>(t);
 }
 
 }  // namespace sdmrt

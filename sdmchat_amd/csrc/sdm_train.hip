@@ -422,7 +422,7 @@ int sdm_rt_rms_norm_backward(const void* x, int64_t x_row_stride, sdm_rt_dtype x
           : (yb ? launch_norm_bwd<float, bf16_t>(x, x_row_stride, dy, dy_row_stride, w, rows, d, eps, dx, dx_row_stride, part, st)
                 : launch_norm_bwd<float, float>(x, x_row_stride, dy, dy_row_stride, w, rows, d, eps, dx, dx_row_stride, part, st));
   if (rc || !dw) return rc;
-  hipLaunchKernelGGL((reduce_records_kernel<float, float>), dim3((d + 63) / 64), dim3(64 * kRedGroups), 0, st, part,
+  hipLaunchKernelGGL(reduce_records_kernel<float>, dim3((d + 63) / 64), dim3(64 * kRedGroups), 0, st, part,
                      norm_bwd_blocks(rows), static_cast<int64_t>(d), static_cast<int64_t>(d), dw);
   return check_launch("rms norm weight gradient");
 }
