@@ -431,8 +431,8 @@ size_t sdm_rt_table_backward_workspace_bytes(const sdm_rt_dims* dims);
  *   slots, weights, scores   [B][H][T][pitch] as sdm_rt_address wrote them for q
  *   values       [H][M][dh] value tables (dtype values_dtype); dims->head_dim = dh
  *   dy           [B*T rows] of H * dh: the gradient of the read (sdm_rt_table_read's out), dtype dy_dtype
- * writes d_q (float32 rows), d_values ([H][M][dh] float32, overwritten; each row summed over its picks in pick order:
- * the picks are sorted by slot with a stable radix sort), d_keys1 / d_keys2 (both or neither) and d_log_scale ([H] or
+ * writes d_q (float32 rows), d_values ([H][M][dh] float32, overwritten; each row summed over its picks in pick order,
+ * in pieces: the picks are sorted by slot with a stable radix sort), d_keys1 / d_keys2 (both or neither) and d_log_scale ([H] or
  * NULL).  Every sum runs in a fixed order, so the result is deterministic. */
 int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params,
                           const void* q, int64_t q_row_stride, sdm_rt_dtype in_dtype,

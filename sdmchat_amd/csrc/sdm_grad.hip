@@ -1679,8 +1679,8 @@ __global__ void __launch_bounds__(64 * kRedGroups) grad_sums_kernel(GradSumsArgs
 //                                                           backward takes; one wave per (token, head), lane l takes
 //                                                           columns 4l, 4l + 256, ...)
 //   d_values[h][s]       = sum over the picks (n, j) of slot s of w_j dy[n][h]   (table_values_grad_kernel: the picks
-//                          sorted by (head, slot) with a stable radix sort, so each row is one wave's sum in pick
-//                          order -- no atomics, a fixed order)
+//                          sorted by (head, slot) with a stable radix sort and summed in pieces in pick order -- no
+//                          float atomics, a fixed order)
 template <int KP, typename VT, typename DyT>
 __global__ void __launch_bounds__(256) table_grad_kernel(const int32_t* __restrict__ slots,
                                                          const float* __restrict__ wts,
@@ -1747,25 +1747,37 @@ __global__ void __launch_bounds__(256) pick_keys_kernel(const int32_t* __restric
   vals[e] = static_cast<int32_t>(e);
 }
 
-// d_values[h][s] = sum of w_e dy[n_e][h] over the picks e of (h, s), in the sorted (entry) order; one wave per row,
-// lane l takes columns 4l, 4l + 256, ...; four picks' loads in flight at a time
+// d_values[h][s] = sum of w_e dy[n_e][h] over the picks e of (h, s), in two launches.  The sorted picks are cut every
+// kValuesSeg entries and a wave sums one piece's runs of equal keys in pick order, lane l columns 4l, 4l + 256, ...: a
+// run that is its whole row goes to d_values, one that crosses an edge of the piece to part: [2 s] continues a row
+// begun before piece s, [2 s + 1] begins a row that goes on after it.  table_values_join_kernel adds a row's pieces in
+// order and clears the rows without a pick.  The load follows the picks and not the rows: text repeats its tokens, so a
+// few rows hold hundreds of picks, and with one wave per row the longest row's chain of batches was the kernel's time
+// (B=4, T=1024, 4,096 rows of 768, k=16, a Zipf stream: 190 us; now 49 us and the join's 6; the
+// floor is the 101 MB of dy rows gathered through the caches).  Pieces of 32: the partial sums then take at most a
+// quarter of the gathered bytes again, and 2,048 waves are all resident at three to a SIMD.
+constexpr int kValuesSeg = 32;
+
 template <typename DyT>
-__global__ void __launch_bounds__(256) table_values_grad_kernel(const int32_t* __restrict__ sorted_vals,
+__global__ void __launch_bounds__(256) table_values_grad_kernel(const int32_t* __restrict__ sorted_keys,
+                                                                const int32_t* __restrict__ sorted_vals,
                                                                 const int32_t* __restrict__ offsets,
-                                                                const int32_t* __restrict__ count,
                                                                 const float* __restrict__ wts,
                                                                 const DyT* __restrict__ dy, int64_t dy_stride,
-                                                                float* __restrict__ d_values, int T, int H, int KP,
-                                                                int M, int dh) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);   // h * M + s
+                                                                float* __restrict__ d_values,
+                                                                float* __restrict__ part, int T, int H, int KP, int M,
+                                                                int dh) {
   const int lane = threadIdx.x & 63;
-  if (row >= static_cast<int64_t>(H) * M) return;   // whole waves
-  const int h = static_cast<int>(row / M);
-  const int off = offsets[row];
-  const int cnt = count[row];
-  float* dst = d_values + row * dh;
+  const int seg = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + (threadIdx.x >> 6));
+  const int live = offsets[H * M];   // the pads' key comes last
+  const int64_t begin = static_cast<int64_t>(seg) * kValuesSeg;
+  if (begin >= live) return;   // whole waves
+  const int i_begin = static_cast<int>(begin);
+  const int n = min(kValuesSeg, live - i_begin);
+  const int before = i_begin > 0 ? sorted_keys[i_begin - 1] : -1;
+  const int after = i_begin + n < live ? sorted_keys[i_begin + n] : -1;
   // up to CS column steps of 256 held in registers; the picks QS at a time: their indexes and weights, then every
-  // row segment, all loads of a batch in flight together; the sum runs in pick order
+  // row segment, all loads of a batch in flight together
   constexpr int CS = 4, QS = 8;
   for (int cb = 0; cb < dh; cb += 256 * CS) {
     float acc[CS][4];
@@ -1773,38 +1785,91 @@ __global__ void __launch_bounds__(256) table_values_grad_kernel(const int32_t* _
     for (int s = 0; s < CS; ++s)
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[s][c] = 0.f;
-    for (int i0 = 0; i0 < cnt; i0 += QS) {
+    int cur = sorted_keys[i_begin];
+    bool first = true;   // the run of cur begins at the piece's first entry
+    auto flush = [&](bool last) {
+      float* dst = d_values + static_cast<int64_t>(cur) * dh;
+      if (first && cur == before) {
+        dst = part + 2 * static_cast<int64_t>(seg) * dh;
+      } else if (last && cur == after) {
+        dst = part + (2 * static_cast<int64_t>(seg) + 1) * dh;
+      }
+#pragma unroll
+      for (int s = 0; s < CS; ++s) {
+        const int c0 = cb + 256 * s + 4 * lane;
+        if (c0 < dh) store_vals<4, float>(dst + c0, acc[s]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[s][c] = 0.f;
+      }
+    };
+    for (int i0 = 0; i0 < n; i0 += QS) {
       int64_t ro[QS];
       float w[QS];
+      int key[QS];
 #pragma unroll
       for (int q = 0; q < QS; ++q) {
-        const int i = min(i0 + q, cnt - 1);
-        const int64_t e = sorted_vals[off + i];   // ((b * H + h) * T + t) * KP + j
-        const int64_t u = e / KP;
-        const int64_t b = u / (static_cast<int64_t>(H) * T);
-        const int64_t t = u - (b * H + h) * T;
-        w[q] = i0 + q < cnt ? wts[e] : 0.f;
-        ro[q] = (b * T + t) * dy_stride + static_cast<int64_t>(h) * dh;
+        const int i = i_begin + min(i0 + q, n - 1);
+        const uint32_t e = static_cast<uint32_t>(sorted_vals[i]);   // ((b * H + h) * T + t) * KP + j, below 2^31
+        const uint32_t u = e / static_cast<uint32_t>(KP);
+        const uint32_t bh = u / static_cast<uint32_t>(T);
+        const uint32_t b = bh / static_cast<uint32_t>(H);
+        const uint32_t t = u - bh * static_cast<uint32_t>(T), h = bh - b * static_cast<uint32_t>(H);
+        w[q] = i0 + q < n ? wts[e] : 0.f;
+        key[q] = sorted_keys[i];
+        ro[q] = (static_cast<int64_t>(b) * T + t) * dy_stride + static_cast<int64_t>(h) * dh;
       }
+      float g[QS][CS][4];
 #pragma unroll
       for (int q = 0; q < QS; ++q) {
 #pragma unroll
         for (int s = 0; s < CS; ++s) {
           const int c0 = cb + 256 * s + 4 * lane;
-          if (c0 < dh) {
-            float g[4];
-            load_vals<4, DyT>(dy + ro[q] + c0, g);
+          if (c0 < dh) load_vals<4, DyT>(dy + ro[q] + c0, g[q][s]);
+        }
+      }
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[s][c] = fmaf(w[q], g[c], acc[s][c]);
-          }
+      for (int q = 0; q < QS; ++q) {
+        if (key[q] != cur) {   // the same for the whole wave
+          flush(false);
+          cur = key[q];
+          first = false;
+        }
+        if (i0 + q < n) {   // past the piece's end nothing is added: 0 * dy would keep an infinity's NaN
+#pragma unroll
+          for (int s = 0; s < CS; ++s)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[s][c] = fmaf(w[q], g[q][s][c], acc[s][c]);
         }
       }
     }
+    flush(true);
+  }
+}
+
+// d_values rows without a pick: zero; rows cut over several pieces: their partial sums in order; one wave per row
+__global__ void __launch_bounds__(256) table_values_join_kernel(const int32_t* __restrict__ offsets,
+                                                                const int32_t* __restrict__ count,
+                                                                const float* __restrict__ part,
+                                                                float* __restrict__ d_values, int n_rows, int dh) {
+  const int row = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + (threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  if (row >= n_rows) return;   // whole waves
+  const int off = offsets[row], cnt = count[row];
+  const int s0 = off / kValuesSeg, s1 = (off + max(cnt, 1) - 1) / kValuesSeg;
+  if (cnt > 0 && s0 == s1) return;   // written by its one piece
+  for (int c0 = 4 * lane; c0 < dh; c0 += 256) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    if (cnt > 0) {
+      load_vals<4, float>(part + (2 * static_cast<int64_t>(s0) + 1) * dh + c0, acc);
+#pragma unroll 8
+      for (int s = s0 + 1; s <= s1; ++s) {
+        float v[4];
+        load_vals<4, float>(part + 2 * static_cast<int64_t>(s) * dh + c0, v);
 #pragma unroll
-    for (int s = 0; s < CS; ++s) {
-      const int c0 = cb + 256 * s + 4 * lane;
-      if (c0 < dh) store_vals<4, float>(dst + c0, acc[s]);
+        for (int c = 0; c < 4; ++c) acc[c] += v[c];
+      }
     }
+    store_vals<4, float>(d_values + static_cast<int64_t>(row) * dh + c0, acc);
   }
 }
 
@@ -1994,8 +2059,11 @@ struct TablePlan {
   Plan p;
   int n_blk, addr_waves, tiles, key_bits;
   int64_t n_entries;
-  size_t off_dw, off_pf, off_pd, off_pk, off_keys, off_count, off_offsets, off_cub, cub_bytes, total;
+  size_t off_dw, off_pf, off_pd, off_pk, off_keys, off_count, off_offsets, off_part, off_cub, cub_bytes, total;
 };
+
+// pieces of the sorted picks in the value-table gradient
+int64_t values_pieces(int64_t n_entries) { return (n_entries + kValuesSeg - 1) / kValuesSeg; }
 
 int make_table_plan(const sdm_rt_dims* d, TablePlan* g) {
   int rc = make_plan(d, &g->p, false);
@@ -2031,6 +2099,8 @@ int make_table_plan(const sdm_rt_dims* d, TablePlan* g) {
   o = align_up(o + sizeof(int32_t) * n_keys, 256);
   g->off_offsets = o;
   o = align_up(o + sizeof(int32_t) * n_keys, 256);
+  g->off_part = o;
+  o = align_up(o + 2 * sizeof(float) * static_cast<size_t>(values_pieces(g->n_entries)) * p.dh, 256);
   size_t sort_bytes = 0, scan_bytes = 0;
   if (hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, static_cast<const int32_t*>(nullptr),
                                          static_cast<int32_t*>(nullptr), static_cast<const int32_t*>(nullptr),
@@ -2370,7 +2440,7 @@ int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, 
   float* pf = reinterpret_cast<float*>(ws + g.off_pf);
   double* pd = reinterpret_cast<double*>(ws + g.off_pd);
   float* pk = reinterpret_cast<float*>(ws + g.off_pk);
-  // 1. the value table gradient: picks sorted by (head, slot), then one wave per row
+  // 1. the value table gradient: picks sorted by (head, slot), summed by pieces, then the rows cut over several joined
   {
     int32_t* kin = reinterpret_cast<int32_t*>(ws + g.off_keys);
     int32_t* kout = kin + g.n_entries;
@@ -2392,17 +2462,21 @@ int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, 
     if (hipcub::DeviceRadixSort::SortPairs(ws + g.off_cub, cb, kin, kout, vin, vout, static_cast<int>(g.n_entries), 0,
                                            g.key_bits, st) != hipSuccess)
       return set_err(SDM_RT_ELAUNCH, "table backward: sort failed");
-    const unsigned rblocks = static_cast<unsigned>((static_cast<int64_t>(p.H) * p.M + 3) / 4);
+    float* part = reinterpret_cast<float*>(ws + g.off_part);
+    const unsigned sblocks = static_cast<unsigned>((values_pieces(g.n_entries) + 3) / 4);
     if (dy_dtype == SDM_RT_BF16) {
-      hipLaunchKernelGGL(table_values_grad_kernel<bf16_t>, dim3(rblocks), dim3(256), 0, st, vout, offsets, count,
-                         weights, static_cast<const bf16_t*>(dy), dy_row_stride, d_values, p.T, p.H, p.pitch, p.M,
-                         p.dh);
+      hipLaunchKernelGGL(table_values_grad_kernel<bf16_t>, dim3(sblocks), dim3(256), 0, st, kout, vout, offsets,
+                         weights, static_cast<const bf16_t*>(dy), dy_row_stride, d_values, part, p.T, p.H, p.pitch,
+                         p.M, p.dh);
     } else {
-      hipLaunchKernelGGL(table_values_grad_kernel<float>, dim3(rblocks), dim3(256), 0, st, vout, offsets, count,
-                         weights, static_cast<const float*>(dy), dy_row_stride, d_values, p.T, p.H, p.pitch, p.M,
-                         p.dh);
+      hipLaunchKernelGGL(table_values_grad_kernel<float>, dim3(sblocks), dim3(256), 0, st, kout, vout, offsets,
+                         weights, static_cast<const float*>(dy), dy_row_stride, d_values, part, p.T, p.H, p.pitch,
+                         p.M, p.dh);
     }
     if ((rc = check_launch("table values grad"))) return rc;
+    hipLaunchKernelGGL(table_values_join_kernel, dim3(static_cast<unsigned>((n_keys + 2) / 4)), dim3(256), 0, st,
+                       offsets, count, part, d_values, p.H * p.M, p.dh);
+    if ((rc = check_launch("table values join"))) return rc;
   }
   // 2. the per-pick gradients
   {

@@ -20,13 +20,15 @@ from tests.test_gpu_grad import _mixer64, _rms64
 pytestmark = pytest.mark.gpu
 
 
-def check_table(name, seed, B, T, H, dh, d_a, n_sub, k, dtype=torch.float32):
+def check_table(name, seed, B, T, H, dh, d_a, n_sub, k, dtype=torch.float32, same=0):
     say(f"[table grad] {name}: B={B} T={T} H={H} dh={dh} d_a={d_a} n_sub={n_sub} k={k} {dtype}")
     g = torch.Generator().manual_seed(seed)
     t = dict(q=torch.randn(B, T, H * d_a, generator=g).to(dtype).float(),
              keys1=torch.randn(H, n_sub, d_a // 2, generator=g), keys2=torch.randn(H, n_sub, d_a // 2, generator=g),
              log_scale=math.log(8.0) + 0.3 * torch.randn(H, generator=g),
              values=torch.randn(H, n_sub * n_sub, dh, generator=g))
+    if same:   # the first `same` tokens of every row ask alike: their picks fall on the same k rows
+        t["q"][:, :same] = t["q"][:1, :1]
     wgt = torch.randn(B, T, H * dh, generator=torch.Generator().manual_seed(seed + 7))
     dev = {n: v.to("cuda").to(dtype if n == "q" else torch.float32).requires_grad_(True) for n, v in t.items()}
     cfg = dict(k=k)
@@ -68,6 +70,13 @@ def test_table_grad_trained_sdm_layer_shape():
 def test_table_grad_at_the_sub_key_limit_of_the_tiles(n_sub):
     """64 sub-keys per half on addr_grad_tile_kernel, 65 on addr_grad_kernel."""
     check_table("limit", 5, 3, 45, 1, 16, 32, n_sub, 16)
+
+
+@pytest.mark.parametrize("T,same,dh", [(1, 0, 4), (32, 32, 8), (65, 33, 260), (97, 97, 1028), (301, 290, 20)])
+def test_table_grad_rows_cut_over_pieces_of_the_sorted_picks(T, same, dh):
+    """Rows of no pick, of one piece's edge (32 picks), of a few and of many pieces; columns past one step of 256 and
+    past the 1,024 that a wave holds."""
+    check_table("pieces", 6, 2, T, 2, dh, 8, 8, 8, same=same)
 
 
 def _trained64(P, pre, x, si, H, d_a):
