@@ -96,7 +96,8 @@ int sdm_rt_prepare_key_pieces(const sdm_rt_dims* dims, const sdm_rt_params* para
 /* Bytes of workspace sdm_rt_forward needs for these dimensions (0 on invalid dims): the chunk plans (33 KB per
  * 64 positions of one head at k <= 8) and their sizes, the scan's progress counters and status word and, with
  * out_norm and more than one column group per head, the out-norm's partial sums (512 bytes per 64 positions of a
- * head and group). */
+ * head and group); for a few long sequences also the states that segments of them start from (at most 34 MB; a call
+ * given less runs them in one piece). */
 size_t sdm_rt_workspace_bytes(const sdm_rt_dims* dims);
 
 /* With the write gate, sdm_rt_forward (and sdm_rt_forward_noalloc, in its scratch) leaves in its workspace a copy
@@ -150,8 +151,8 @@ int sdm_rt_forward(const sdm_rt_dims* dims, const sdm_rt_params* params,
 /* sdm_rt_forward without a workspace argument: the same kernels run on a scratch array that the library holds on
  * each device it runs on (a fixed sdm_rt_noalloc_scratch_bytes() = 128 MiB, kept until the process ends), so the
  * call allocates no device memory.  It has no counterpart in the reference; it is for callers that cannot allocate
- * (code under HIP graph capture, tight serving loops).  A call whose workspace (sdm_rt_workspace_bytes) exceeds the
- * scratch returns SDM_RT_ENOSPACE without launching anything.  All calls on one device share its scratch: calls that
+ * (code under HIP graph capture, tight serving loops).  A call whose workspace (sdm_rt_workspace_bytes, less the states of
+ * segments) exceeds the scratch returns SDM_RT_ENOSPACE without launching anything.  All calls on one device share its scratch: calls that
  * overlap on one device (on different streams, or from different threads) race and must be serialised by the
  * caller.  Arguments as sdm_rt_forward. */
 size_t sdm_rt_noalloc_scratch_bytes(void);

@@ -43,8 +43,22 @@ static int state_copy(float* dst, const float* src, int64_t n, hipStream_t st) {
   return check_launch("state copy");
 }
 
+// whether the final state is written over the initial one
+static bool state_overlaps(const Plan& p, const CoreIO& io) {
+  if (!io.state_in_mem || !io.state_out_mem) return false;
+  const size_t n_cnt = sizeof(float) * static_cast<size_t>(p.B) * p.H * p.M;
+  auto range = [](const float* a, size_t na, const float* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
+  };
+  return range(io.state_in_mem, n_cnt * p.dh, io.state_out_mem, n_cnt * p.dh) ||
+         range(io.state_in_mem, n_cnt * p.dh, io.state_out_cnt, n_cnt) ||
+         range(io.state_in_cnt, n_cnt, io.state_out_mem, n_cnt * p.dh) ||
+         range(io.state_in_cnt, n_cnt, io.state_out_cnt, n_cnt);
+}
+
 int run_core(const Plan& p, const sdm_rt_dims* dims, const sdm_rt_params* prm, const CoreIO& io, void* workspace,
-             hipStream_t st) {
+             size_t workspace_bytes, hipStream_t st) {
   char* ws = static_cast<char*>(workspace);
   int32_t* sizes = reinterpret_cast<int32_t*>(ws + p.off_sizes);
   unsigned char* plans = reinterpret_cast<unsigned char*>(ws + p.off_plans);
@@ -120,9 +134,21 @@ int run_core(const Plan& p, const sdm_rt_dims* dims, const sdm_rt_params* prm, c
   s.read_mean = dims->read_mean;
   s.read_eps = dims->read_eps;
   s.out_eps = dims->out_norm_eps;
-  if (pick)
+  if (pick) {
+    s.segs = 1;
+    s.seg_chunks = p.n_chunks;
+    const PickSegments sg = pick_segments(p);
+    // not where the state goes back over the state it came from: the last segment may end before the first begins
+    if (sg.segs > 1 && workspace_bytes >= p.total + sg.bytes && !state_overlaps(p, io)) {
+      s.segs = sg.segs;
+      s.seg_chunks = sg.seg_chunks;
+      s.seg_mem = reinterpret_cast<float*>(ws + p.total);
+      s.seg_cnt = reinterpret_cast<float*>(ws + p.total + sg.off_cnt);
+      s.seg_fade = reinterpret_cast<float*>(ws + p.total + sg.off_fade);
+    }
     return io.in_dtype == SDM_RT_BF16 ? launch_pick_scan_bf16(p, s, io.out_dtype, st)
                                       : launch_pick_scan_f32(p, s, io.out_dtype, st);
+  }
   return io.in_dtype == SDM_RT_BF16 ? launch_scan_bf16(p, s, io.out_dtype, st) : launch_scan_f32(p, s, io.out_dtype, st);
 }
 
@@ -135,7 +161,7 @@ extern "C" {
 size_t sdm_rt_workspace_bytes(const sdm_rt_dims* dims) {
   Plan p;
   if (make_plan(dims, &p) != SDM_RT_OK) return 0;
-  return p.total;
+  return p.total + (pick_path(p) ? pick_segments(p).bytes : 0);   // a call with p.total alone runs unsegmented
 }
 
 size_t sdm_rt_gate_copy_offset(const sdm_rt_dims* dims) {
@@ -241,7 +267,7 @@ int sdm_rt_forward(const sdm_rt_dims* dims, const sdm_rt_params* params, const v
   io.state_in_cnt = state_in_cnt;
   io.state_out_mem = state_out_mem;
   io.state_out_cnt = state_out_cnt;
-  return run_core(p, dims, params, io, workspace, st);
+  return run_core(p, dims, params, io, workspace, workspace_bytes, st);
 }
 
 }  // extern "C"

@@ -1753,7 +1753,7 @@ __global__ void __launch_bounds__(256) pick_keys_kernel(const int32_t* __restric
 // begun before piece s, [2 s + 1] begins a row that goes on after it.  table_values_join_kernel adds a row's pieces in
 // order and clears the rows without a pick.  The load follows the picks and not the rows: text repeats its tokens, so a
 // few rows hold hundreds of picks, and with one wave per row the longest row's chain of batches was the kernel's time
-// (B=4, T=1024, 4,096 rows of 768, k=16, a Zipf stream: 190 us; now 49 us and the join's 6; the
+// (B=4, T=1024, 4,096 rows of 768, k=16, a Zipf stream: 190 us; now 49 us and 10 for the join; the
 // floor is the 101 MB of dy rows gathered through the caches).  Pieces of 32: the partial sums then take at most a
 // quarter of the gathered bytes again, and 2,048 waves are all resident at three to a SIMD.
 constexpr int kValuesSeg = 32;
@@ -2169,7 +2169,7 @@ int sdm_rt_forward_train(const sdm_rt_dims* dims, const sdm_rt_params* params, c
   io.saved = saved;   // the plan kernel's picks, weights (gate included) and scores
   io.read_out = saved->read;
   io.den_out = dims->read_mean ? saved->den : nullptr;
-  return run_core(p, dims, params, io, workspace, st);
+  return run_core(p, dims, params, io, workspace, workspace_bytes, st);
 }
 
 size_t sdm_rt_backward_workspace_bytes(const sdm_rt_dims* dims) {

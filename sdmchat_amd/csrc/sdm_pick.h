@@ -28,6 +28,8 @@
 namespace sdmrt {
 
 constexpr int kPickCols = 32;        // value columns per workgroup
+// measured costs of pick_segments' rule, in ns: a chunk of the scan, a chunk of the write sums, the rest of a segment
+constexpr int kPickChunkNs = 3100, kSumChunkNs = 2400, kSegmentNs = 25600;
 
 // LDS of one pick scan workgroup: the slab A[M + 1][32] and counts cnt[M + 1], by chunk parity two buffers of the
 // chunk's value rows [64][32] (float32, whatever the value type) and of its staged variable part, the fade powers
@@ -41,6 +43,40 @@ __host__ __device__ constexpr size_t pick_lds_bytes(int M, int n_chunks) {
 // the pick scan serves this shape (values of vb bytes)
 inline bool pick_path(const Plan& p) {
   return use_mf(p) && p.pitch == 8 && p.dh % kPickCols == 0 && p.M <= 1024 && pick_lds_bytes(p.M, p.n_chunks) <= kLdsBytes;
+}
+
+// Segments of the sequence that the pick scan runs side by side.  The scan is serial over a slab's chunks and has one
+// workgroup per slab and column group, so a few slabs leave most of the 256 compute units idle.  The state is linear in
+// its start, so pick_sum_kernel first sums every segment's writes from an empty slab (the chunk step without reads,
+// about 2.4 us a chunk against 3.1 us), pick_join_kernel carries the sums over the segments, and the scan runs all
+// segments at once, each from its own state.  Taken where this is the shorter: the chunks of a segment at both rates
+// and 25.6 us for the two launches, the states' way through memory and the slabs' loads, against the whole sequence at
+// the scan's rate.  Measured with 12 slabs of two groups, scan alone and in segments, whole layer in bfloat16: T=704
+// 90 and 90 us, 1,024 107 and 91, 2,048 168 and 111, 8,192 497 and 200 (scan 399; sums 37, join 10, scan 55); 36 slabs,
+// T=2,048 206 and 189.
+struct PickSegments {
+  int segs, seg_chunks;
+  size_t off_cnt, off_fade, bytes;   // of the workspace behind Plan::total
+};
+
+inline PickSegments pick_segments(const Plan& p) {
+  PickSegments r{1, p.n_chunks, 0, 0, 0};
+  const int64_t slabs = static_cast<int64_t>(p.B) * p.H;
+  const int groups = p.dh / kPickCols;
+  if (slabs < 1 || groups < 1 || p.n_chunks < 2) return r;
+  // workgroups are laid out in eighths (one XCD each) of slabs and segments; all resident, one to a compute unit
+  const int64_t most = 256 / groups / 8 * 8 / slabs;
+  if (most < 2) return r;
+  const int k = static_cast<int>(most < p.n_chunks ? most : p.n_chunks);
+  const int seg_chunks = (p.n_chunks + k - 1) / k;
+  if (kSumChunkNs * seg_chunks + kPickChunkNs * seg_chunks + kSegmentNs >= kPickChunkNs * p.n_chunks) return r;
+  r.seg_chunks = seg_chunks;
+  r.segs = (p.n_chunks + seg_chunks - 1) / seg_chunks;
+  const size_t n_cnt = static_cast<size_t>(r.segs - 1) * slabs * p.M;
+  r.off_cnt = align_up(sizeof(float) * n_cnt * p.dh, 256);
+  r.off_fade = r.off_cnt + align_up(sizeof(float) * n_cnt, 256);
+  r.bytes = r.off_fade + align_up(sizeof(float) * (r.segs - 1) * slabs, 256);
+  return r;
 }
 
 template <int CTRL>
@@ -66,7 +102,242 @@ constexpr int kPickThreads = 512;    // 64 positions x 8 picks
 constexpr int kTeamWriters = 32;     // a wave with a slot of this many later writers in a chunk writes in teams
 constexpr int kPrefetchContribs = 40;  // a wave with a position of more contributions loads their entries together
 
-template <typename VT, typename OutT>
+// eight 4-column pieces of a position's value row in the lane's read order, from the piece f that each of the
+// position's eight lanes holds (lane x holds piece x): pieces j ^ 1, j ^ 2, j ^ 3 by quad permutes, j ^ 7 by the half-row
+// mirror, and j ^ 6, j ^ 5, j ^ 4 by the mirror of the first three
+__device__ __forceinline__ void spread_pieces(const float4& f, float (&vp)[32]) {
+  const float x[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float t1 = dppf<0xb1>(x[e]), t2 = dppf<0x4e>(x[e]), t3 = dppf<0x1b>(x[e]);
+    vp[e] = x[e];
+    vp[4 + e] = t1;
+    vp[8 + e] = t2;
+    vp[12 + e] = t3;
+    vp[16 + e] = dppf<0x141>(x[e]);
+    vp[20 + e] = dppf<0x141>(t1);
+    vp[24 + e] = dppf<0x141>(t2);
+    vp[28 + e] = dppf<0x141>(t3);
+  }
+}
+
+// The writes of one segment (not the last) of a slab's 32-column group, summed from an empty slab: pick_scan_kernel's
+// plain chunk step without its reads, so a chunk needs one barrier and its lanes only their own rows.  Leaves the
+// segment's state contribution in seg_mem / seg_cnt and its fade in seg_fade.  Bound by the chunk's chain of dependent
+// LDS accesses, the longest list of a slot's later writers in it: 37 us for 13 chunks with the slab's clear and store
+// (loads two chunks ahead instead of one: the same).
+template <typename VT>
+__global__ void __launch_bounds__(kPickThreads) pick_sum_kernel(ScanArgs a) {
+  constexpr int CW = kPickCols;
+  constexpr int VS = kVarStage;
+  constexpr int NT = kPickThreads;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int M = a.M;
+  const int G = a.groups;
+  const int jr = (static_cast<int>(blockIdx.x) >> 3) / G;
+  const int g = (static_cast<int>(blockIdx.x) >> 3) - jr * G;
+  const int vs = 8 * jr + (blockIdx.x & 7);
+  const int seg = vs / a.S;
+  if (seg >= a.segs - 1) return;
+  const int s = vs - seg * a.S;
+  const int b_row = s / a.H;
+  const int h = s - b_row * a.H;
+  const int c_begin = seg * a.seg_chunks;
+  const int c_end = c_begin + a.seg_chunks;   // whole chunks: the last segment is another's
+  float* A = lds;                                                          // the scan's LDS (pick_lds_bytes)
+  float* cnt = A + static_cast<size_t>(M + 1) * CW;
+  float* s_v = cnt + pad4(M + 1);
+  unsigned char* var = reinterpret_cast<unsigned char*>(s_v + 2 * kChunk * CW);
+  float* pw = reinterpret_cast<float*>(var + 2 * VS);
+  int32_t* s_sizes = reinterpret_cast<int32_t*>(pw + 68);
+  const int tid = threadIdx.x;
+  const int p = tid >> 3;
+  const int j = tid & 7;
+  const int col0 = g * CW;
+  const int fcol = 4 * j;
+  int soff[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) soff[k] = 16 * (j ^ (k < 4 ? k : 11 - k));
+  const float lam = a.decay[h];
+  const unsigned char* plans_s = a.plans + static_cast<int64_t>(s) * a.n_chunks * PickGeom::stride();
+  const VT* v_b = static_cast<const VT*>(a.v) + static_cast<int64_t>(b_row) * a.T * a.v_stride +
+                  static_cast<int64_t>(h) * a.dh + col0;
+  for (int i = tid; i < (M + 1) * CW / 4; i += NT) reinterpret_cast<float4*>(A)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int m = tid; m <= M; m += NT) cnt[m] = 0.f;
+  for (int i = tid; i < a.seg_chunks; i += NT) s_sizes[i] = a.sizes[static_cast<int64_t>(s) * a.n_chunks + c_begin + i];
+  float lam_chunk = lam;   // lam^64
+#pragma unroll
+  for (int bit = 0; bit < 6; ++bit) lam_chunk *= lam_chunk;
+
+  auto load_w = [&](int c) {
+    return *reinterpret_cast<const uint3*>(plans_s + static_cast<uint32_t>(c) * static_cast<uint32_t>(PickGeom::stride()) +
+                                           PickGeom::kRec * (j * kChunk + p) + PickGeom::off_w());
+  };
+  auto load_v = [&](int c) {   // row p, columns 4 j ... 4 j + 3 of the group, as float32
+    const VT* src = v_b + static_cast<uint32_t>(c * kChunk + p) * static_cast<uint32_t>(a.v_stride) + fcol;
+    float f[4];
+    load_vals<4, VT>(src, f);
+    return make_float4(f[0], f[1], f[2], f[3]);
+  };
+  auto load_var = [&](int c, int bytes) {
+    const unsigned char* src = plans_s + static_cast<uint32_t>(c) * static_cast<uint32_t>(PickGeom::stride()) +
+                               PickGeom::off_var() + 8 * tid;
+    return 8 * tid < min(bytes, VS) ? *reinterpret_cast<const uint2*>(src) : make_uint2(0u, 0u);
+  };
+  auto stage = [&](int buf, const float4& vv, const uint2& vr) {
+    *reinterpret_cast<float4*>(s_v + buf * kChunk * CW + p * CW + fcol) = vv;
+    reinterpret_cast<uint2*>(var + buf * VS)[tid] = vr;
+  };
+  uint3 wr = load_w(c_begin);
+  float4 v_cur = load_v(c_begin);
+  stage(0, v_cur, load_var(c_begin, a.sizes[static_cast<int64_t>(s) * a.n_chunks + c_begin]));
+  float mu = 1.f, fade = 1.f;
+  bool emptied = false;
+  lds_barrier();
+  unsigned char* A_b = reinterpret_cast<unsigned char*>(A);
+  for (int c = c_begin; c < c_end; ++c) {
+    const int buf = (c - c_begin) & 1;
+    const int cn = min(c + 1, c_end - 1);
+    const uint3 wr_n = load_w(cn);
+    const float4 v_n = load_v(cn);
+    const uint2 var_n = load_var(cn, s_sizes[cn - c_begin]);
+    const unsigned char* varc = var + buf * VS;
+    const float* s_vc = s_v + buf * kChunk * CW;
+    const unsigned char* gvar =
+        plans_s + static_cast<uint32_t>(c) * static_cast<uint32_t>(PickGeom::stride()) + PickGeom::off_var();
+    auto add_vrow = [&](float cf, int v, float (&acc)[32]) {
+      const float* vrow = s_vc + v * CW;
+      VPiece<float> vq[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) vq[k].load(vrow + soff[k] / 4);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) vq[k].fma4(cf, acc + 4 * k);
+    };
+    // fade the slab (folded into mu; rescaled when mu gets small); a chunk with a reset empties it
+    const bool chunk_reset = reinterpret_cast<const uint32_t*>(varc)[1] & 0x80000000u;
+    mu *= lam_chunk;
+    fade *= lam_chunk;
+    if (chunk_reset) {
+      emptied = true;
+      float4* a4 = reinterpret_cast<float4*>(A);
+      for (int i = tid; i < (M + 1) * CW / 4; i += NT) a4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int i = tid; i <= M; i += NT) cnt[i] = 0.f;
+      mu = 1.f;
+      lds_barrier();
+    } else if (!(mu >= kMuFloor)) {
+      float4* a4 = reinterpret_cast<float4*>(A);
+      for (int i = tid; i < (M + 1) * CW / 4; i += NT) {
+        const float4 t = a4[i];
+        a4[i] = make_float4(t.x * mu, t.y * mu, t.z * mu, t.w * mu);
+      }
+      for (int i = tid; i <= M; i += NT) cnt[i] *= mu;
+      mu = 1.f;
+      lds_barrier();
+    }
+    // every owner adds its own faded value and those of the slot's later writers to the slot's row
+    const int wslot = static_cast<int>(wr.x & 0x7ffu);
+    float vp[32];
+    spread_pieces(v_cur, vp);
+    if (wslot != M) {
+      const float inv_mu = fast_rcp(mu);
+      unsigned char* row = A_b + wslot * (CW * 4);
+      float y[32];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float4 q4 = *reinterpret_cast<const float4*>(row + soff[k]);
+        y[4 * k] = q4.x;
+        y[4 * k + 1] = q4.y;
+        y[4 * k + 2] = q4.z;
+        y[4 * k + 3] = q4.w;
+      }
+      float cw = cnt[wslot];
+      const float a0 = __uint_as_float(wr.y) * inv_mu;
+#pragma unroll
+      for (int k = 0; k < 32; ++k) y[k] = fmaf(a0, vp[k], y[k]);
+      cw += a0;
+      const int n_l = static_cast<int>((wr.x >> 17) & 63u);
+      if (n_l > 0) {
+        const float a1 = __uint_as_float(wr.z) * inv_mu;
+        add_vrow(a1, static_cast<int>((wr.x >> 11) & 63u), y);
+        cw += a1;
+        const int w_e0 = static_cast<int>(wr.x >> 23);
+        for (int e = 0; e < n_l - 1; ++e) {
+          const int o = PickGeom::off_ent() + 8 * min(w_e0 + e, PickGeom::max_entries() - 1);
+          const uint2 en = o + 8 <= VS ? *reinterpret_cast<const uint2*>(varc + o) : *reinterpret_cast<const uint2*>(gvar + o);
+          const float ae = __uint_as_float(en.x) * inv_mu;
+          add_vrow(ae, static_cast<int>(en.y & 63u), y);
+          cw += ae;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        *reinterpret_cast<float4*>(row + soff[k]) = make_float4(y[4 * k], y[4 * k + 1], y[4 * k + 2], y[4 * k + 3]);
+      cnt[wslot] = cw;
+    }
+    wr = wr_n;
+    v_cur = v_n;
+    stage(buf ^ 1, v_n, var_n);   // the buffer held the chunk before, done before the last barrier
+    lds_barrier();
+  }
+  const int64_t vrow = (static_cast<int64_t>(seg) * a.S + s) * M;
+  for (int i = tid; i < M * (CW / 4); i += NT) {
+    const int m = i / (CW / 4), q = i - m * (CW / 4);
+    const float4 t = reinterpret_cast<const float4*>(A)[i];
+    *reinterpret_cast<float4*>(a.seg_mem + (vrow + m) * a.dh + col0 + 4 * q) =
+        make_float4(mu * t.x, mu * t.y, mu * t.z, mu * t.w);
+  }
+  if (g == 0) {
+    for (int m = tid; m < M; m += NT) a.seg_cnt[vrow + m] = mu * cnt[m];
+    if (tid == 0) a.seg_fade[static_cast<int64_t>(seg) * a.S + s] = emptied ? -1.f : fade;
+  }
+}
+
+// The segments' sums, carried: in place, the state after segment q = its sum + fade_q * the state it began with.  One
+// thread per four values of a slab (of dh columns, or of its counts); four segments' loads in flight.
+static __global__ void __launch_bounds__(256) pick_join_kernel(ScanArgs a) {
+  const int64_t per = static_cast<int64_t>(a.M) * (a.dh / 4);   // float4s of a slab's rows, then M counts
+  const int64_t n_mem = a.S * per;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int q_end = a.segs - 1;
+  auto carry = [&](auto* base, const float* in, int64_t at, int64_t step, int s) {
+    using V = typename std::remove_pointer<decltype(base)>::type;
+    constexpr int N = sizeof(V) / sizeof(float);
+    float x[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) x[e] = in ? in[at * N + e] : 0.f;
+    for (int q0 = 0; q0 < q_end; q0 += 4) {
+      V v[4];
+      float f[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = min(q0 + u, q_end - 1);
+        v[u] = base[q * step + at];
+        f[u] = a.seg_fade[static_cast<int64_t>(q) * a.S + s];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (q0 + u < q_end) {
+          float* e = reinterpret_cast<float*>(&v[u]);
+#pragma unroll
+          for (int k = 0; k < N; ++k) {
+            x[k] = f[u] < 0.f ? e[k] : fmaf(f[u], x[k], e[k]);
+            e[k] = x[k];
+          }
+          base[(q0 + u) * step + at] = v[u];
+        }
+      }
+    }
+  };
+  if (i < n_mem) {
+    carry(reinterpret_cast<float4*>(a.seg_mem), a.state_in_mem, i, n_mem, static_cast<int>(i / per));
+  } else if (i - n_mem < static_cast<int64_t>(a.S) * a.M) {
+    const int64_t m = i - n_mem;
+    carry(a.seg_cnt, a.state_in_cnt, m, static_cast<int64_t>(a.S) * a.M, static_cast<int>(m / a.M));
+  }
+}
+
+// SEGS: several segments (a kernel of its own: the segment's bounds as variables cost a long grid of slabs 1.5%)
+template <typename VT, typename OutT, bool SEGS>
 __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
   constexpr int CW = kPickCols;
   constexpr int VS = kVarStage;
@@ -78,8 +349,12 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
   const int xcd = bid & 7;
   const int jr = (bid >> 3) / G;
   const int g = (bid >> 3) - jr * G;
-  const int s = 8 * jr + xcd;
-  if (s >= a.S) return;
+  const int vs = 8 * jr + xcd;   // segment and slab
+  const int seg = SEGS ? vs / a.S : 0;
+  if (SEGS ? seg >= a.segs : vs >= a.S) return;
+  const int s = vs - seg * a.S;
+  const int c_begin = SEGS ? seg * a.seg_chunks : 0;
+  const int c_end = SEGS ? min(c_begin + a.seg_chunks, a.n_chunks) : a.n_chunks;
   const int b_row = s / a.H;
   const int h = s - b_row * a.H;
   float* A = lds;                                                          // [M + 1][32]
@@ -105,13 +380,23 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
   const VT* v_b = static_cast<const VT*>(a.v) + static_cast<int64_t>(b_row) * a.T * a.v_stride +
                   static_cast<int64_t>(h) * a.dh + col0;
 
-  for (int i = tid; i < (M + 1) * CW; i += NT) {
-    const int m = i / CW;
-    const int cc = i - m * CW;
-    A[i] = (a.state_in_mem && m < M) ? a.state_in_mem[(static_cast<int64_t>(s) * M + m) * a.dh + col0 + cc] : 0.f;
+  const int64_t seg_row = (static_cast<int64_t>(seg - 1) * a.S + s) * M;   // segments past the first: the carried state
+  if (SEGS && seg > 0) {
+    for (int i = tid; i < (M + 1) * (CW / 4); i += NT) {
+      const int m = i / (CW / 4), q = i - m * (CW / 4);
+      reinterpret_cast<float4*>(A)[i] = m < M ? *reinterpret_cast<const float4*>(a.seg_mem + (seg_row + m) * a.dh + col0 + 4 * q)
+                                              : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    for (int m = tid; m <= M; m += NT) cnt[m] = m < M ? a.seg_cnt[seg_row + m] : 0.f;
+  } else {
+    for (int i = tid; i < (M + 1) * CW; i += NT) {
+      const int m = i / CW;
+      const int cc = i - m * CW;
+      A[i] = (a.state_in_mem && m < M) ? a.state_in_mem[(static_cast<int64_t>(s) * M + m) * a.dh + col0 + cc] : 0.f;
+    }
+    for (int m = tid; m <= M; m += NT)
+      cnt[m] = (a.state_in_cnt && m < M) ? a.state_in_cnt[static_cast<int64_t>(s) * M + m] : 0.f;
   }
-  for (int m = tid; m <= M; m += NT)
-    cnt[m] = (a.state_in_cnt && m < M) ? a.state_in_cnt[static_cast<int64_t>(s) * M + m] : 0.f;
   for (int i = tid; i < a.n_chunks; i += NT) s_sizes[i] = a.sizes[static_cast<int64_t>(s) * a.n_chunks + i];
   if (tid <= kChunk) {
     float v = 1.f, sq = lam;   // lam^tid by squaring (as the plan computes it; exact for lam = 0 and lam = 1)
@@ -243,9 +528,9 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
       return make_float4(__uint_as_float(vv.x), __uint_as_float(vv.y), __uint_as_float(vv.z), __uint_as_float(vv.w));
   };
   uint3 rr, wr;
-  load_recs(0, rr, wr);
-  VQuad v_cur = load_v(0);
-  stage(0, v_cur, load_var(0, a.sizes[static_cast<int64_t>(s) * a.n_chunks]));
+  load_recs(c_begin, rr, wr);
+  VQuad v_cur = load_v(c_begin);
+  stage(c_begin, v_cur, load_var(c_begin, a.sizes[static_cast<int64_t>(s) * a.n_chunks + c_begin]));
   lds_barrier();
   const float lam_chunk = pw[kChunk];
   const float inv_dh = 1.f / static_cast<float>(a.dh);
@@ -262,11 +547,11 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
   crowded = __ballot(crowded) != 0ull;
   auto chunk_loop = [&](auto early_t) {
     constexpr bool EARLY = decltype(early_t)::value;
-    for (int c = 0; c < a.n_chunks; ++c) {
-      const bool fin2 = xnorm && c >= 2;
+    for (int c = c_begin; c < c_end; ++c) {
+      const bool fin2 = xnorm && c >= c_begin + 2;
       // the next chunk's records, values and variable part are loaded into registers during this chunk (the last
       // chunk loads its own again)
-      const int cn = min(c + 1, a.n_chunks - 1);
+      const int cn = min(c + 1, c_end - 1);
       uint3 rr_n, wr_n;
       load_recs(cn, rr_n, wr_n);
       const VQuad v_n = load_v(cn);
@@ -357,26 +642,8 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
         }
         cw_old = cnt[wslot];
       }
-      // the eight pieces of value row p in the lane's read order, from the pieces the position's eight lanes staged
-      // (lane x holds piece x): pieces j ^ 1, j ^ 2, j ^ 3 by quad permutes, j ^ 7 by the half-row mirror, and
-      // j ^ 6, j ^ 5, j ^ 4 by the mirror of the first three
-      float vp[32];
-      {
-        const float4 f = as_f4(v_cur);
-        const float x[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float t1 = dppf<0xb1>(x[e]), t2 = dppf<0x4e>(x[e]), t3 = dppf<0x1b>(x[e]);
-          vp[e] = x[e];
-          vp[4 + e] = t1;
-          vp[8 + e] = t2;
-          vp[12 + e] = t3;
-          vp[16 + e] = dppf<0x141>(x[e]);
-          vp[20 + e] = dppf<0x141>(t1);
-          vp[24 + e] = dppf<0x141>(t2);
-          vp[28 + e] = dppf<0x141>(t3);
-        }
-      }
+      float vp[32];   // value row p in the lane's read order
+      spread_pieces(as_f4(v_cur), vp);
       // reduce-scatter over the eight pick lanes of the position: 32 -> 16 -> 8 -> 4 columns
 #pragma unroll
       for (int k = 0; k < 16; ++k) acc[k] += dppf<0x141>(acc[16 + k]);   // row_half_mirror: lane 7 - j
@@ -728,11 +995,12 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
   if (crowded) chunk_loop(std::true_type{});
   else chunk_loop(std::false_type{});
   if (xnorm) {   // the last two chunks (or one)
-    const int n = a.n_chunks;
-    if (n >= 2) finish(n - 2, rq[1], sq[1], G == 2 ? xget(n - 2, 1 - g) : 0ull);
+    const int n = c_end;
+    if (n - c_begin >= 2) finish(n - 2, rq[1], sq[1], G == 2 ? xget(n - 2, 1 - g) : 0ull);
     finish(n - 1, rq[0], sq[0], G == 2 ? xget(n - 1, 1 - g) : 0ull);
   }
 
+  if (SEGS && seg < a.segs - 1) return;
   if (a.state_out_mem) {
     for (int i = tid; i < M * CW; i += NT) {
       const int m = i / CW;
@@ -748,14 +1016,35 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
 template <typename VT, typename OutT>
 int launch_pick_scan_t(const Plan& p, const ScanArgs& a, hipStream_t st) {
   const size_t lds = pick_lds_bytes(p.M, p.n_chunks);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pick_scan_kernel<VT, OutT>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     static_cast<int>(kLdsBytes));
+  const bool segs = a.segs > 1;
+  static const hipError_t attr1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&pick_scan_kernel<VT, OutT, false>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                      static_cast<int>(kLdsBytes));
+  static const hipError_t attr2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&pick_scan_kernel<VT, OutT, true>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                      static_cast<int>(kLdsBytes));
+  const hipError_t attr = segs ? attr2 : attr1;
   if (attr != hipSuccess) return set_err(SDM_RT_ELAUNCH, "pick scan: cannot enable %zu bytes of LDS", kLdsBytes);
   if (a.groups * kPickCols != p.dh || a.sync_stride < a.groups || !pick_path(p))
     return set_err(SDM_RT_EINVAL, "pick scan: %d groups for head_dim %d", a.groups, p.dh);
-  const int slabs8 = (p.B * p.H + 7) / 8 * 8;
-  hipLaunchKernelGGL((pick_scan_kernel<VT, OutT>), dim3(slabs8 * a.groups), dim3(kPickThreads), lds, st, a);
+  if (segs) {
+    static const hipError_t sum_attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pick_sum_kernel<VT>),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                           static_cast<int>(kLdsBytes));
+    if (sum_attr != hipSuccess) return set_err(SDM_RT_ELAUNCH, "pick sums: cannot enable %zu bytes of LDS", kLdsBytes);
+    const int sums8 = (a.S * (a.segs - 1) + 7) / 8 * 8;
+    hipLaunchKernelGGL((pick_sum_kernel<VT>), dim3(sums8 * a.groups), dim3(kPickThreads), lds, st, a);
+    if (const int rc = check_launch("pick sums")) return rc;
+    const int64_t n = static_cast<int64_t>(a.S) * a.M * (a.dh / 4 + 1);
+    hipLaunchKernelGGL(pick_join_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, a);
+    if (const int rc = check_launch("pick join")) return rc;
+  }
+  const int slabs8 = (a.S * a.segs + 7) / 8 * 8;
+  if (segs) {
+    hipLaunchKernelGGL((pick_scan_kernel<VT, OutT, true>), dim3(slabs8 * a.groups), dim3(kPickThreads), lds, st, a);
+  } else {
+    hipLaunchKernelGGL((pick_scan_kernel<VT, OutT, false>), dim3(slabs8 * a.groups), dim3(kPickThreads), lds, st, a);
+  }
   return check_launch("pick scan");
 }
 

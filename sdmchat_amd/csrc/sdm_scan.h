@@ -43,6 +43,11 @@ struct ScanArgs {
   float read_eps, out_eps;
   uint32_t spin_limit;         // polls of a partner's progress before a wait gives up (0: give up at once)
   int crowded_bytes;           // pick scan: a chunk plan's variable part past this makes its slab crowded
+  // pick scan over several segments of the sequence at once (pick_segments): segment q takes chunks q seg_chunks ...
+  int segs, seg_chunks;
+  float* seg_mem;              // [segs - 1][S][M][dh]: the state that segments 1, 2, ... begin with
+  float* seg_cnt;              // [segs - 1][S][M]
+  float* seg_fade;             // [segs - 1][S]: the fade over a segment, or -1 when a reset in it empties the slab
 };
 
 constexpr uint32_t kSpinLimit = 1u << 20;   // the default polls of a partner's progress before a wait gives up

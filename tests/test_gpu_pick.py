@@ -10,10 +10,13 @@ state carry, the final state, resets, crowded chunks whose plans overflow what t
 value rows, three column groups sharing the out-norm, and the read modes.  Tolerances as there: float32 1e-5,
 bfloat16 2e-3 plus half a bfloat16 ulp.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from sdmchat_amd import core
 from tests._gpu_util import assert_close, bf16_round, check_core, core_inputs, gpu_address, gpu_core, say
 
 pytestmark = pytest.mark.gpu
@@ -111,7 +114,6 @@ def test_crowded_chunks_read_past_the_staged_plan():
     parts run past the 4 KB the scan stages in LDS and the rest is read from the plan in global memory.  The
     workspace shows that pick plans were written (their headers, at the pick plan's offset, hold the sizes) and
     that they overflowed."""
-    from sdmchat_amd import core
     B, T, H = 2, 200, 4
     kz, qz, V, g, p = core_inputs(B, T, H, 32, 16, 8, seed=191, addr_bias=4.0)
     check_core(kz, qz, V, g, p, 8)
@@ -189,7 +191,6 @@ def test_bench_shape_crowded_bf16():
     contributions past the eight a record keeps and slots with many later writers; variable parts past the 4 KB the
     scan stages, read from the plan), bf16: every pick against the oracle and every slab's read-out against the fp64
     recurrence on the kernel's picks."""
-    from sdmchat_amd import core
     kz, qz, V, g, p = core_inputs(8, 2048, 12, 64, 64, 32, seed=171, addr_bias=4.0)
     kz, qz, V, g = (bf16_round(a) for a in (kz, qz, V, g))
     flips = check_core(kz, qz, V, g, p, 8, dtype=torch.bfloat16, tol=2e-3, rescaled=True)
@@ -256,7 +257,6 @@ def test_crowded_slabs_early_write_sums_give_the_same_bits(dtype):
     token (crowded) beside rows of varied tokens, with resets and a fade that rescales the slab every chunk: the
     read-out and the final state with the default threshold, with every slab on the plain step and with every slab
     on the early step are equal bit for bit."""
-    from sdmchat_amd import core
     B, T, H, dh, n_sub = 4, 300, 4, 64, 16
     kz, qz, V, g, p = core_inputs(B, T, H, dh, 32, n_sub, seed=307, decays=(0.0, 0.3, 0.97, 1.0))
     for arr in (kz, qz, g):   # rows 0 and 2: one repeated token
@@ -338,3 +338,67 @@ def test_a_wait_that_gives_up_is_reported(k, what):
     torch.cuda.synchronize()
     assert bool(torch.isfinite(r).all())
     assert_close(r.cpu().numpy(), gpu_core(kz, qz, V, g, p, k), 0.0, msg=f"{what}: clean call after the error path")
+
+
+@pytest.mark.parametrize("B,T,H,dh,dtype,decays,resets", [
+    (1, 897, 2, 64, torch.float32, (0.97, 1.0), ()),               # one position past 14 chunks: a short last segment
+    (1, 1024, 1, 128, torch.float32, (0.0,), ()),                  # four column groups; a fade of 0
+    (2, 1500, 1, 32, torch.float32, (0.3,), (0, 700, 701, 1499)),  # one column group; rescaled slabs and resets
+    (1, 2600, 3, 64, torch.bfloat16, (0.9, 0.999, 1.0), (64, 1300)),
+])
+def test_segments_side_by_side_match_the_sequence_in_pieces(B, T, H, dh, dtype, decays, resets):
+    """A few long sequences run in segments (pick_sum_kernel, pick_join_kernel, then the scan of every segment from its
+    own state); pieces of 128 positions, each from the state of the one before, do not.  Both from a state that is not
+    empty.  The sums are the same ones in float32 in another order: a state of up to T terms of size one, each rounded
+    at 2^-24 of a sum that the fades and the mean read keep of order one, so 2e-5; the read-outs in float32."""
+    kz, qz, V, g, p = core_inputs(B, T, H, dh, 64, 32, seed=61 + T, decays=decays, addr_bias=0.3)
+    if dtype == torch.bfloat16:
+        kz, qz, V, g = (bf16_round(a) for a in (kz, qz, V, g))
+    lib = core._lib.load()
+    nbytes = [core.workspace_bytes(core.make_dims(B, 64 * c, H, dh, 64, 32, 8)) for c in (2, 3, (T + 63) // 64)]
+    chunk = nbytes[1] - nbytes[0]
+    assert nbytes[2] > nbytes[1] + chunk * ((T + 63) // 64 - 3) + 4 * 1024 * dh * B * H   # room for segments' states
+    rng = np.random.Generator(np.random.PCG64(T))
+    cnt = rng.random((B, H, 1024)).astype(np.float32)
+    state = (cnt[..., None] * rng.standard_normal((B, H, 1024, dh)).astype(np.float32), cnt)
+    reset = np.zeros((B, T), bool)
+    reset[0, list(resets)] = True
+    kw = dict(dtype=dtype, out_dtype=torch.float32, want_state=True)
+    say(f"[segments] B={B} T={T} H={H} dh={dh} {dtype}")
+    r, (mem, c) = gpu_core(kz, qz, V, g, p, 8, state_in=state, reset=reset, **kw)
+    want, st = [], state
+    for t0 in range(0, T, 128):
+        sl = slice(t0, min(t0 + 128, T))
+        rr, st = gpu_core(kz[:, sl], qz[:, sl], V[:, sl], g[:, sl], p, 8, state_in=st, reset=reset[:, sl], **kw)
+        want.append(rr)
+    np.testing.assert_allclose(r, np.concatenate(want, 1), atol=2e-5, rtol=2e-5)
+    np.testing.assert_allclose(mem, st[0], atol=2e-5, rtol=2e-5)
+    np.testing.assert_allclose(c, st[1], atol=2e-5, rtol=2e-5)
+
+
+def test_segments_state_written_over_its_input():
+    """A state written back over the one it came from takes the unsegmented scan: the last segment could end before the
+    first has read."""
+    kz, qz, V, g, p = core_inputs(1, 1024, 2, 32, 64, 32, seed=62)
+    tp = {n: torch.from_numpy(v).cuda() for n, v in p.items()}
+    t = [torch.from_numpy(a).cuda() for a in (kz, qz, V, g)]
+    mem, cnt = torch.randn(1, 2, 1024, 32).cuda(), torch.rand(1, 2, 1024).cuda()
+    kw = dict(keys1=tp["keys1"], keys2=tp["keys2"], log_scale=tp["log_scale"], decay=tp["decay"],
+              addr_b=tp["addr_b"], onorm_w=tp["onorm_w"], gate_bias=tp["gate_bias"], k=8)
+    say("[segments] in place")
+    r, (m1, c1) = core.core_forward(*t, state_in=(mem, cnt), want_state=True, **kw)
+    prm, held = core._params(mem.device, tp["keys1"], tp["keys2"], tp["addr_b"], tp["log_scale"], tp["decay"],
+                             tp["onorm_w"], tp["gate_bias"])
+    dims = core.make_dims(1, 1024, 2, 32, 64, 32, 8)
+    lib = core._lib.load()
+    ws = torch.empty(core.workspace_bytes(dims), dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(r)
+    rc = lib.sdm_rt_forward(ctypes.byref(dims), ctypes.byref(prm), core._ptr(t[0]), 128, core._ptr(t[1]), 128,
+                            core._ptr(t[2]), 64, core._ptr(t[3]), 2, 0, None, core._ptr(out), 64, 0, core._ptr(mem),
+                            core._ptr(cnt), core._ptr(mem), core._ptr(cnt), core._ptr(ws), ws.numel(),
+                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    core._lib.check(rc, lib)
+    torch.cuda.synchronize()
+    for a, b in ((out, r), (mem, m1), (cnt, c1)):
+        torch.testing.assert_close(a, b, atol=2e-5, rtol=2e-5)
+    del held
