@@ -43,6 +43,7 @@ struct ScanArgs {
   float read_eps, out_eps;
   uint32_t spin_limit;         // polls of a partner's progress before a wait gives up (0: give up at once)
   int crowded_bytes;           // pick scan: a chunk plan's variable part past this makes its slab crowded
+  int var_stage;               // scan_kernel: bytes of a plan's variable part staged in LDS (scan_var_stage)
   // pick scan over several segments of the sequence at once (pick_segments): segment q takes chunks q seg_chunks ...
   int segs, seg_chunks;
   float* seg_mem;              // [segs - 1][S][M][dh]: the state that segments 1, 2, ... begin with
@@ -170,7 +171,7 @@ template <int CW, int KP, typename VT, typename OutT>
 __global__ void __launch_bounds__(kScanThreads) scan_kernel(ScanArgs a) {
   constexpr int CPL = CW / 8;
   constexpr PlanGeom pg{KP};
-  constexpr int VS = kVarStage;
+  const int VS = a.var_stage;
   constexpr int NR = pg.pos_bytes() / 16;                   // 16-byte words of a position record
   constexpr int REC_PIECES = kChunk * pg.pos_bytes() / 16;  // a multiple of 64 (64 (KP + 3))
   constexpr int V_ROW = CW * static_cast<int>(sizeof(VT));  // bytes of a position's values in the group
@@ -243,8 +244,8 @@ __global__ void __launch_bounds__(kScanThreads) scan_kernel(ScanArgs a) {
     for (int blk = wave; blk * 64 < REC_PIECES; blk += kScanThreads / 64)
       copy_to_lds(base + 16 * (blk * 64 + lane), recs + 1024 * blk);
     const int pieces = min((bytes + 15) >> 4, VS / 16);
-    for (int blk = wave; blk * 64 < VS / 16; blk += kScanThreads / 64)
-      copy_to_lds(base + pg.off_var() + 16 * min(blk * 64 + lane, max(pieces - 1, 0)),
+    for (int blk = wave; blk * 64 < pieces; blk += kScanThreads / 64)
+      copy_to_lds(base + pg.off_var() + 16 * min(blk * 64 + lane, pieces - 1),
                   var + (c & 1) * VS + 1024 * blk);
     if (a.v_direct) {
       for (int blk = wave; blk * 64 < V_PIECES; blk += kScanThreads / 64) {
@@ -398,11 +399,22 @@ __global__ void __launch_bounds__(kScanThreads) scan_kernel(ScanArgs a) {
     }
     if (n_in > kInline) {   // contributions past the inline ones (rare: the branch diverges between positions)
       auto over = [&](auto st) {
-        for (int e = 0; e < n_in - kInline; ++e) {
-          const uint2 t = ent_at(ro + e, st);
-          const Seg<CPL> vq = lds_seg<CPL>(&s_vc[(t.y & 63u) * CW + cl]);
+        // four entries at a time, their loads together: one after another each costs two LDS round trips
+        const int n = n_in - kInline;
+        for (int e = 0; e < n; e += 4) {
+          uint2 t[4];
+          Seg<CPL> vq[4];
 #pragma unroll
-          for (int k = 0; k < CPL; ++k) acc[k] = fmaf(__uint_as_float(t.x), vq.v[k], acc[k]);
+          for (int u = 0; u < 4; ++u) t[u] = ent_at(ro + min(e + u, n - 1), st);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) vq[u] = lds_seg<CPL>(&s_vc[(t[u].y & 63u) * CW + cl]);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (e + u < n) {
+#pragma unroll
+              for (int k = 0; k < CPL; ++k) acc[k] = fmaf(__uint_as_float(t[u].x), vq[u].v[k], acc[k]);
+            }
+          }
         }
       };
       if (all_staged) over(std::true_type{});
@@ -524,17 +536,24 @@ __global__ void __launch_bounds__(kScanThreads) scan_kernel(ScanArgs a) {
           const float cold = *crow;
           const int e0 = static_cast<int>(xr.y & 0xffffu), n = min(static_cast<int>(xr.y >> 16), kChunk);
           float csum_w = 0.f;
-          for (int e = 0; e < n; e += 2) {   // two writers at a time (the second one's weight is 0 past n)
-            const uint2 e_0 = ent_at(e0 + e, st);
-            const uint2 e_1 = ent_at(e0 + min(e + 1, n - 1), st);
-            const float c_0 = __uint_as_float(e_0.x) * inv_mu;
-            const float c_1 = e + 1 < n ? __uint_as_float(e_1.x) * inv_mu : 0.f;
-            float v0[8], v1[8];
-            lds_vals8(&s_vc[(e_0.y & 63u) * CW + 8 * l_s], v0);
-            lds_vals8(&s_vc[(e_1.y & 63u) * CW + 8 * l_s], v1);
+          for (int e = 0; e < n; e += 4) {   // four writers at a time
+            uint2 en[4];
+            float v[4][8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) z[k] = fmaf(c_1, v1[k], fmaf(c_0, v0[k], z[k]));
-            csum_w += c_0 + c_1;
+            for (int u = 0; u < 4; ++u) en[u] = ent_at(e0 + min(e + u, n - 1), st);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) lds_vals8(&s_vc[(en[u].y & 63u) * CW + 8 * l_s], v[u]);
+            float ce[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              ce[u] = e + u < n ? __uint_as_float(en[u].x) * inv_mu : 0.f;
+              if (e + u < n) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) z[k] = fmaf(ce[u], v[u][k], z[k]);
+              }
+            }
+            csum_w += ce[0] + ce[1];
+            csum_w += ce[2] + ce[3];
           }
           lds_row8_store(row, z);
           if (l_s == 0) *crow = cold + csum_w;
@@ -571,6 +590,17 @@ __global__ void __launch_bounds__(kScanThreads) scan_kernel(ScanArgs a) {
   }
 }
 
+// Bytes of a chunk's variable plan part that the scan stages in LDS (two buffers; kVarStage of them are in lds): as
+// much of the largest part as the LDS takes without fewer workgroups on a compute unit (at most two fit its registers).
+// Entries past it are read from memory, a round trip each.  With it and the entries taken four at a time, 16 picks over
+// packed documents (60 slabs of 13 chunks, 4 groups): 108 -> 103 us.
+inline int scan_var_stage(size_t lds, int KP) {
+  const size_t budget = lds <= kLdsBytes / 2 ? kLdsBytes / 2 : kLdsBytes;
+  const size_t most = (16 + 8 * static_cast<size_t>(PlanGeom{KP}.max_entries()) + 1023) / 1024 * 1024;
+  const size_t room = kVarStage + (budget - lds) / 2 / 1024 * 1024;
+  return static_cast<int>(most < room ? most : room);
+}
+
 template <int CW, int KP, typename VT, typename OutT>
 int launch_scan_t(const Plan& p, const ScanArgs& a, hipStream_t st) {
   const size_t lds = scan_lds_bytes(p.M, CW, p.n_chunks, KP, static_cast<int>(sizeof(VT)));
@@ -581,7 +611,10 @@ int launch_scan_t(const Plan& p, const ScanArgs& a, hipStream_t st) {
   if (a.groups * CW != p.dh || a.sync_stride < a.groups)
     return set_err(SDM_RT_EINVAL, "scan: %d groups of %d columns for head_dim %d", a.groups, CW, p.dh);
   const int slabs8 = (p.B * p.H + 7) / 8 * 8;
-  hipLaunchKernelGGL((scan_kernel<CW, KP, VT, OutT>), dim3(slabs8 * a.groups), dim3(kScanThreads), lds, st, a);
+  ScanArgs args = a;
+  args.var_stage = scan_var_stage(lds, KP);
+  hipLaunchKernelGGL((scan_kernel<CW, KP, VT, OutT>), dim3(slabs8 * a.groups), dim3(kScanThreads),
+                     lds + 2 * static_cast<size_t>(args.var_stage - kVarStage), st, args);
   return check_launch("scan");
 }
 

@@ -189,3 +189,10 @@ def test_crowded_chunks_read_past_the_staged_plan():
     sizes = ws.buf[:4 * n_plans].cpu().view(torch.int32)   # the workspace starts with the plans' variable-part sizes
     say(f"variable-part bytes per plan: max {int(sizes.max())}, mean {float(sizes.float().mean()):.0f}")
     assert int(sizes.max()) > 4096
+
+
+@pytest.mark.parametrize("n_sub,H,dh", [(32, 2, 16), (60, 1, 8)])
+def test_crowded_plans_of_sixteen_picks(n_sub, H, dh):
+    """Plans whose variable part is past 4 KB: 1,024 locations leave LDS for the largest one, 3,600 for 5 KB, past which
+    the scan reads the plan from memory."""
+    check_core(*core_inputs(1, 150, H, dh, 32, n_sub, seed=93, addr_bias=4.0), 16)
