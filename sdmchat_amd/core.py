@@ -23,7 +23,32 @@ def make_dims(B, T, heads, head_dim, addr_dim, n_sub, k, read_mode="mean", out_n
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def _stream(device):
+    """The raw handle of the current stream of a tensor's device (without the Stream object, whose construction takes
+    about 2 us: a decode step of one layer asks four times)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _NoAutocast:
+    """torch.autocast("cuda", enabled=False), entered only where autocast is on (entering and leaving it takes about
+    5 us of a call's host time)."""
+
+    __slots__ = ("ctx",)
+
+    def __enter__(self):
+        self.ctx = torch.autocast("cuda", enabled=False) if torch.is_autocast_enabled("cuda") else None
+        if self.ctx is not None:
+            self.ctx.__enter__()
+
+    def __exit__(self, *exc):
+        if self.ctx is not None:
+            self.ctx.__exit__(*exc)
+
+
+no_autocast = _NoAutocast
 
 
 def _rows16(t2):
@@ -36,6 +61,13 @@ def _f32(t, device):
     if t is None:
         return None
     return t.detach().to(device=device, dtype=torch.float32).contiguous()
+
+
+def _bytes(reset, device):
+    """A reset mask as the contiguous bytes the kernels read: a boolean mask's own, else a copy."""
+    if reset.dtype == torch.bool and reset.device == device and reset.is_contiguous():
+        return reset.view(torch.uint8)
+    return reset.to(device=device, dtype=torch.uint8).contiguous()
 
 
 def _rows(x, name, B, T, width):
@@ -77,9 +109,9 @@ def _params(device, keys1, keys2, addr_b, log_scale, decay, onorm_w, gate_bias, 
     nbytes = lib.sdm_rt_key_pieces_bytes(ctypes.byref(dims)) if pieces else 0
     if nbytes:
         pieces = torch.empty(nbytes, dtype=torch.uint8, device=held[0].device)
-        stream = torch.cuda.current_stream(pieces.device).cuda_stream
+        stream = _stream(pieces.device)
         _lib.check(lib.sdm_rt_prepare_key_pieces(ctypes.byref(dims), ctypes.byref(prm), _ptr(pieces), nbytes,
-                                                 ctypes.c_void_p(stream)), lib)
+                                                 stream), lib)
         prm.key_pieces = _ptr(pieces)
         prm.key_pieces_bytes = nbytes
         held.append(pieces)
@@ -137,9 +169,9 @@ def address(z, keys1, keys2, k, log_scale, addr_b=None, gate_logits=None, gate_b
     slots = torch.empty(B, H, T, pitch, dtype=torch.int32, device=dev)
     scores = torch.empty(B, H, T, pitch, dtype=torch.float32, device=dev)
     weights = torch.empty(B, H, T, pitch, dtype=torch.float32, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_address(ctypes.byref(dims), ctypes.byref(prm), _ptr(z), zs, _ptr(gate_logits), gs, _DT[z.dtype],
-                            _ptr(slots), _ptr(scores), _ptr(weights), None, 0, ctypes.c_void_p(stream))
+                            _ptr(slots), _ptr(scores), _ptr(weights), None, 0, stream)
     _lib.check(rc, lib)
     del held
     if padded:   # the kernel's own [B, H, T, pitch] arrays (pads: slot -1, weight 0)
@@ -155,7 +187,7 @@ def gate_copy(workspace, B, T, H, dh, d_a, n_sub, k, dtype, read_mode="mean", ou
     lib = _lib.load()
     dims = make_dims(B, T, H, dh, d_a, n_sub, k, read_mode, out_norm, True, read_eps, out_norm_eps)
     off = lib.sdm_rt_gate_copy_offset(ctypes.byref(dims))
-    n = B * T * H * torch.empty(0, dtype=dtype).element_size()
+    n = B * T * H * dtype.itemsize
     buf = workspace.buf
     if off == 0 or buf is None or buf.numel() < off + n:
         raise RuntimeError("gate_copy: the workspace holds no gate copy for these dimensions")
@@ -224,23 +256,23 @@ def core_forward(kz, qz, v, gate_logits, *, keys1, keys2, log_scale, decay, addr
     if reset is not None:
         if tuple(reset.shape) != (B, T):
             raise ValueError(f"reset must be [B={B}, T={T}]")
-        rs = reset.to(device=dev, dtype=torch.uint8).contiguous()
-    stream = torch.cuda.current_stream(dev).cuda_stream
+        rs = _bytes(reset, dev)
+    stream = _stream(dev)
     if no_alloc:
         rc = lib.sdm_rt_forward_noalloc(ctypes.byref(dims), ctypes.byref(prm), _ptr(kz), ks, _ptr(qz), qs, _ptr(v),
                                         vs, _ptr(gate_logits), gs, _DT[dt], _ptr(rs), _ptr(out), ostride,
                                         _DT[out_dtype], _ptr(mem_in), _ptr(cnt_in), _ptr(mem_out), _ptr(cnt_out),
-                                        ctypes.c_void_p(stream))
+                                        stream)
     else:
         nbytes = lib.sdm_rt_workspace_bytes(ctypes.byref(dims))  # 0 for invalid dims: the call below reports why
         ws = (workspace or CoreWorkspace()).get(nbytes, dev)
         rc = lib.sdm_rt_forward(ctypes.byref(dims), ctypes.byref(prm), _ptr(kz), ks, _ptr(qz), qs, _ptr(v), vs,
                                 _ptr(gate_logits), gs, _DT[dt], _ptr(rs), _ptr(out), ostride, _DT[out_dtype],
                                 _ptr(mem_in), _ptr(cnt_in), _ptr(mem_out), _ptr(cnt_out), _ptr(ws), ws.numel(),
-                                ctypes.c_void_p(stream))
+                                stream)
     _lib.check(rc, lib)
     if check:
-        rc = lib.sdm_rt_status(ctypes.byref(dims), None if no_alloc else _ptr(ws), ctypes.c_void_p(stream))
+        rc = lib.sdm_rt_status(ctypes.byref(dims), None if no_alloc else _ptr(ws), stream)
         _lib.check(rc, lib)
     if want_state:
         return out, (mem_out, cnt_out)
@@ -293,9 +325,9 @@ def table_read(slots, weights, values, k, out_dtype=torch.float32, out=None):
     if out is None:
         out = torch.empty(B, T, H * dh, dtype=out_dtype, device=dev)
     ostride = _rows(out, "out", B, T, H * dh)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_table_read(ctypes.byref(dims), _ptr(sl), _ptr(wt), _ptr(vals), _DT[vals.dtype], _ptr(out), ostride,
-                               _DT[out.dtype], ctypes.c_void_p(stream))
+                               _DT[out.dtype], stream)
     _lib.check(rc, lib)
     return out
 
@@ -343,10 +375,10 @@ def table_step(hx, wq, keys1, keys2, log_scale, values, k, params=None, want_q=F
     weights = torch.empty(B, H, T, pitch, dtype=torch.float32, device=dev)
     out = torch.empty(B, T, H * dh, dtype=torch.bfloat16, device=dev)
     q = torch.empty(B, T, H * d_a, dtype=torch.bfloat16, device=dev) if want_q else None
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_table_step(ctypes.byref(dims), ctypes.byref(prm), _ptr(x2), x2.stride(0), d, _ptr(wq), wq.stride(0),
                                _ptr(vals), _ptr(q), H * d_a, _ptr(slots), _ptr(scores), _ptr(weights), _ptr(out),
-                               H * dh, ctypes.c_void_p(stream))
+                               H * dh, stream)
     _lib.check(rc, lib)
     del held
     return out, slots, scores, weights, q
@@ -392,11 +424,11 @@ def table_step_residual(x, y, norm_w, eps, wq, keys1, keys2, log_scale, values, 
     out = torch.empty(B, T, H * dh, dtype=torch.bfloat16, device=dev)
     q = torch.empty(B, T, H * d_a, dtype=torch.bfloat16, device=dev) if want_q else None
     hx = torch.empty(B, T, d, dtype=torch.bfloat16, device=dev) if want_hx else None
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_table_step_residual(ctypes.byref(dims), ctypes.byref(prm), _ptr(x), d, _ptr(y), d, _ptr(wf),
                                         float(eps), _ptr(s), d, _ptr(hx), d, d, _ptr(wq), wq.stride(0), _ptr(vals),
                                         _ptr(q), H * d_a, _ptr(slots), _ptr(scores), _ptr(weights), _ptr(out), H * dh,
-                                        ctypes.c_void_p(stream))
+                                        stream)
     _lib.check(rc, lib)
     del held
     return s, out, slots, scores, weights, q, hx
@@ -490,18 +522,18 @@ def decode_step(kz, qz, v, gate_logits, state, *, keys1, keys2, log_scale, decay
     if reset is not None:
         if tuple(reset.shape) != (B,):
             raise ValueError(f"reset must be [B={B}]")
-        rs = reset.to(device=dev, dtype=torch.uint8).contiguous()
+        rs = _bytes(reset, dev)
     out_dtype = out_dtype or dt
     if out is None:
         out = torch.empty(B, H * dh, dtype=out_dtype, device=dev)
     ostride = _rows2(out, "out", B, H * dh)
     nbytes = lib.sdm_rt_decode_workspace_bytes(ctypes.byref(dims))
     ws = (workspace or CoreWorkspace()).get(nbytes, dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_decode_step(ctypes.byref(dims), ctypes.byref(prm), _ptr(kz), ks, _ptr(qz), qs, _ptr(v), vs,
                                 _ptr(gate_logits), gs, _DT[dt], _ptr(rs), _ptr(state.mem), _ptr(state.cnt),
                                 _ptr(state.scale), _ptr(state.last), _ptr(out), ostride, _DT[out_dtype], _ptr(ws), ws.numel(),
-                                ctypes.c_void_p(stream))
+                                stream)
     _lib.check(rc, lib)
     return out
 
@@ -539,10 +571,10 @@ def rms_norm(x, w, eps=1e-6, out_dtype=None, out=None):
     o2 = out.view(-1, d)
     wf = _f32_weight(w, x.device)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _stream(x.device)
     rc = lib.sdm_rt_rms_norm(_ptr(x2), x2.stride(0) if x2.numel() else d, _DT[x.dtype], x2.shape[0], d, _ptr(wf),
                              float(eps), _ptr(o2), o2.stride(0) if o2.numel() else d, _DT[out_dtype],
-                             ctypes.c_void_p(stream))
+                             stream)
     _lib.check(rc, lib)
     return out
 
@@ -599,10 +631,10 @@ def rms_norm_backward(x, w, dy, eps, need_x=True, need_w=True):
     lib = _lib.load()
     nbytes = lib.sdm_rt_rms_norm_backward_workspace_bytes(rows, d) if need_w else 0
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _stream(x.device)
     _lib.check(lib.sdm_rt_rms_norm_backward(_ptr(x2), x2.stride(0), _DT[x.dtype], _ptr(dy2), dy2.stride(0),
                                             _DT[dy.dtype], rows, d, _ptr(wf), float(eps), _ptr(dx), d, _ptr(dw),
-                                            _ptr(ws), nbytes, ctypes.c_void_p(stream)), lib)
+                                            _ptr(ws), nbytes, stream), lib)
     return dx, None if dw is None else dw.to(w.dtype)
 
 
@@ -624,9 +656,9 @@ def weight_grad(dy, x):
     out = torch.empty(n, k, dtype=torch.float32, device=dy.device)
     nbytes = lib.sdm_rt_weight_grad_workspace_bytes(rows, n, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dy.device) if nbytes else None
-    stream = torch.cuda.current_stream(dy.device).cuda_stream
+    stream = _stream(dy.device)
     _lib.check(lib.sdm_rt_weight_grad(_ptr(dy), dy.stride(0), _ptr(x), x.stride(0), rows, n, k, _ptr(out), _ptr(ws),
-                                      nbytes, ctypes.c_void_p(stream)), lib)
+                                      nbytes, stream), lib)
     return out
 
 
@@ -637,7 +669,7 @@ class LinearFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, out_dtype):
-        with torch.autocast("cuda", enabled=False):
+        with no_autocast():
             x16, w16 = x.to(torch.bfloat16), w.to(torch.bfloat16)
             ctx.save_for_backward(x16, w16)
             ctx.dtypes = (x.dtype, w.dtype)
@@ -647,7 +679,7 @@ class LinearFunction(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, dy):
         x16, w16 = ctx.saved_tensors
-        with torch.autocast("cuda", enabled=False):
+        with no_autocast():
             dy16 = dy.to(torch.bfloat16)
             dx = torch.matmul(dy16, w16).to(ctx.dtypes[0]) if ctx.needs_input_grad[0] else None
             dw = None
@@ -691,9 +723,9 @@ def add_rms_norm(x, y, w, eps=1e-6, out_dtype=None, inplace=True):
     wf = _f32_weight(w, x.device)
     lib = _lib.load()
     rows = x.numel() // d
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _stream(x.device)
     rc = lib.sdm_rt_add_rms_norm(_ptr(x), d, _ptr(y), d, _DT[x.dtype], rows, d, _ptr(wf), float(eps), _ptr(s), d,
-                                 _ptr(out), d, _DT[out_dtype], ctypes.c_void_p(stream))
+                                 _ptr(out), d, _DT[out_dtype], stream)
     _lib.check(rc, lib)
     return s, out
 
@@ -708,9 +740,9 @@ def silu_mul(gate_up):
         g2 = g2.contiguous()
     out = torch.empty(gate_up.shape[:-1] + (f2 // 2,), dtype=gate_up.dtype, device=gate_up.device)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(gate_up.device).cuda_stream
+    stream = _stream(gate_up.device)
     rc = lib.sdm_rt_silu_mul(_ptr(g2), g2.stride(0), _DT[gate_up.dtype], g2.shape[0], f2 // 2, _ptr(out), f2 // 2,
-                             ctypes.c_void_p(stream))
+                             stream)
     _lib.check(rc, lib)
     return out
 
@@ -743,9 +775,9 @@ def linear(x, w, bias=None, as_matmul=False):
         bias = bias.contiguous()
     y = torch.empty(x.shape[:-1] + (n,), dtype=torch.bfloat16, device=x.device)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _stream(x.device)
     rc = lib.sdm_rt_gemm_rows(_ptr(x2), x2.stride(0), _ptr(w), w.stride(0), _ptr(bias), _ptr(y), n, rows, n, k,
-                              ctypes.c_void_p(stream))
+                              stream)
     _lib.check(rc, lib)
     return y
 
@@ -784,9 +816,9 @@ def linear_residual(x, y, norm_w, eps, w, bias=None):
     out = torch.empty(x.shape[:-1] + (n,), dtype=torch.bfloat16, device=x.device)
     wf = _f32_weight(norm_w, x.device)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _stream(x.device)
     rc = lib.sdm_rt_gemm_rows_residual(_ptr(x), k, _ptr(y), k, _ptr(wf), float(eps), _ptr(s), k, _ptr(w), w.stride(0),
-                                       _ptr(bias), _ptr(out), n, rows, n, k, ctypes.c_void_p(stream))
+                                       _ptr(bias), _ptr(out), n, rows, n, k, stream)
     _lib.check(rc, lib)
     return s, out
 
@@ -824,10 +856,10 @@ def linear_embed(idx, table, norm_w, eps, w, bias=None):
     out = torch.empty(rows, n, dtype=torch.bfloat16, device=idx.device)
     wf = _f32_weight(norm_w, idx.device)
     lib = _lib.load()
-    stream = torch.cuda.current_stream(idx.device).cuda_stream
+    stream = _stream(idx.device)
     rc = lib.sdm_rt_gemm_rows_embed(_ptr(idx), _ptr(table), table.stride(0), table.shape[0], _ptr(wf), float(eps),
                                     _ptr(x), k, _ptr(w), w.stride(0), _ptr(bias), _ptr(out), n, rows, n, k,
-                                    ctypes.c_void_p(stream))
+                                    stream)
     _lib.check(rc, lib)
     return x, out
 
@@ -886,10 +918,10 @@ def core_forward_train(kz, qz, v, gate_logits, *, params, k, read_mode="mean", o
     saved["reset"] = rs
     nbytes = lib.sdm_rt_workspace_bytes(ctypes.byref(dims))
     ws = (workspace or CoreWorkspace()).get(nbytes, dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_forward_train(ctypes.byref(dims), ctypes.byref(params[0]), _ptr(kz), ks, _ptr(qz), qs, _ptr(v),
                                   vs, _ptr(gate_logits), gs, _DT[dt], _ptr(rs), _ptr(out), H * dh, _DT[out_dtype],
-                                  ctypes.byref(sv), _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
+                                  ctypes.byref(sv), _ptr(ws), ws.numel(), stream)
     _lib.check(rc, lib)
     return out, saved
 
@@ -941,11 +973,11 @@ def core_backward(kz, qz, v, gate_logits, saved, dy, *, params, k, read_mode="me
     sv = _lib.SdmRtSaved(*[_ptr(saved[n]) for n in _SAVED])
     nbytes = lib.sdm_rt_backward_workspace_bytes(ctypes.byref(dims))
     ws = (workspace or CoreWorkspace()).get(nbytes, dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_backward_typed(ctypes.byref(dims), ctypes.byref(params[0]), _ptr(kz), ks, _ptr(qz), qs, _ptr(v),
                                    vs, _ptr(gate_logits), gs, _DT[v.dtype], _ptr(saved["reset"]), ctypes.byref(sv),
                                    _ptr(dy), dys, _DT[dy.dtype], ctypes.byref(gr), _DT[gdt], _ptr(ws), ws.numel(),
-                                   ctypes.c_void_p(stream))
+                                   stream)
     _lib.check(rc, lib)
     return g
 
@@ -1004,8 +1036,7 @@ _SAVED = ("slots_w", "weights_w", "scores_w", "slots_r", "weights_r", "scores_r"
 def _decay_grad(decay, log_decay):
     """d loss / d decay from lam * d loss / d lam (0 at lam = 0)."""
     lam = decay.detach().to(torch.float32)
-    return torch.where(lam > 0, log_decay / torch.where(lam > 0, lam, torch.ones_like(lam)),
-                       torch.zeros_like(lam)).to(decay.dtype)
+    return torch.where(lam > 0, log_decay / lam, 0.0).to(decay.dtype)
 
 
 def mixer_train_fits(x, weights):
@@ -1042,16 +1073,16 @@ class MixerFunction(torch.autograd.Function):
         B, T, d = x.shape
         H, za = keys1.shape[0], wk.shape[0]
         gated = wg is not None
-        with torch.autocast("cuda", enabled=False):
+        with no_autocast():
             hx = rms_norm(x, norm_w, cfg["eps"], out_dtype=dt)
             W = torch.empty(ra + d, d, dtype=dt, device=x.device)
             bias = torch.empty(ra + d, dtype=dt, device=x.device) if gated else None
             ws = [None if w is None else _aligned(w.detach()) for w in (wk, wq, wg, wv)]
             bgc = None if bg is None else bg.detach().to(ws[0].dtype).contiguous()
             lib = _lib.load()
-            stream = torch.cuda.current_stream(x.device).cuda_stream
+            stream = _stream(x.device)
             _lib.check(lib.sdm_rt_pack_projection(*[_ptr(w) for w in ws], _ptr(bgc), _DT[ws[0].dtype], za, H, ra, d,
-                                                  _ptr(W), _ptr(bias), _DT[dt], ctypes.c_void_p(stream)), lib)
+                                                  _ptr(W), _ptr(bias), _DT[dt], stream), lib)
             pa = torch.nn.functional.linear(hx, W[:ra], None if bias is None else bias[:ra])
             V = torch.nn.functional.linear(hx, W[ra:])
             g = pa[..., 2 * za:2 * za + H] if gated else None
@@ -1076,7 +1107,7 @@ class MixerFunction(torch.autograd.Function):
         B, T, d = x.shape
         H = keys1.shape[0]
         need = ctx.needs_input_grad
-        with torch.autocast("cuda", enabled=False):
+        with no_autocast():
             params = _params(x.device, keys1, keys2, addr_b, log_scale, decay, onorm_w, None, pieces=False)
             dp = torch.empty(B, T, ra + d, dtype=pa.dtype, device=x.device)
             g = pa[..., 2 * za:2 * za + H] if gated else None
@@ -1131,12 +1162,12 @@ def table_backward(q, slots, weights, scores, values, dy, *, k, params, workspac
              log_scale=torch.empty(H, **f32))
     nbytes = lib.sdm_rt_table_backward_workspace_bytes(ctypes.byref(dims))
     ws = (workspace or CoreWorkspace()).get(nbytes, dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     rc = lib.sdm_rt_table_backward(ctypes.byref(dims), ctypes.byref(params[0]), _ptr(q), qs, _DT[q.dtype],
                                    _ptr(slots), _ptr(weights), _ptr(scores), _ptr(vals), _DT[vals.dtype], _ptr(dy),
                                    dys, _DT[dy.dtype], _ptr(g["q"]), H * d_a, _ptr(g["values"]), _ptr(g["keys1"]),
                                    _ptr(g["keys2"]), _ptr(g["log_scale"]), _ptr(ws), ws.numel(),
-                                   ctypes.c_void_p(stream))
+                                   stream)
     _lib.check(rc, lib)
     return g
 

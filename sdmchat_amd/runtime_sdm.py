@@ -162,17 +162,17 @@ class RunTimeSdm(nn.Module):
             return torch.float32
         raise ValueError(f"unsupported input dtype {x.dtype}")
 
-    def _project(self, x, dt, hx=None):
+    def _project(self, x, dt, hx=None, fused=None):
         """RMSNorm then the projections wk, wq, wv, wg (prepare, track4_onesdm_models.py:197-206): one GEMM for
         [wk; wq; wg] and one for wv (one GEMM of the whole buffer for a few rows).  Returns views kz, qz
         [B, T, H * d_a] and gate logits [B, T, H] (None without the write gate) of the first map's output, and V
         [B, T, d].  The gate bias is the GEMM's bias, so W_g hx + b rounds to dt once, as wg(hx) does; addr_b is
         added inside the core.  hx: the normed input when the caller computed it (in dt, as the norm below gives
-        it)."""
+        it).  fused: _fused_weight(dt), when the caller has it."""
         H, d_a = self.h, self.d_a
         if hx is None:
             hx = core.rms_norm(x, self.norm.w, self.norm.eps, out_dtype=dt)   # the norm, then the cast to dt
-        W, bias = self._fused_weight(dt)[:2]
+        W, bias = (fused or self._fused_weight(dt))[:2]
         ra = self._rows_a()
         if hx.numel() // hx.shape[-1] <= core.GEMM_ROWS_MAX:
             proj = core.linear(hx, W, bias)                            # [B, T, ra + d]
@@ -252,11 +252,12 @@ class RunTimeSdm(nn.Module):
             return self._forward_train(x, reset)
         dt = self._compute_dtype(x)
         H = self.h
-        with torch.autocast("cuda", enabled=False):
-            kz, qz, V, g = self._project(x, dt, hx)
-            wo = self._fused_weight(dt)[2]
+        with core.no_autocast():
+            fused = self._fused_weight(dt)
+            kz, qz, V, g = self._project(x, dt, hx, fused)
+            wo = fused[2]
             res = core.core_forward(
-                kz, qz, V, g, keys1=self.keys1, keys2=self.keys2, log_scale=self.log_scale, decay=self.decay(),
+                kz, qz, V, g, keys1=self.keys1, keys2=self.keys2, log_scale=self.log_scale, decay=None,
                 addr_b=self.addr_b, onorm_w=self.onorm_w if self.out_norm else None,
                 gate_bias=None, k=self.k, read_mode=self.read_mode,
                 out_norm=self.out_norm, read_eps=self.read_eps, out_norm_eps=self.out_norm_eps, out_dtype=dt,
@@ -332,17 +333,19 @@ class RunTimeSdm(nn.Module):
             raise RuntimeError("RunTimeSdm.step is inference only: call it under torch.no_grad() or "
                                "torch.inference_mode()")
         dt = self._compute_dtype(x2)
-        with torch.autocast("cuda", enabled=False):
-            kz, qz, V, g = self._project(x2.unsqueeze(1), dt, None if hx is None else hx.reshape(x2.shape[0], 1, -1))
-            y = self._step_projected(kz, qz, V, g, state, reset, dt, x.dtype)
+        with core.no_autocast():
+            fused = self._fused_weight(dt)
+            kz, qz, V, g = self._project(x2.unsqueeze(1), dt, None if hx is None else hx.reshape(x2.shape[0], 1, -1),
+                                         fused)
+            y = self._step_projected(kz, qz, V, g, state, reset, dt, x.dtype, fused)
         return y.reshape(x.shape)
 
-    def _step_projected(self, kz, qz, V, g, state, reset, dt, out_dtype):
+    def _step_projected(self, kz, qz, V, g, state, reset, dt, out_dtype, fused):
         """The step after the projections (kz, qz, V, g: [B, 1, ...] views): the decode step, then wo."""
-        wo = self._fused_weight(dt)[2]
+        wo = fused[2]
         r = core.decode_step(
             kz[:, 0], qz[:, 0], V[:, 0], None if g is None else g[:, 0], state, keys1=self.keys1,
-            keys2=self.keys2, log_scale=self.log_scale, decay=self.decay(), addr_b=self.addr_b,
+            keys2=self.keys2, log_scale=self.log_scale, decay=None, addr_b=self.addr_b,
             onorm_w=self.onorm_w if self.out_norm else None, gate_bias=None,
             k=self.k, read_mode=self.read_mode, out_norm=self.out_norm, read_eps=self.read_eps,
             out_norm_eps=self.out_norm_eps, reset=reset, out_dtype=dt, workspace=self._ws,
@@ -378,14 +381,15 @@ class RunTimeSdm(nn.Module):
         B = x2.shape[0]
         H, d_a = self.h, self.d_a
         dt = torch.bfloat16
-        W, bias = self._fused_weight(dt)[:2]
+        fused = self._fused_weight(dt)
+        W, bias = fused[:2]
         ra = self._rows_a()
         s, proj = core.linear_residual(x2, y.reshape(-1, self.d), self.norm.w, self.norm.eps, W, bias)
         proj = proj.view(B, 1, -1)
         pa, V = proj[..., :ra], proj[..., ra:]
         o_q, o_g = H * d_a, 2 * H * d_a
         g = pa[..., o_g:o_g + H] if self.write_gate else None
-        out = self._step_projected(pa[..., :o_q], pa[..., o_q:o_g], V, g, state, reset, dt, x.dtype)
+        out = self._step_projected(pa[..., :o_q], pa[..., o_q:o_g], V, g, state, reset, dt, x.dtype, fused)
         return s.reshape(x.shape), out.reshape(x.shape)
 
     def embed_fits(self, idx, table):
@@ -408,14 +412,15 @@ class RunTimeSdm(nn.Module):
         B = idx.shape[0]
         H, d_a = self.h, self.d_a
         dt = torch.bfloat16
-        W, bias = self._fused_weight(dt)[:2]
+        fused = self._fused_weight(dt)
+        W, bias = fused[:2]
         ra = self._rows_a()
         x, proj = core.linear_embed(idx, table, self.norm.w, self.norm.eps, W, bias)
         proj = proj.view(B, 1, -1)
         pa, V = proj[..., :ra], proj[..., ra:]
         o_q, o_g = H * d_a, 2 * H * d_a
         g = pa[..., o_g:o_g + H] if self.write_gate else None
-        out = self._step_projected(pa[..., :o_q], pa[..., o_q:o_g], V, g, state, reset, dt, dt)
+        out = self._step_projected(pa[..., :o_q], pa[..., o_q:o_g], V, g, state, reset, dt, dt, fused)
         return x, out.reshape(B, self.d)
 
     def forward_sequential(self, x, reset=None):

@@ -87,7 +87,7 @@ class TrainedSdm(nn.Module):
         """x (B, T, d) -> soft weights (B*T, h, kk) and slot ids (B*T, h, kk), as the reference's address()."""
         self._check(x)
         B, T, _ = x.shape
-        with torch.autocast("cuda", enabled=False):
+        with core.no_autocast():
             si, _, w = self._picks(x, self._compute_dtype(x))
         kk = min(self.k, min(self.k, self.n_sub) ** 2)
         return (w[..., :kk].permute(0, 2, 1, 3).reshape(B * T, self.h, kk),
@@ -123,7 +123,7 @@ class TrainedSdm(nn.Module):
             return self._forward_train(x)
         B, T, _ = x.shape
         dt = self._compute_dtype(x)
-        with torch.autocast("cuda", enabled=False):
+        with core.no_autocast():
             if hx is None:
                 hx = core.rms_norm(x, self.norm.w, self.norm.eps, out_dtype=dt)
             wq, wo = self._weights(dt)
@@ -157,7 +157,7 @@ class TrainedSdm(nn.Module):
         shape = x.shape
         x3, y3 = x.reshape(-1, 1, shape[-1]) if x.dim() == 2 else x, y.reshape(-1, 1, shape[-1]) if y.dim() == 2 else y
         B, T, _ = x3.shape
-        with torch.autocast("cuda", enabled=False):
+        with core.no_autocast():
             wq, wo = self._weights(torch.bfloat16)
             prm = self._prm.get(x.device, self.keys1, self.keys2, None, self.log_scale, None, None, None)
             s, r, si, _, _, q, hx = core.table_step_residual(x3, y3, self.norm.w, self.norm.eps, wq, self.keys1,
