@@ -1060,7 +1060,7 @@ class MixerFunction(torch.autograd.Function):
     compute type, so the projections' input gradient and weight gradients are one product each, and the norm's backward
     takes the product as it is.  Op by op (slices of the maps' outputs, casts, two products each way, their sums) the
     same step moved every row about thirty times: a training step of the layer at B=8, T=2048 under bfloat16 autocast took
-    1.99 ms that way and takes 1.25 ms (84 launches, now 40).
+    1.99 ms that way; as one function 1.25 ms (84 launches, then 40), with the core backward of today 1.12 ms.
 
     apply(x, norm_w, wk, wq, wv, wg, bg, keys1, keys2, addr_b, log_scale, decay, onorm_w, cfg) -> r [B, T, H * dh] in
     the compute type.  wg and bg may be None (no write gate), onorm_w too.  cfg: dict with dtype (mixer_train_fits),
