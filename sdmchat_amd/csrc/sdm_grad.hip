@@ -1681,7 +1681,43 @@ __global__ void __launch_bounds__(64 * kRedGroups) grad_sums_kernel(GradSumsArgs
 //   d_values[h][s]       = sum over the picks (n, j) of slot s of w_j dy[n][h]   (table_values_grad_kernel: the picks
 //                          sorted by (head, slot) with a stable radix sort and summed in pieces in pick order -- no
 //                          float atomics, a fixed order)
-template <int KP, typename VT, typename DyT>
+// Four consecutive values of a row as they lie in memory: one load each, converted where they are used.  VEC: the rows
+// start on a multiple of four values (checked on the host).  load_vals checks each address instead, and a load behind a
+// branch of its own is waited for there, so a batch's loads run one after another (B=4, T=1024, rows of 768, k=16: values
+// gradient 49 -> 42 us, per-pick gradients 23.5 -> 19.6 us).
+template <typename T, bool VEC>
+struct Quad {
+  using Raw = typename std::conditional<sizeof(T) == 2, uint2, float4>::type;
+  Raw r;
+  __device__ __forceinline__ void load(const T* p) {
+    if constexpr (VEC) {
+      r = *reinterpret_cast<const Raw*>(p);
+    } else {
+      T* d = reinterpret_cast<T*>(&r);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = p[k];
+    }
+  }
+  __device__ __forceinline__ void get(float (&v)[4]) const {
+    if constexpr (sizeof(T) == 2) {
+      v[0] = __uint_as_float(r.x << 16);
+      v[1] = __uint_as_float(r.x & 0xffff0000u);
+      v[2] = __uint_as_float(r.y << 16);
+      v[3] = __uint_as_float(r.y & 0xffff0000u);
+    } else {
+      v[0] = r.x;
+      v[1] = r.y;
+      v[2] = r.z;
+      v[3] = r.w;
+    }
+  }
+};
+
+inline bool quad_rows(const void* p, int64_t stride, sdm_rt_dtype t) {
+  return reinterpret_cast<uintptr_t>(p) % (t == SDM_RT_BF16 ? 8 : 16) == 0 && stride % 4 == 0;
+}
+
+template <int KP, typename VT, typename DyT, bool VEC>
 __global__ void __launch_bounds__(256) table_grad_kernel(const int32_t* __restrict__ slots,
                                                          const float* __restrict__ wts,
                                                          const VT* __restrict__ values, const DyT* __restrict__ dy,
@@ -1705,13 +1741,18 @@ __global__ void __launch_bounds__(256) table_grad_kernel(const int32_t* __restri
   (void)wts;
   const VT* tab = values + static_cast<int64_t>(h) * M * dh;
   for (int c0 = 4 * lane; c0 < dh; c0 += 256) {
-    float g[4];
-    load_vals<4, DyT>(dy + n * dy_stride + static_cast<int64_t>(h) * dh + c0, g);
+    Quad<DyT, VEC> gq;
+    gq.load(dy + n * dy_stride + static_cast<int64_t>(h) * dh + c0);
     // every pick's row, pads included (their dots are dropped below): unconditional loads issue together
+    Quad<VT, VEC> vq[KP];
+#pragma unroll
+    for (int j = 0; j < KP; ++j) vq[j].load(tab + static_cast<int64_t>(sl[j]) * dh + c0);
+    float g[4];
+    gq.get(g);
 #pragma unroll
     for (int j = 0; j < KP; ++j) {
       float v[4];
-      load_vals<4, VT>(tab + static_cast<int64_t>(sl[j]) * dh + c0, v);
+      vq[j].get(v);
 #pragma unroll
       for (int e = 0; e < 4; ++e) d[j] = fmaf(g[e], v[e], d[j]);
     }
@@ -1753,12 +1794,12 @@ __global__ void __launch_bounds__(256) pick_keys_kernel(const int32_t* __restric
 // begun before piece s, [2 s + 1] begins a row that goes on after it.  table_values_join_kernel adds a row's pieces in
 // order and clears the rows without a pick.  The load follows the picks and not the rows: text repeats its tokens, so a
 // few rows hold hundreds of picks, and with one wave per row the longest row's chain of batches was the kernel's time
-// (B=4, T=1024, 4,096 rows of 768, k=16, a Zipf stream: 190 us; now 49 us and 10 for the join; the
+// (B=4, T=1024, 4,096 rows of 768, k=16, a Zipf stream: 190 us; now 42 us and 10 for the join; the
 // floor is the 101 MB of dy rows gathered through the caches).  Pieces of 32: the partial sums then take at most a
 // quarter of the gathered bytes again, and 2,048 waves are all resident at three to a SIMD.
 constexpr int kValuesSeg = 32;
 
-template <typename DyT>
+template <typename DyT, bool VEC>
 __global__ void __launch_bounds__(256) table_values_grad_kernel(const int32_t* __restrict__ sorted_keys,
                                                                 const int32_t* __restrict__ sorted_vals,
                                                                 const int32_t* __restrict__ offsets,
@@ -1818,13 +1859,13 @@ __global__ void __launch_bounds__(256) table_values_grad_kernel(const int32_t* _
         key[q] = sorted_keys[i];
         ro[q] = (static_cast<int64_t>(b) * T + t) * dy_stride + static_cast<int64_t>(h) * dh;
       }
-      float g[QS][CS][4];
+      Quad<DyT, VEC> gq[QS][CS];
 #pragma unroll
       for (int q = 0; q < QS; ++q) {
 #pragma unroll
         for (int s = 0; s < CS; ++s) {
           const int c0 = cb + 256 * s + 4 * lane;
-          if (c0 < dh) load_vals<4, DyT>(dy + ro[q] + c0, g[q][s]);
+          if (c0 < dh) gq[q][s].load(dy + ro[q] + c0);
         }
       }
 #pragma unroll
@@ -1836,9 +1877,12 @@ __global__ void __launch_bounds__(256) table_values_grad_kernel(const int32_t* _
         }
         if (i0 + q < n) {   // past the piece's end nothing is added: 0 * dy would keep an infinity's NaN
 #pragma unroll
-          for (int s = 0; s < CS; ++s)
+          for (int s = 0; s < CS; ++s) {
+            float g[4];
+            gq[q][s].get(g);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[s][c] = fmaf(w[q], g[q][s][c], acc[s][c]);
+            for (int c = 0; c < 4; ++c) acc[s][c] = fmaf(w[q], g[c], acc[s][c]);
+          }
         }
       }
     }
@@ -2464,15 +2508,16 @@ int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, 
       return set_err(SDM_RT_ELAUNCH, "table backward: sort failed");
     float* part = reinterpret_cast<float*>(ws + g.off_part);
     const unsigned sblocks = static_cast<unsigned>((values_pieces(g.n_entries) + 3) / 4);
+    const bool vec = quad_rows(dy, dy_row_stride, dy_dtype);
+#define SDM_RT_TV(DT, VEC)                                                                                          \
+  hipLaunchKernelGGL((table_values_grad_kernel<DT, VEC>), dim3(sblocks), dim3(256), 0, st, kout, vout, offsets,     \
+                     weights, static_cast<const DT*>(dy), dy_row_stride, d_values, part, p.T, p.H, p.pitch, p.M, p.dh)
     if (dy_dtype == SDM_RT_BF16) {
-      hipLaunchKernelGGL(table_values_grad_kernel<bf16_t>, dim3(sblocks), dim3(256), 0, st, kout, vout, offsets,
-                         weights, static_cast<const bf16_t*>(dy), dy_row_stride, d_values, part, p.T, p.H, p.pitch,
-                         p.M, p.dh);
+      if (vec) SDM_RT_TV(bf16_t, true); else SDM_RT_TV(bf16_t, false);
     } else {
-      hipLaunchKernelGGL(table_values_grad_kernel<float>, dim3(sblocks), dim3(256), 0, st, kout, vout, offsets,
-                         weights, static_cast<const float*>(dy), dy_row_stride, d_values, part, p.T, p.H, p.pitch,
-                         p.M, p.dh);
+      if (vec) SDM_RT_TV(float, true); else SDM_RT_TV(float, false);
     }
+#undef SDM_RT_TV
     if ((rc = check_launch("table values grad"))) return rc;
     hipLaunchKernelGGL(table_values_join_kernel, dim3(static_cast<unsigned>((n_keys + 2) / 4)), dim3(256), 0, st,
                        offsets, count, part, d_values, p.H * p.M, p.dh);
@@ -2482,18 +2527,22 @@ int sdm_rt_table_backward(const sdm_rt_dims* dims, const sdm_rt_params* params, 
   {
     const int64_t waves = static_cast<int64_t>(p.B) * p.T * p.H;
     const unsigned blocks = static_cast<unsigned>((waves + 3) / 4);
-#define SDM_RT_TG(KP, VT, DT)                                                                                      \
-  hipLaunchKernelGGL((table_grad_kernel<KP, VT, DT>), dim3(blocks), dim3(256), 0, st, slots, weights,              \
+    const bool vec = quad_rows(dy, dy_row_stride, dy_dtype) && quad_rows(values, p.dh, values_dtype);
+#define SDM_RT_TG_V(KP, VT, DT, VEC)                                                                                \
+  hipLaunchKernelGGL((table_grad_kernel<KP, VT, DT, VEC>), dim3(blocks), dim3(256), 0, st, slots, weights,              \
                      static_cast<const VT*>(values), static_cast<const DT*>(dy), dy_row_stride, dw, p.B, p.T, p.H,  \
                      p.M, p.dh, p.kk)
+#define SDM_RT_TG(KP, VT, DT) \
+  if (vec) SDM_RT_TG_V(KP, VT, DT, true); else SDM_RT_TG_V(KP, VT, DT, false)
 #define SDM_RT_TG_DT(KP, VT) \
-  if (dy_dtype == SDM_RT_BF16) SDM_RT_TG(KP, VT, bf16_t); else SDM_RT_TG(KP, VT, float)
+  if (dy_dtype == SDM_RT_BF16) { SDM_RT_TG(KP, VT, bf16_t); } else { SDM_RT_TG(KP, VT, float); }
 #define SDM_RT_TG_KP(VT) \
   if (p.pitch == 8) { SDM_RT_TG_DT(8, VT); } else { SDM_RT_TG_DT(16, VT); }
     if (values_dtype == SDM_RT_BF16) { SDM_RT_TG_KP(bf16_t); } else { SDM_RT_TG_KP(float); }
 #undef SDM_RT_TG_KP
 #undef SDM_RT_TG_DT
 #undef SDM_RT_TG
+#undef SDM_RT_TG_V
     if ((rc = check_launch("table grad"))) return rc;
   }
   // 3. softmax and product-key backward of the read set (no gate, no address bias)

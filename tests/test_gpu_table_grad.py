@@ -161,3 +161,25 @@ def test_table_backward_is_deterministic():
     torch.cuda.synchronize()
     for n in g1:
         assert torch.equal(g1[n], g2[n]), n
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_table_backward_on_rows_of_any_alignment(dtype):
+    """Rows of dy that start on no multiple of four values give the aligned rows' bits: the same sums."""
+    g = torch.Generator().manual_seed(11)
+    B, T, H, dh, d_a, n_sub, k = 2, 70, 2, 268, 16, 8, 16
+    q = torch.randn(B, T, H * d_a, generator=g).cuda()
+    k1, k2 = (torch.randn(H, n_sub, d_a // 2, generator=g).cuda() for _ in range(2))
+    ls = torch.full((H,), math.log(8.0)).cuda()
+    vals = torch.randn(H, n_sub * n_sub, dh, generator=g).cuda()
+    dy = torch.randn(B, T, H * dh, generator=g).cuda().to(dtype)
+    wide = torch.zeros(B, T, H * dh + 3, device="cuda", dtype=dtype)
+    wide[..., 1:1 + H * dh] = dy
+    say(f"[table grad] unaligned rows {dtype}")
+    prm = core._params(q.device, k1, k2, None, ls, None, None, None)
+    sl, sc, wt = core.address(q, k1, k2, k, ls, padded=True, params=prm)
+    g1 = core.table_backward(q, sl, wt, sc, vals, dy, k=k, params=prm)
+    g2 = core.table_backward(q, sl, wt, sc, vals, wide[..., 1:1 + H * dh], k=k, params=prm)
+    torch.cuda.synchronize()
+    for n in g1:
+        assert torch.equal(g1[n], g2[n]), n
