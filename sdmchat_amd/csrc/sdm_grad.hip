@@ -851,11 +851,12 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
     }
 
     // the written rows' new values (no other group writes them, so they can be summed before the reads are done):
-    // the old row faded by the chunk (as mu; by `keep` itself where the slab is emptied or rescaled), the slot's first
-    // writer and its later ones from the chain.  Group g takes records g + 64 k; null records (row M) write nothing
+    // the old row faded by the chunk (as mu; by itself where the slab is rescaled; none of it where a reset empties the
+    // slab, chosen and not multiplied by zero, which would keep an infinity's NaN), the slot's first writer and its
+    // later ones from the chain.  Group g takes records g + 64 k; null records (row M) write nothing
     const float mu_all = mu * pw[L];
-    const bool fold = rmask != 0 || !(mu_all >= kMuFloor);   // the slab takes the scale in: mu restarts at 1
-    const float keep = rmask ? 0.f : fold ? mu_all : 1.f;
+    // the slab takes the scale in, mu restarts at 1 (the same in every lane: a branch around it costs a chunk nothing)
+    const bool fold = __builtin_amdgcn_readfirstlane(rmask != 0 || !(mu_all >= kMuFloor));
     const float inv_mu = fold ? 1.f : fast_rcp(mu_all);
     const unsigned char* gext = chains + static_cast<int64_t>(c) * chain_stride(KP) + 16 + 8 * kChunk * KP;
     auto ext_at = [&](int e) {
@@ -883,13 +884,20 @@ __global__ void __launch_bounds__(kGradScanThreads) grad_scan_kernel(GradScanArg
       }
       const uint2 ow = cur.own_w[k0 / 8];   // the lane's count: record k0 + l8
       own_slot[k0 / 8] = static_cast<int>(ow.x & 0xffffu);
-      const float cold = cnt[own_slot[k0 / 8]] * keep;
+      float cold = cnt[own_slot[k0 / 8]];
+      if (fold) {
+        cold = rmask ? 0.f : cold * mu_all;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+          for (int k = 0; k < CPL; ++k) x[k0 + j].v[k] = rmask ? 0.f : x[k0 + j].v[k] * mu_all;
+      }
       float dcc = __uint_as_float(ow.y & 0x7fffffffu) * s_wc[(ow.x >> 16) & 63u];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float dc = __uint_as_float(wr[j].y & 0x7fffffffu) * inv_mu;
 #pragma unroll
-        for (int k = 0; k < CPL; ++k) x[k0 + j].v[k] = fmaf(dc, vq[j].v[k], x[k0 + j].v[k] * keep);
+        for (int k = 0; k < CPL; ++k) x[k0 + j].v[k] = fmaf(dc, vq[j].v[k], x[k0 + j].v[k]);
       }
       // the later writers of two records at a time, the next entries loaded ahead: a chain costs one LDS round trip a
       // writer, and the two records' overlap

@@ -173,6 +173,32 @@ def test_in_chunk_and_carried_gradients_at_chunk_edges(T, dh, k, reset_p, overla
     check_case("chunk", 41, 2, T, 2, dh, 16, 8, k, dtype=dtype, reset_p=reset_p, overlap=overlap)
 
 
+@pytest.mark.parametrize("bad", ["v", "dy"])
+@pytest.mark.parametrize("k", [8, 16])
+def test_a_reset_keeps_a_non_finite_document_out_of_its_neighbours_gradients(k, bad):
+    """Three packed documents; an infinity in the middle one's values (or a NaN in its dy) leaves the row gradients of the
+    other two as they are without it, bit for bit: both scans empty the memory at a reset and do not scale what it held
+    by zero.  The read-outs kept for the backward are those of finite values."""
+    B, T, H, dh = 1, 300, 2, 32
+    t, _ = make(43, B, T, H, dh, 16, 8, overlap=0.9)
+    d = {n: t[n].cuda() for n in NAMES}
+    reset = torch.zeros(B, T, dtype=torch.bool, device="cuda")
+    reset[0, [100, 230]] = True
+    cfg = dict(k=k, read_mode="mean", out_norm=True, read_eps=1e-3, out_norm_eps=1e-2)
+    prm = core._params(d["v"].device, *[d[n] for n in ("keys1", "keys2", "addr_b", "log_scale", "decay", "onorm_w",
+                                                       "gate_bias")])
+    _, saved = core.core_forward_train(d["kz"], d["qz"], d["v"], d["gl"], params=prm, reset=reset, **cfg)
+    dy = torch.randn(B, T, H * dh, generator=torch.Generator().manual_seed(6)).cuda()
+    v2, dy2 = d["v"].clone(), dy.clone()
+    (v2 if bad == "v" else dy2)[0, 150] = math.inf if bad == "v" else math.nan
+    g0 = core.core_backward(d["kz"], d["qz"], d["v"], d["gl"], saved, dy, params=prm, **cfg)
+    g1 = core.core_backward(d["kz"], d["qz"], v2, d["gl"], saved, dy2, params=prm, **cfg)
+    other = [*range(100), *range(230, T)]
+    assert not bool(torch.isfinite(g1["v" if bad == "dy" else "qz"][:, 100:230]).all())
+    for n in ("kz", "qz", "v", "gate_logits"):
+        assert torch.equal(g1[n][:, other], g0[n][:, other]), n
+
+
 def test_backward_is_deterministic():
     t, reset = make(16, 1, 200, 4, 32, 16, 8, overlap=0.7)
     cfg = dict(k=8, read_mode="mean", out_norm=True, read_eps=1e-3, out_norm_eps=1e-2)
