@@ -1063,10 +1063,10 @@ __device__ __forceinline__ float pick_sum(float v) {
 }
 
 
+// one block of addr_grad_kernel, on addr_grad_lds(n_sub, HALF, its waves) bytes of LDS
 template <int HALF, int KP, typename InT>
-__global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel(AddrGradArgs a) {
+__device__ __forceinline__ void addr_grad_block(const AddrGradArgs& a, unsigned char* albuf) {
   constexpr int DA = 2 * HALF;
-  extern __shared__ __attribute__((aligned(16))) unsigned char albuf[];
   const int W = blockDim.x >> 6;
   const int n_sub = a.n_sub;
   const int KS = 2 * n_sub * HALF;                                // sub-key values of both halves
@@ -1254,6 +1254,12 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
   }
 }
 
+template <int HALF, int KP, typename InT>
+__global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel(AddrGradArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char agbuf[];
+  addr_grad_block<HALF, KP, InT>(a, agbuf);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // addr_grad_tile_kernel: the same gradients for n_sub <= 64, 32 tokens of one (head, address set) at a time on the
 // matrix cores.  Per tile a wave
@@ -1271,6 +1277,9 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
 // copy's rate) and the latency of a tile's chain (loads, k LDS additions, products) with two waves per SIMD: the
 // kernel takes 256 registers, and at three waves (168, 73 of them spilled) it took 141 us.
 // Sub-keys past n_sub, columns past the address and tokens past the end are zero rows and columns of the tiles.
+// The products run over every sub-key and 32 tokens, and 0 times an infinity is NaN: a block that meets an address or a
+// sub-key that is not finite does all its tokens again one at a time (addr_grad_block), so that it reaches no more than
+// its own picks.
 // Waves per block 4; tiles per wave chosen by addr_tiles (enough blocks for the chip first, then longer waves, since
 // every wave loads the head's sub-keys and leaves a partial sum).
 constexpr int kAddrTile = 32;
@@ -1311,8 +1320,12 @@ __host__ __device__ constexpr int addr_tile_pitch(int nsb) { return 64 * nsb + 4
 __host__ __device__ constexpr size_t addr_tile_lds(int n_sub, int half, int nsb) {
   const size_t g = sizeof(float) * (kAddrTileWaves * kAddrTile * addr_tile_pitch(nsb) + 64 * nsb * 32);
   const size_t d = sizeof(float) * kAddrTileWaves * 2 * static_cast<size_t>(n_sub) * half;
-  return (g > d ? g : d) + kAddrTileWaves * (sizeof(double) + sizeof(float) * (2 * half + 2));
+  const size_t t = (g > d ? g : d) + kAddrTileWaves * (sizeof(double) + sizeof(float) * (2 * half + 2));
+  const size_t o = (addr_grad_lds(n_sub, half, kAddrTileWaves) + 7) / 8 * 8;   // one token at a time
+  return t > o ? t : o;
 }
+
+__device__ __forceinline__ bool finite_f32(float v) { return fabsf(v) <= 3.402823466e38f; }
 
 template <int HALF, int NSB, int KP, typename InT>
 __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(AddrGradArgs a) {
@@ -1339,6 +1352,8 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
   // the unit sub-keys, [half][sub-key][column of its tile]: zero past n_sub and, with both halves in one tile, in the
   // other half's columns
   float* kn = reinterpret_cast<float*>(albuf) + kAddrTileWaves * kAddrTile * GP;
+  __shared__ int s_odd[kAddrTileWaves];   // whether the wave met an address or a sub-key that is not finite
+  bool fin = true;
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     const float* keys = a.keys[p] + static_cast<int64_t>(h) * n_sub * HALF;
@@ -1348,7 +1363,9 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
       const int i = i0 + hw;
       const float v = own && i < n_sub ? keys[i * HALF + c] : 0.f;
       const float nrm = fmaxf(sqrtf(col_sum<HALF>(v * v, col)), 1e-12f);
-      kn[(p * SB + i) * 32 + col] = v / nrm;
+      const float kv = v / nrm;
+      fin = fin && finite_f32(kv);
+      kn[(p * SB + i) * 32 + col] = kv;
     }
   }
   __syncthreads();
@@ -1544,6 +1561,19 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
     }
     wave_lds_fence();
   }
+  // an address element that is not finite has left NaN in its column of every sub-key's sum
+  bool odd = __ballot(!fin) != 0ull;
+#pragma unroll
+  for (int p = 0; p < NT; ++p) {
+    bool bad = true;
+#pragma unroll
+    for (int q = 0; q < NSB; ++q)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad = bad && !finite_f32(dk[p][q][r]);
+    const unsigned long long b = __ballot(bad);
+    odd = odd || (static_cast<uint32_t>(b) & static_cast<uint32_t>(b >> 32)) != 0u;   // a column's rows: both half-waves
+  }
+  if (lane == 0) s_odd[w] = odd;
   // block sums in a fixed order: waves -> LDS -> threads
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -1554,6 +1584,12 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
 #pragma unroll
   for (int p = 0; p < NT; ++p) acc_ab[p] += __shfl_xor(acc_ab[p], 32);
   __syncthreads();   // every wave's G is done with
+  if (s_odd[0] | s_odd[1] | s_odd[2] | s_odd[3]) {   // rare
+    __threadfence();   // the block's row gradients, written again by other threads
+    __syncthreads();
+    addr_grad_block<HALF, KP, InT>(a, albuf);
+    return;
+  }
   float* dkb = reinterpret_cast<float*>(albuf);
   unsigned char* tail = albuf + (addr_tile_lds(n_sub, HALF, NSB) -
                                  kAddrTileWaves * (sizeof(double) + sizeof(float) * (2 * HALF + 2)));

@@ -173,6 +173,61 @@ def test_in_chunk_and_carried_gradients_at_chunk_edges(T, dh, k, reset_p, overla
     check_case("chunk", 41, 2, T, 2, dh, 16, 8, k, dtype=dtype, reset_p=reset_p, overlap=overlap)
 
 
+@pytest.mark.parametrize("n_sub,d_a,k,value", [
+    (32, 64, 8, math.inf), (32, 64, 8, math.nan), (50, 32, 16, math.inf),   # a column tile per half; two row blocks
+    (33, 48, 8, math.nan), (12, 6, 4, math.inf), (12, 6, 4, math.nan),      # ... and both halves in one tile
+])
+def test_non_finite_addresses_and_sub_keys_reach_only_their_picks(n_sub, d_a, k, value):
+    """A token with a non-finite address spoils the gradients of the sub-keys that it picked, and a non-finite sub-key
+    those of the tokens that picked it, in the address half that holds it: all others stay what they are without it,
+    though addr_grad_tile_kernel's products run over every sub-key and 32 tokens (its blocks that meet one take their
+    tokens one by one, sums of up to 150 tokens in another order: 150 2^-24 of the largest).  The picks are those of
+    finite inputs."""
+    B, T, H, dh, half = 1, 150, 2, 16, d_a // 2
+    t, _ = make(44, B, T, H, dh, d_a, n_sub, overlap=0.8)
+    d = {n: t[n].cuda() for n in NAMES}
+    cfg = dict(k=k, read_mode="mean", out_norm=True, read_eps=1e-3, out_norm_eps=1e-2)
+
+    def prm(**over):
+        p = dict(d, **over)
+        return core._params(p["keys1"].device, *[p[n] for n in ("keys1", "keys2", "addr_b", "log_scale", "decay",
+                                                                "onorm_w", "gate_bias")])
+    clean = prm()
+    _, saved = core.core_forward_train(d["kz"], d["qz"], d["v"], d["gl"], params=clean, **cfg)
+    dy = torch.randn(B, T, H * dh, generator=torch.Generator().manual_seed(9)).cuda()
+
+    def back(kz=d["kz"], params=clean):
+        return core.core_backward(kz, d["qz"], d["v"], d["gl"], saved, dy, params=params, **cfg)
+
+    def same(a, b):
+        return (a - b).abs().max().item() <= 150 * 2.0 ** -24 * b.abs().max().item()
+    g0 = back()
+    kk = min(k, min(k, n_sub) ** 2)
+    h, tok, sub = 1, 70, int(saved["slots_w"][0, 1, 70, 0]) // n_sub
+    # an address: element 1 of the first half
+    kz = d["kz"].clone()
+    kz[0, tok, h * d_a + 1] = value
+    g1 = back(kz=kz)
+    picked = torch.zeros(n_sub, dtype=torch.bool, device="cuda")
+    picked[(saved["slots_w"][0, h, tok, :kk] // n_sub).long()] = True
+    assert not bool(torch.isfinite(g1["keys1"][h][picked]).all(-1).any())
+    assert same(g1["keys1"][h][~picked], g0["keys1"][h][~picked])
+    assert same(g1["keys2"], g0["keys2"]) and torch.equal(g1["keys1"][0], g0["keys1"][0])
+    rest = [i for i in range(T) if i != tok]
+    assert same(g1["kz"][:, rest], g0["kz"][:, rest]) and torch.equal(g1["qz"], g0["qz"])
+    # a sub-key of the first half
+    keys1 = d["keys1"].clone()
+    keys1[h, sub, 0] = value
+    g2 = back(params=prm(keys1=keys1))
+    hit = ((saved["slots_w"][0, h, :, :kk] // n_sub) == sub).any(-1)
+    assert 0 < int(hit.sum()) < T
+    z2, z0 = (g["kz"][0].view(T, H, d_a) for g in (g2, g0))
+    assert not bool(torch.isfinite(z2[hit, h, :half]).any())
+    assert same(z2[~hit], z0[~hit]) and same(z2[:, h, half:], z0[:, h, half:]) and torch.equal(z2[:, 0], z0[:, 0])
+    other = [i for i in range(n_sub) if i != sub]
+    assert same(g2["keys1"][h][other], g0["keys1"][h][other]) and same(g2["keys2"], g0["keys2"])
+
+
 @pytest.mark.parametrize("bad", ["v", "dy"])
 @pytest.mark.parametrize("k", [8, 16])
 def test_a_reset_keeps_a_non_finite_document_out_of_its_neighbours_gradients(k, bad):
