@@ -53,7 +53,9 @@ inline bool pick_path(const Plan& p) {
 // and 25.6 us for the two launches, the states' way through memory and the slabs' loads, against the whole sequence at
 // the scan's rate.  Measured with 12 slabs of two groups, scan alone and in segments, whole layer in bfloat16: T=704
 // 90 and 90 us, 1,024 107 and 91, 2,048 168 and 111, 8,192 497 and 200 (scan 399; sums 37, join 10, scan 55); 36 slabs,
-// T=2,048 206 and 189.
+// T=2,048 206 and 189.  The rates of crowded addresses (one repeated token: scan 4.6 us a chunk, sums 3.8) leave the line
+// where it is: the core on one repeated token, whole and in segments, 12 slabs, T=768 111 and 101 us, 36 slabs, T=2,048
+// 216 and 185, 60 slabs, T=8,192 844 and 827 (varied tokens 59 and 59, 129 and 110, 472 and 447).
 struct PickSegments {
   int segs, seg_chunks;
   size_t off_cnt, off_fade, bytes;   // of the workspace behind Plan::total
@@ -121,8 +123,77 @@ __device__ __forceinline__ void spread_pieces(const float4& f, float (&vp)[32]) 
   }
 }
 
+// A wave with a slot of many later writers (crowded addresses) writes as eight teams: team j, the lanes of pick j of the
+// wave's eight positions, takes the owned slots of its members one after another.  This sums member k's: the member's row
+// y and count cw (its own value added) and the slot's later writers (every eighth, from the lane's index in the team) per
+// lane, then over the team (lanes 8 apart) by a fixed butterfly that leaves each lane one four-column piece of the row
+// (h4; number lane / 8 of the read order) and the slot's count (ct).  Every lane of the wave calls it, with its own write
+// record wr; mslot: the member's slot (M: it owns none).  ent(i): the chunk's entry i; add(c, v, acc): value row v times c.
+template <typename Ent, typename Add>
+__device__ __forceinline__ void team_row(int k, int lane, int M, const uint3& wr, const float (&y)[32], float cw,
+                                         float inv_mu, const Ent& ent, const Add& add, float (&h4)[4], float& ct,
+                                         int& mslot) {
+  const int mi = lane >> 3;   // the lane's member index in its team
+  const int src = 8 * k + (lane & 7);
+  const uint32_t mx = static_cast<uint32_t>(__shfl(static_cast<int>(wr.x), src));
+  const uint32_t mz = static_cast<uint32_t>(__shfl(static_cast<int>(wr.z), src));
+  mslot = static_cast<int>(mx & 0x7ffu);
+  float part[32];
+  float cwp = 0.f;
+  const bool self = mi == k && mslot != M;   // the member itself: its row with its own value added
+#pragma unroll
+  for (int q = 0; q < 32; ++q) part[q] = self ? y[q] : 0.f;
+  if (self) cwp = cw;
+  if (mslot != M) {   // later writers mi, mi + 8, ...: 0 is the inline one, i > 0 entry w_e0 + i - 1
+    const int n_l = static_cast<int>((mx >> 17) & 63u);
+    const int w_e0 = static_cast<int>(mx >> 23);
+    for (int i = mi; i < n_l; i += 8) {
+      const uint2 it = i == 0 ? make_uint2(mz, (mx >> 11) & 63u) : ent(w_e0 + i - 1);
+      const float ae = __uint_as_float(it.x) * inv_mu;
+      add(ae, static_cast<int>(it.y & 63u), part);
+      cwp += ae;
+    }
+  }
+  // over the team: lanes 32 apart (32 -> 16 values), 16 apart (-> 8), 8 apart (-> 4)
+  float h16[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part[q]), __float_as_uint(part[16 + q]), false,
+                                                     false);
+    h16[q] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);   // lane < 32: values q, else 16 + q
+  }
+  const bool b4 = lane & 16, b3 = lane & 8;
+  float h8[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float keep = b4 ? h16[8 + q] : h16[q];
+    h8[q] = keep + __shfl_xor(b4 ? h16[q] : h16[8 + q], 16);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float keep = b3 ? h8[4 + q] : h8[q];
+    h4[q] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(b3 ? h8[q] : h8[4 + q]), 0x128, 0xf,
+                                                              0xf, false));   // row_ror:8
+  }
+  ct = cwp;
+  ct += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ct), 0x128, 0xf, 0xf, false));
+  ct += __shfl_xor(ct, 16);
+  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ct), __float_as_uint(ct), false, false);
+  ct = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
+
+// the team's store of member k's slot: the lane's piece and the count
+__device__ __forceinline__ void team_store(int k, int lane, int M, unsigned char* A, float* cnt, const float (&h4)[4],
+                                           float ct, int mslot) {
+  if (mslot == M) return;
+  const int mi = lane >> 3;
+  const int piece = (lane & 7) ^ (mi < 4 ? mi : 11 - mi);
+  *reinterpret_cast<float4*>(A + mslot * (kPickCols * 4) + 16 * piece) = make_float4(h4[0], h4[1], h4[2], h4[3]);
+  if (mi == k) cnt[mslot] = ct;
+}
+
 // The writes of one segment (not the last) of a slab's 32-column group, summed from an empty slab: pick_scan_kernel's
-// plain chunk step without its reads, so a chunk needs one barrier and its lanes only their own rows.  Leaves the
+// plain chunk step without its reads, so a chunk needs one barrier and its waves only their own rows.  Leaves the
 // segment's state contribution in seg_mem / seg_cnt and its fade in seg_fade.  Bound by the chunk's chain of dependent
 // LDS accesses, the longest list of a slot's later writers in it: 37 us for 13 chunks with the slab's clear and store
 // (loads two chunks ahead instead of one: the same).
@@ -151,6 +222,7 @@ __global__ void __launch_bounds__(kPickThreads) pick_sum_kernel(ScanArgs a) {
   float* pw = reinterpret_cast<float*>(var + 2 * VS);
   int32_t* s_sizes = reinterpret_cast<int32_t*>(pw + 68);
   const int tid = threadIdx.x;
+  const int lane = tid & 63;
   const int p = tid >> 3;
   const int j = tid & 7;
   const int col0 = g * CW;
@@ -234,14 +306,21 @@ __global__ void __launch_bounds__(kPickThreads) pick_sum_kernel(ScanArgs a) {
       mu = 1.f;
       lds_barrier();
     }
-    // every owner adds its own faded value and those of the slot's later writers to the slot's row
+    // every owner adds its own faded value and those of the slot's later writers to the slot's row; a wave with a slot
+    // of many of them in teams, as the scan (one repeated token, 60 slabs of 128 chunks in two segments: 14.4 us a chunk
+    // by the owners alone, 3.8 us in teams)
     const int wslot = static_cast<int>(wr.x & 0x7ffu);
-    float vp[32];
+    const bool own = wslot != M;
+    const float inv_mu = fast_rcp(mu);
+    auto ent = [&](int i) {
+      const int o = PickGeom::off_ent() + 8 * min(i, PickGeom::max_entries() - 1);
+      return o + 8 <= VS ? *reinterpret_cast<const uint2*>(varc + o) : *reinterpret_cast<const uint2*>(gvar + o);
+    };
+    float vp[32], y[32];
+    float cw = 0.f;
     spread_pieces(v_cur, vp);
-    if (wslot != M) {
-      const float inv_mu = fast_rcp(mu);
-      unsigned char* row = A_b + wslot * (CW * 4);
-      float y[32];
+    unsigned char* row = A_b + wslot * (CW * 4);
+    if (own) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const float4 q4 = *reinterpret_cast<const float4*>(row + soff[k]);
@@ -250,29 +329,40 @@ __global__ void __launch_bounds__(kPickThreads) pick_sum_kernel(ScanArgs a) {
         y[4 * k + 2] = q4.z;
         y[4 * k + 3] = q4.w;
       }
-      float cw = cnt[wslot];
       const float a0 = __uint_as_float(wr.y) * inv_mu;
 #pragma unroll
       for (int k = 0; k < 32; ++k) y[k] = fmaf(a0, vp[k], y[k]);
-      cw += a0;
-      const int n_l = static_cast<int>((wr.x >> 17) & 63u);
+      cw = cnt[wslot] + a0;
+    }
+    const int n_l = own ? static_cast<int>((wr.x >> 17) & 63u) : 0;
+    if (!__ballot(n_l >= kTeamWriters)) {
       if (n_l > 0) {
         const float a1 = __uint_as_float(wr.z) * inv_mu;
         add_vrow(a1, static_cast<int>((wr.x >> 11) & 63u), y);
         cw += a1;
         const int w_e0 = static_cast<int>(wr.x >> 23);
         for (int e = 0; e < n_l - 1; ++e) {
-          const int o = PickGeom::off_ent() + 8 * min(w_e0 + e, PickGeom::max_entries() - 1);
-          const uint2 en = o + 8 <= VS ? *reinterpret_cast<const uint2*>(varc + o) : *reinterpret_cast<const uint2*>(gvar + o);
+          const uint2 en = ent(w_e0 + e);
           const float ae = __uint_as_float(en.x) * inv_mu;
           add_vrow(ae, static_cast<int>(en.y & 63u), y);
           cw += ae;
         }
       }
+      if (own) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        *reinterpret_cast<float4*>(row + soff[k]) = make_float4(y[4 * k], y[4 * k + 1], y[4 * k + 2], y[4 * k + 3]);
-      cnt[wslot] = cw;
+        for (int k = 0; k < 8; ++k)
+          *reinterpret_cast<float4*>(row + soff[k]) = make_float4(y[4 * k], y[4 * k + 1], y[4 * k + 2], y[4 * k + 3]);
+        cnt[wslot] = cw;
+      }
+    } else {
+      const unsigned long long owners = __ballot(own);
+      for (int k = 0; k < 8; ++k) {
+        if (!((owners >> (8 * k)) & 0xffull)) continue;   // no owner among the teams' members k
+        float h4[4], ct;
+        int ms;
+        team_row(k, lane, M, wr, y, cw, inv_mu, ent, add_vrow, h4, ct, ms);
+        team_store(k, lane, M, A_b, cnt, h4, ct, ms);
+      }
     }
     wr = wr_n;
     v_cur = v_n;
@@ -722,69 +812,9 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
       }
       const int n_l_own = wslot != M ? static_cast<int>((wr.x >> 17) & 63u) : 0;
       const bool teams = __ballot(n_l_own >= kTeamWriters);
-      // the teams of a crowded wave (as in the plain step): team j, the lanes of pick j of the wave's eight positions,
-      // sums the owned slots of its members one after another and leaves each lane one four-column piece (h4) of the
-      // member's row and the team the slot's count (ct)
+      // the teams of a crowded wave (team_row)
       const unsigned long long owners = __ballot(wslot != M);
-      const int mi = lane >> 3;   // the lane's member index in its team
-      auto team_member = [&](int k, float (&h4)[4], float& ct, int& mslot) {
-        const int src = 8 * k + j;
-        const uint32_t mx = static_cast<uint32_t>(__shfl(static_cast<int>(wr.x), src));
-        const uint32_t mz = static_cast<uint32_t>(__shfl(static_cast<int>(wr.z), src));
-        mslot = static_cast<int>(mx & 0x7ffu);
-        float part[32];
-        float cwp = 0.f;
-        const bool self = mi == k && mslot != M;   // the member itself: its row with its own value added
-#pragma unroll
-        for (int q = 0; q < 32; ++q) part[q] = self ? y[q] : 0.f;
-        if (self) cwp = cw;
-        if (mslot != M) {   // later writers mi, mi + 8, ...: 0 is the inline one, i > 0 entry w_e0 + i - 1
-          const int n_l = static_cast<int>((mx >> 17) & 63u);
-          const int w_e0 = static_cast<int>(mx >> 23);
-          for (int i = mi; i < n_l; i += 8) {
-            const uint2 it = i == 0 ? make_uint2(mz, (mx >> 11) & 63u) : ent_at(w_e0 + i - 1, std::false_type{});
-            const float ae = __uint_as_float(it.x) * inv_mu;
-            add_vrow(ae, static_cast<int>(it.y & 63u), part);
-            cwp += ae;
-          }
-        }
-        // over the team: lanes 32 apart (32 -> 16 values), 16 apart (-> 8), 8 apart (-> 4)
-        float h16[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part[q]), __float_as_uint(part[16 + q]),
-                                                           false, false);
-          h16[q] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);   // lane < 32: values q, else 16 + q
-        }
-        const bool b4 = lane & 16, b3 = lane & 8;
-        float h8[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const float keep = b4 ? h16[8 + q] : h16[q];
-          h8[q] = keep + __shfl_xor(b4 ? h16[q] : h16[8 + q], 16);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float keep = b3 ? h8[4 + q] : h8[q];
-          h4[q] = keep + __int_as_float(__builtin_amdgcn_update_dpp(
-                             0, __float_as_int(b3 ? h8[q] : h8[4 + q]), 0x128, 0xf, 0xf, false));   // row_ror:8
-        }
-        ct = cwp;
-        ct += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ct), 0x128, 0xf, 0xf, false));
-        ct += __shfl_xor(ct, 16);
-        {
-          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ct), __float_as_uint(ct), false, false);
-          ct = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-        }
-      };
-      // the team's store of member k's slot: the lane's piece (number mi of the read order) and the count
-      auto team_store = [&](int k, const float (&h4)[4], float ct, int mslot) {
-        if (mslot != M) {
-          const int piece = j ^ (mi < 4 ? mi : 11 - mi);
-          *reinterpret_cast<float4*>(A_w + mslot * (CW * 4) + 16 * piece) = make_float4(h4[0], h4[1], h4[2], h4[3]);
-          if (mi == k) cnt[mslot] = ct;
-        }
-      };
+      auto ent = [&](int e) { return ent_at(e, std::false_type{}); };
       uint32_t members = 0;   // members with owned slots (bit k: member k)
 #pragma unroll
       for (int k = 0; k < 8; ++k) members |= ((owners >> (8 * k)) & 0xffull) ? (1u << k) : 0u;
@@ -807,7 +837,7 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
           }
         }
       } else if (team_now) {
-        team_member(k1, h4a, cta, msa);
+        team_row(k1, lane, M, wr, y, cw, inv_mu, ent, add_vrow, h4a, cta, msa);
       }
       lds_barrier();
       // the partner's partial sums of chunk c - 2 (used when it finishes, at the end of this chunk)
@@ -836,14 +866,14 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
           cnt[wslot] = cw;
         }
       } else if (team_now) {
-        team_store(k1, h4a, cta, msa);
+        team_store(k1, lane, M, A_w, cnt, h4a, cta, msa);
       } else {
         for (int k = 0; k < 8; ++k) {   // several members: each summed and stored in turn, after the barrier
           if (!((members >> k) & 1u)) continue;
           float h4[4], ct;
           int ms;
-          team_member(k, h4, ct, ms);
-          team_store(k, h4, ct, ms);
+          team_row(k, lane, M, wr, y, cw, inv_mu, ent, add_vrow, h4, ct, ms);
+          team_store(k, lane, M, A_w, cnt, h4, ct, ms);
         }
       }
       } else {
@@ -914,73 +944,15 @@ __global__ void __launch_bounds__(kPickThreads) pick_scan_kernel(ScanArgs a) {
           cnt[wslot] = cw;
         }
       } else {
-        // A wave with a slot of many later writers (crowded addresses) writes as eight teams: team j, the lanes of
-        // pick j of the wave's eight positions, takes the owned slots of its members one after another; the member's
-        // row (its own value added) and the slot's later writers (every eighth, from the member's index in the team)
-        // are summed per lane, then over the team (lanes 8 apart) by a fixed butterfly that leaves each lane one
-        // four-column piece of the row, which it stores.
-        const unsigned long long owners = __ballot(wslot != M);
-        const int mi = lane >> 3;   // the lane's member index in its team
-        auto team = [&](auto st) {
-          for (int k = 0; k < 8; ++k) {
-            if (!((owners >> (8 * k)) & 0xffull)) continue;   // no owner among the teams' members k
-            const int src = 8 * k + j;
-            const uint32_t mx = static_cast<uint32_t>(__shfl(static_cast<int>(wr.x), src));
-            const uint32_t mz = static_cast<uint32_t>(__shfl(static_cast<int>(wr.z), src));
-            const int mslot = static_cast<int>(mx & 0x7ffu);
-            float part[32];
-            float cwp = 0.f;
-            const bool self = mi == k && mslot != M;   // the member itself: its row with its own value added
-#pragma unroll
-            for (int q = 0; q < 32; ++q) part[q] = self ? y[q] : 0.f;
-            if (self) cwp = cw;
-            if (mslot != M) {   // later writers mi, mi + 8, ...: 0 is the inline one, i > 0 entry w_e0 + i - 1
-              const int n_l = static_cast<int>((mx >> 17) & 63u);
-              const int w_e0 = static_cast<int>(mx >> 23);
-              for (int i = mi; i < n_l; i += 8) {
-                const uint2 it = i == 0 ? make_uint2(mz, (mx >> 11) & 63u) : ent_at(w_e0 + i - 1, st);
-                const float ae = __uint_as_float(it.x) * inv_mu;
-                add_vrow(ae, static_cast<int>(it.y & 63u), part);
-                cwp += ae;
-              }
-            }
-            // over the team: lanes 32 apart (32 -> 16 values), 16 apart (-> 8), 8 apart (-> 4)
-            float h16[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-              const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part[q]), __float_as_uint(part[16 + q]),
-                                                               false, false);
-              h16[q] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);   // lane < 32: values q, else 16 + q
-            }
-            const bool b4 = lane & 16, b3 = lane & 8;
-            float h8[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const float keep = b4 ? h16[8 + q] : h16[q];
-              h8[q] = keep + __shfl_xor(b4 ? h16[q] : h16[8 + q], 16);
-            }
-            float h4[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const float keep = b3 ? h8[4 + q] : h8[q];
-              h4[q] = keep + __int_as_float(__builtin_amdgcn_update_dpp(
-                                 0, __float_as_int(b3 ? h8[q] : h8[4 + q]), 0x128, 0xf, 0xf, false));   // row_ror:8
-            }
-            float ct = cwp;
-            ct += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ct), 0x128, 0xf, 0xf, false));
-            ct += __shfl_xor(ct, 16);
-            {
-              const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ct), __float_as_uint(ct), false, false);
-              ct = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-            }
-            if (mslot != M) {   // the lane's piece: number mi of the read order
-              const int piece = j ^ (mi < 4 ? mi : 11 - mi);
-              *reinterpret_cast<float4*>(A_w + mslot * (CW * 4) + 16 * piece) = make_float4(h4[0], h4[1], h4[2], h4[3]);
-              if (mi == k) cnt[mslot] = ct;
-            }
-          }
-        };
-        team(std::false_type{});   // rare: one instance, the entries staged or not
+        const unsigned long long owners = __ballot(wslot != M);   // the teams of a crowded wave (team_row)
+        auto ent = [&](int e) { return ent_at(e, std::false_type{}); };   // rare: one instance, staged or not
+        for (int k = 0; k < 8; ++k) {
+          if (!((owners >> (8 * k)) & 0xffull)) continue;   // no owner among the teams' members k
+          float h4[4], ct;
+          int ms;
+          team_row(k, lane, M, wr, y, cw, inv_mu, ent, add_vrow, h4, ct, ms);
+          team_store(k, lane, M, A_w, cnt, h4, ct, ms);
+        }
       }
       }
       mu = mu_new;

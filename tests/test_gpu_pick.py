@@ -376,6 +376,59 @@ def test_segments_side_by_side_match_the_sequence_in_pieces(B, T, H, dh, dtype, 
     np.testing.assert_allclose(c, st[1], atol=2e-5, rtol=2e-5)
 
 
+def _pieces(kz, qz, V, g, p, reset, **kw):
+    """The core over pieces of 128 positions, each from the state that the one before left: unsegmented calls."""
+    want, st = [], None
+    for t0 in range(0, kz.shape[1], 128):
+        sl = slice(t0, min(t0 + 128, kz.shape[1]))
+        rr, st = gpu_core(kz[:, sl], qz[:, sl], V[:, sl], g[:, sl], p, 8, state_in=st, reset=reset[:, sl], **kw)
+        want.append(rr)
+    return np.concatenate(want, 1), st
+
+
+def _segmented(B, T, H, dh, n_sub, d_a=64):
+    """Whether a call's workspace holds the states of segments."""
+    nbytes = [core.workspace_bytes(core.make_dims(B, 64 * c, H, dh, d_a, n_sub, 8)) for c in (2, 3, (T + 63) // 64)]
+    chunk = nbytes[1] - nbytes[0]
+    return nbytes[2] > nbytes[1] + chunk * ((T + 63) // 64 - 3) + 4 * n_sub * n_sub * dh * B * H
+
+
+@pytest.mark.parametrize("pattern,dtype", [("bias", torch.float32), ("same", torch.float32), ("same", torch.bfloat16),
+                                           ("cycle3", torch.float32), ("three_in_four", torch.bfloat16)])
+def test_segments_of_crowded_prompts(pattern, dtype):
+    """Segments where tokens repeat (or share a large address bias): slots of up to 63 later writers in a chunk, plans
+    past the 4 KB that are staged, so the sums read entries from memory and add in teams and the segments' scans run
+    the step whose owners sum before the read barrier.  With a reset inside a segment, at a segment's first position and
+    none; bounds as above."""
+    B, T, H, dh, n_sub = 1, 1300, 12, 64, 32   # seven segments of three chunks, the last of 148 positions
+    kz, qz, V, g, p = core_inputs(B, T, H, dh, 64, n_sub, seed=71, decays=(0.3, 0.97, 1.0) * 4,
+                                  addr_bias=4.0 if pattern == "bias" else 0.3)
+    if pattern != "bias":
+        kz, qz, g = (_repeat(a, pattern) for a in (kz, qz, g))
+    if dtype == torch.bfloat16:
+        kz, qz, V, g = (bf16_round(a) for a in (kz, qz, V, g))
+    assert _segmented(B, T, H, dh, n_sub)
+    ws = core.CoreWorkspace()
+    tp = {n: torch.from_numpy(v).cuda() for n, v in p.items()}
+    core.core_forward(*(torch.from_numpy(a).cuda().to(dtype) for a in (kz, qz, V, g)), keys1=tp["keys1"],
+                      keys2=tp["keys2"], log_scale=tp["log_scale"], decay=tp["decay"], addr_b=tp["addr_b"],
+                      onorm_w=tp["onorm_w"], gate_bias=tp["gate_bias"], k=8, workspace=ws)
+    sizes = ws.buf[:4 * H * 21].cpu().view(torch.int32)
+    say(f"[segments] {pattern} {dtype}: variable parts up to {int(sizes.max())} B")
+    assert pattern not in ("bias", "same") or int(sizes.max()) > 4096
+    for resets in ((), (130, 131, 576)):
+        reset = np.zeros((B, T), bool)
+        reset[0, list(resets)] = True
+        kw = dict(dtype=dtype, out_dtype=torch.float32, want_state=True)
+        r, (mem, c) = gpu_core(kz, qz, V, g, p, 8, reset=reset, **kw)
+        want, st = _pieces(kz, qz, V, g, p, reset, **kw)
+        np.testing.assert_allclose(r, want, atol=2e-5, rtol=2e-5)
+        # one location takes all T writes of weight up to one: sums of T terms, of which T^0.5 roundings add up
+        scale = max(1.0, float(np.abs(st[0]).max()), float(st[1].max()))
+        np.testing.assert_allclose(mem, st[0], atol=2e-5 * scale, rtol=2e-5)
+        np.testing.assert_allclose(c, st[1], atol=2e-5 * scale, rtol=2e-5)
+
+
 def test_segments_state_written_over_its_input():
     """A state written back over the one it came from takes the unsegmented scan: the last segment could end before the
     first has read."""
