@@ -57,6 +57,12 @@ def _rows16(t2):
     return t2.stride(1) == 1 and t2.data_ptr() % 16 == 0 and (t2.stride(0) * es) % 16 == 0
 
 
+def _own_rows(t2):
+    """A 2-D view as rows that the kernels take: itself where the rows are 16-byte aligned (_rows16) and do not overlap (a
+    row broadcast over many has stride 0), else a copy."""
+    return t2 if _rows16(t2) and t2.stride(0) >= t2.shape[1] else t2.clone(memory_format=torch.contiguous_format)
+
+
 def _f32(t, device):
     if t is None:
         return None
@@ -563,8 +569,8 @@ def rms_norm(x, w, eps=1e-6, out_dtype=None, out=None):
         raise ValueError(f"rms_norm: dtype {x.dtype} is not float32 or bfloat16")
     d = x.shape[-1]
     x2 = x.reshape(-1, d)
-    if x2.numel() and not _rows16(x2):   # the kernel reads rows in 16-byte pieces
-        x2 = x2.contiguous()
+    if x2.numel():
+        x2 = _own_rows(x2)
     out_dtype = out_dtype or x.dtype
     if out is None:
         out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
@@ -620,11 +626,7 @@ def rms_norm_backward(x, w, dy, eps, need_x=True, need_w=True):
         dx = r * (gw - n * (gw * n).mean(-1, keepdim=True)) if need_x else None
         dw = (g * n).reshape(-1, d).sum(0) if need_w else None
         return None if dx is None else dx.to(x.dtype), None if dw is None else dw.to(w.dtype)
-    x2, dy2 = x.reshape(rows, d), dy.reshape(rows, d)
-    if not _rows16(x2):
-        x2 = _aligned(x2)
-    if not _rows16(dy2):
-        dy2 = _aligned(dy2)
+    x2, dy2 = _own_rows(x.reshape(rows, d)), _own_rows(dy.reshape(rows, d))
     dx = torch.empty(x.shape, dtype=x.dtype, device=x.device) if need_x else None
     wf = _aligned(_f32_weight(w, x.device))
     dw = torch.empty(d, dtype=torch.float32, device=x.device) if need_w else None
@@ -651,8 +653,7 @@ def weight_grad(dy, x):
     lib = _lib.load()
     rows, n = dy.shape
     k = x.shape[1]
-    dy = dy if _rows16(dy) else _aligned(dy)
-    x = x if _rows16(x) else _aligned(x)
+    dy, x = _own_rows(dy), _own_rows(x)
     out = torch.empty(n, k, dtype=torch.float32, device=dy.device)
     nbytes = lib.sdm_rt_weight_grad_workspace_bytes(rows, n, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dy.device) if nbytes else None

@@ -125,3 +125,48 @@ def test_offloaded_saved_tensors_give_the_same_gradients():
             y = m(x)
         grads.append(torch.autograd.grad(y.square().sum(), [x] + list(m.parameters())))
     assert all(torch.equal(a, b) for a, b in zip(*grads)) and math.isfinite(grads[0][0].sum().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_norm_and_weight_gradients_of_broadcast_rows(dtype):
+    """Gradients whose rows are one row repeated (stride 0, as a sum over tokens leaves them) equal those of the rows
+    written out, as do inputs of such rows."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(3, 7, 64, generator=g, device="cuda").to(dtype).requires_grad_(True)
+    w = torch.rand(64, generator=g, device="cuda").requires_grad_(True)
+    v = torch.randn(64, generator=g, device="cuda").to(dtype)
+    one = torch.randn(64, generator=g, device="cuda").to(dtype)
+    for xi in (x, one.expand(3, 7, 64).requires_grad_(True)):
+        y = core.RmsNormFunction.apply(xi, w, 1e-6, dtype)
+        got = torch.autograd.grad(y, (xi, w), v.expand(3, 7, 64), retain_graph=True)
+        want = torch.autograd.grad(y, (xi, w), v.expand(3, 7, 64).contiguous())
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    if dtype == torch.bfloat16:
+        x2 = x.detach().view(21, 64)
+        for a, b in ((v.expand(21, 64), x2), (x2, one.expand(21, 64))):
+            assert torch.equal(core.weight_grad(a, b), core.weight_grad(a.contiguous(), b.contiguous()))
+
+
+@pytest.mark.parametrize("amp,dtype", [(True, torch.bfloat16), (True, torch.float32), (False, torch.float32)])
+def test_training_steps_on_pooled_sums_and_broadcast_inputs(amp, dtype):
+    """sum over tokens as the loss (its gradient has rows of stride 0), inputs of broadcast rows and inputs that start on
+    no 16 bytes give what dense ones give."""
+    torch.manual_seed(5)
+    m = RunTimeSdm(64, heads=2, n_sub=8, d_a=16, k=4, decays=(0.5, 0.9)).to("cuda").train()
+    t = TrainedSdm(64, 8, heads=2, d_a=8, k=4).to("cuda").train()
+    torch.nn.init.xavier_uniform_(m.wo.weight)
+    torch.nn.init.normal_(t.values)
+    buf = torch.randn(2 * 70 * 64 + 1, device="cuda").to(dtype)
+    inputs = [buf[1:].view(2, 70, 64), torch.randn(64, device="cuda").to(dtype).expand(2, 70, 64)]
+    v = torch.randn(64, device="cuda").to(dtype)
+    for mod in (m, t):
+        for x in inputs:
+            res = []
+            for xi, dy in ((x, v.expand(2, 70, 64)), (x.clone(), v.expand(2, 70, 64).contiguous())):
+                xi = xi.detach().requires_grad_(True)
+                with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+                    y = mod(xi)
+                res.append((y, *torch.autograd.grad(y, [xi, *mod.parameters()], dy, allow_unused=True)))
+            for a, b in zip(*res):   # without autocast wo's gradients are the library's, in an order of its own by strides
+                assert (a is None and b is None) or torch.equal(a, b) or (
+                    not amp and (a - b).abs().max() <= 140 * 2.0 ** -24 * b.abs().max())
