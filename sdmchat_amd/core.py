@@ -587,7 +587,8 @@ def rms_norm(x, w, eps=1e-6, out_dtype=None, out=None):
 
 class RmsNormFunction(torch.autograd.Function):
     """rms_norm as an autograd function: the forward on the RMSNorm kernel (the reference's rounding, SM:63-71), the
-    backward rms_norm_backward.  apply(x, w, eps, out_dtype) -> y."""
+    backward rms_norm_backward, as torch ops where it is to be differentiated again (create_graph).
+    apply(x, w, eps, out_dtype) -> y."""
 
     @staticmethod
     def forward(ctx, x, w, eps, out_dtype):
@@ -598,14 +599,26 @@ class RmsNormFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
-        dx, dw = rms_norm_backward(x, w, dy, ctx.eps, *ctx.needs_input_grad[:2])
-        return dx, dw, None, None
+        grads = _rms_norm_backward_ops if torch.is_grad_enabled() else rms_norm_backward
+        return *grads(x, w, dy, ctx.eps, *ctx.needs_input_grad[:2]), None, None
 
 
 def _aligned(w):
     """A tensor whose data starts 16-byte aligned and is contiguous, a copy where it is not."""
     w = w.contiguous()
     return w if w.data_ptr() % 16 == 0 else w.clone()
+
+
+def _rms_norm_backward_ops(x, w, dy, eps, need_x=True, need_w=True):
+    """rms_norm_backward as torch ops, which autograd can follow."""
+    xf = x.float()
+    r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
+    n = xf * r
+    g = dy.float()
+    gw = g * w.float()
+    dx = r * (gw - n * (gw * n).mean(-1, keepdim=True)) if need_x else None
+    dw = (g * n).reshape(-1, x.shape[-1]).sum(0) if need_w else None
+    return None if dx is None else dx.to(x.dtype), None if dw is None else dw.to(w.dtype)
 
 
 def rms_norm_backward(x, w, dy, eps, need_x=True, need_w=True):
@@ -618,14 +631,7 @@ def rms_norm_backward(x, w, dy, eps, need_x=True, need_w=True):
     if not (need_x or need_w):
         return None, None
     if rows == 0 or d > 2048 or d % 8 or x.dtype not in _DT or dy.dtype not in _DT:
-        xf = x.float()
-        r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
-        n = xf * r
-        g = dy.float()
-        gw = g * w.float()
-        dx = r * (gw - n * (gw * n).mean(-1, keepdim=True)) if need_x else None
-        dw = (g * n).reshape(-1, d).sum(0) if need_w else None
-        return None if dx is None else dx.to(x.dtype), None if dw is None else dw.to(w.dtype)
+        return _rms_norm_backward_ops(x, w, dy, eps, need_x, need_w)
     x2, dy2 = _own_rows(x.reshape(rows, d)), _own_rows(dy.reshape(rows, d))
     dx = torch.empty(x.shape, dtype=x.dtype, device=x.device) if need_x else None
     wf = _aligned(_f32_weight(w, x.device))
@@ -666,27 +672,29 @@ def weight_grad(dy, x):
 class LinearFunction(torch.autograd.Function):
     """F.linear(x, w) under bfloat16 autocast, w any float type, with the weight gradient on sdm_rt_weight_grad: the
     same product in bfloat16, returned in ``out_dtype``.  The gradient of w stays float32 until it is cast to w's dtype
-    (autocast's own rounds it to bfloat16 on the way).  apply(x, w, out_dtype) -> y."""
+    (autocast's own rounds it to bfloat16 on the way); where it is to be differentiated again (create_graph) the
+    backward is torch ops on x and w.  apply(x, w, out_dtype) -> y."""
 
     @staticmethod
     def forward(ctx, x, w, out_dtype):
         with no_autocast():
-            x16, w16 = x.to(torch.bfloat16), w.to(torch.bfloat16)
-            ctx.save_for_backward(x16, w16)
-            ctx.dtypes = (x.dtype, w.dtype)
-            return torch.nn.functional.linear(x16, w16).to(out_dtype)
+            w16 = w.to(torch.bfloat16)
+            ctx.save_for_backward(x, w, w16)
+            return torch.nn.functional.linear(x.to(torch.bfloat16), w16).to(out_dtype)
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy):
-        x16, w16 = ctx.saved_tensors
+        x, w, w16 = ctx.saved_tensors
+        again = torch.is_grad_enabled()
         with no_autocast():
-            dy16 = dy.to(torch.bfloat16)
-            dx = torch.matmul(dy16, w16).to(ctx.dtypes[0]) if ctx.needs_input_grad[0] else None
+            dy16, x16 = dy.to(torch.bfloat16), x.to(torch.bfloat16)
+            if again:
+                w16 = w.to(torch.bfloat16)
+            dx = torch.matmul(dy16, w16).to(x.dtype) if ctx.needs_input_grad[0] else None
             dw = None
             if ctx.needs_input_grad[1]:
                 d2, x2 = dy16.reshape(-1, dy16.shape[-1]), x16.reshape(-1, x16.shape[-1])
-                dw = (weight_grad(d2, x2) if weight_grad_fits(d2, x2) else torch.matmul(d2.t(), x2)).to(ctx.dtypes[1])
+                dw = (torch.matmul(d2.t(), x2) if again or not weight_grad_fits(d2, x2) else weight_grad(d2, x2)).to(w.dtype)
         return dx, dw, None
 
 

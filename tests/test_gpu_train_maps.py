@@ -170,3 +170,40 @@ def test_training_steps_on_pooled_sums_and_broadcast_inputs(amp, dtype):
             for a, b in zip(*res):   # without autocast wo's gradients are the library's, in an order of its own by strides
                 assert (a is None and b is None) or torch.equal(a, b) or (
                     not amp and (a - b).abs().max() <= 140 * 2.0 ** -24 * b.abs().max())
+
+
+@pytest.mark.parametrize("d", [64, 768])
+def test_the_norm_differentiates_twice(d):
+    """The gradients of RmsNormFunction's gradients, against float64: sums of d float32 products in chains of four."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x, dy, a = (torch.randn(3, 5, d, generator=g, device="cuda") for _ in range(3))
+    w, b = torch.rand(d, generator=g, device="cuda") + 0.5, torch.randn(d, generator=g, device="cuda")
+
+    def twice(norm, cast):
+        xs, ws, ds = (cast(t).requires_grad_(True) for t in (x, w, dy))
+        gx, gw = torch.autograd.grad(norm(xs, ws), (xs, ws), ds, create_graph=True)
+        return torch.autograd.grad((gx * cast(a)).sum() + (gw * cast(b)).sum(), (xs, ws, ds))
+    got = twice(lambda x, w: core.RmsNormFunction.apply(x, w, 1e-6, torch.float32), lambda t: t.clone())
+    want = twice(lambda x, w: x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w, lambda t: t.double())
+    for p, q in zip(got, want):
+        assert (p.double() - q).abs().max() <= 4 * d * 2.0 ** -24 * q.abs().max()
+
+
+def test_the_output_map_differentiates_twice():
+    """The gradients of an autocast map's gradients equal those of the module called op by op: the same products, the
+    weight gradient not rounded to bfloat16 on its way (2^-8 of a value a rounding)."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    lin = torch.nn.Linear(64, 40, bias=False).cuda()
+    x, dy = torch.randn(2, 30, 64, generator=g, device="cuda"), torch.randn(2, 30, 40, generator=g, device="cuda")
+    a, b = torch.randn(40, 64, generator=g, device="cuda"), torch.randn(2, 30, 64, generator=g, device="cuda")
+    for dtype in (torch.float32, torch.bfloat16):
+        out = []
+        for f in (lambda v: core.train_linear(lin, v, torch.float32), lambda v: lin(v).float()):
+            xs, ds = x.to(dtype).requires_grad_(True), dy.clone().requires_grad_(True)
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = f(xs)
+            gw, gx = torch.autograd.grad(y, (lin.weight, xs), ds, create_graph=True)
+            out.append(torch.autograd.grad((gw * a).sum() + (gx.float() * b).sum(), (xs, lin.weight, ds)))
+        for p, q in zip(*out):
+            assert p.dtype == q.dtype
+            assert (p.double() - q.double()).abs().max() <= 2e-2 * q.double().abs().max()
