@@ -702,14 +702,24 @@ def autocast_bf16():
     return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
 
 
-def train_linear(lin, x, out_dtype):
-    """lin(x).to(out_dtype) with autograd recording: on LinearFunction under bfloat16 autocast where ``lin`` is a plain
-    nn.Linear without a bias or hooks; else the module itself."""
+def plain_module(mod, cls):
+    """Whether calling ``mod`` runs the forward of ``cls`` and nothing else: no hooks and no forward of its own."""
     hooks = torch.nn.modules.module
-    if (autocast_bf16() and type(lin) is torch.nn.Linear and lin.bias is None and x.is_cuda and x.dtype in _DT
-            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
-                     or hooks._global_forward_hooks or hooks._global_forward_pre_hooks
-                     or hooks._global_backward_hooks or hooks._global_backward_pre_hooks)):
+    return type(mod) is cls and "forward" not in mod.__dict__ and not (
+        mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+        or hooks._global_forward_hooks or hooks._global_forward_pre_hooks
+        or hooks._global_backward_hooks or hooks._global_backward_pre_hooks)
+
+
+def train_linear_fits(lin):
+    """Whether train_linear takes ``lin`` on LinearFunction: a plain nn.Linear without a bias, under bfloat16 autocast."""
+    return autocast_bf16() and plain_module(lin, torch.nn.Linear) and lin.bias is None
+
+
+def train_linear(lin, x, out_dtype):
+    """lin(x).to(out_dtype) with autograd recording: on LinearFunction where it serves ``lin`` (train_linear_fits), else
+    the module itself."""
+    if x.is_cuda and x.dtype in _DT and train_linear_fits(lin):
         return LinearFunction.apply(x, lin.weight, out_dtype)
     return lin(x).to(out_dtype)
 
@@ -1071,9 +1081,9 @@ class MixerFunction(torch.autograd.Function):
     same step moved every row about thirty times: a training step of the layer at B=8, T=2048 under bfloat16 autocast took
     1.99 ms that way; as one function 1.25 ms (84 launches, then 40), with the core backward of today 1.12 ms.
 
-    apply(x, norm_w, wk, wq, wv, wg, bg, keys1, keys2, addr_b, log_scale, decay, onorm_w, cfg) -> r [B, T, H * dh] in
-    the compute type.  wg and bg may be None (no write gate), onorm_w too.  cfg: dict with dtype (mixer_train_fits),
-    eps, first_rows (the padded rows of the first map), k, read_mode, out_norm, read_eps, out_norm_eps, reset and
+    apply(x, norm_w, wk, wq, wv, wg, bg, keys1, keys2, addr_b, log_scale, decay, onorm_w, cfg) -> r [B, T, H * dh].
+    wg and bg may be None (no write gate), onorm_w too.  cfg: dict with dtype (mixer_train_fits), out_dtype (r's), eps,
+    first_rows (the padded rows of the first map), k, read_mode, out_norm, read_eps, out_norm_eps, reset and
     workspace.  After the call cfg["gate_logits"] holds the gate logits [B, T, H] (a view of the first map's output)."""
 
     @staticmethod
@@ -1097,8 +1107,8 @@ class MixerFunction(torch.autograd.Function):
             g = pa[..., 2 * za:2 * za + H] if gated else None
             params = _params(x.device, keys1, keys2, addr_b, log_scale, decay, onorm_w, None)
             opts = {n: cfg[n] for n in ("k", "read_mode", "out_norm", "read_eps", "out_norm_eps")}
-            r, saved = core_forward_train(pa[..., :za], pa[..., za:2 * za], V, g, params=params, out_dtype=dt,
-                                          reset=cfg["reset"], workspace=cfg["workspace"], **opts)
+            r, saved = core_forward_train(pa[..., :za], pa[..., za:2 * za], V, g, params=params,
+                                          out_dtype=cfg["out_dtype"], reset=cfg["reset"], workspace=cfg["workspace"], **opts)
         cfg["gate_logits"] = g
         ctx.opts, ctx.eps, ctx.workspace, ctx.shape = opts, cfg["eps"], cfg["workspace"], (ra, za, gated)
         ctx.dtypes = [None if t is None else t.dtype for t in (wk, wq, wv, wg, bg)]

@@ -218,8 +218,9 @@ class RunTimeSdm(nn.Module):
         gate = (self.wg.weight, self.wg.bias) if self.write_gate else (None, None)
         weights = [self.wk.weight, self.wq.weight, self.wv.weight] + ([gate[0]] if self.write_gate else [])
         dt = core.mixer_train_fits(x, weights)
-        if dt is not None:
-            cfg.update(dtype=dt, eps=self.norm.eps, first_rows=self._rows_a())
+        if dt is not None:   # a wo that is not a plain map gets r in float32
+            cfg.update(dtype=dt, out_dtype=dt if core.train_linear_fits(self.wo) else torch.float32, eps=self.norm.eps,
+                       first_rows=self._rows_a())
             r = core.MixerFunction.apply(grad_scale(x, self.mem_in_grad), self.norm.w, *weights[:3], *gate, self.keys1,
                                          self.keys2, self.addr_b, self.log_scale, self.decay(), onorm_w, cfg)
             g = cfg["gate_logits"]

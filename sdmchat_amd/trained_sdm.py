@@ -101,16 +101,17 @@ class TrainedSdm(nn.Module):
         layer through TableSdmFunction, wo; under bfloat16 autocast the normed input and the read go from one op to the
         next in the bfloat16 that the maps would round them to."""
         B, T, _ = x.shape
-        amp = core.autocast_bf16()
-        w = self.norm.w
-        if x.dtype in (torch.float32, torch.bfloat16) and x.shape[-1] % 8 == 0:
+        if (x.dtype in (torch.float32, torch.bfloat16) and self.d % 8 == 0
+                and core.plain_module(self.norm, RMSNorm)):   # what the norm kernel serves
+            w = self.norm.w
+            amp = core.train_linear_fits(self.wq)
             hx = core.RmsNormFunction.apply(x, w, self.norm.eps,
                                             torch.bfloat16 if amp else torch.promote_types(x.dtype, w.dtype))
             hx = hx if amp else hx.float()
         else:
             hx = self.norm(x).float()
         q = core.train_linear(self.wq, hx, torch.float32)
-        cfg = dict(k=self.k, out_dtype=torch.bfloat16 if amp else torch.float32)
+        cfg = dict(k=self.k, out_dtype=torch.bfloat16 if core.train_linear_fits(self.wo) else torch.float32)
         r = core.TableSdmFunction.apply(q, self.keys1, self.keys2, self.log_scale, self.values, cfg)
         kk = min(self.k, min(self.k, self.n_sub) ** 2)
         self.last_si = cfg["slots"][..., :kk].permute(0, 2, 1, 3).reshape(B * T, self.h, kk)

@@ -207,3 +207,25 @@ def test_the_output_map_differentiates_twice():
         for p, q in zip(*out):
             assert p.dtype == q.dtype
             assert (p.double() - q.double()).abs().max() <= 2e-2 * q.double().abs().max()
+
+
+def test_hooks_and_replaced_forwards_of_the_table_layer_and_the_output_map_run():
+    """A hook on the table layer's norm, and a forward that was put on a norm or a map itself, see every training call."""
+    m = RunTimeSdm(64, heads=2, n_sub=8, d_a=16, k=4, decays=(0.5, 0.9)).to("cuda").train()
+    t = TrainedSdm(64, 8, heads=2, d_a=8, k=4).to("cuda").train()
+    x = torch.randn(2, 40, 64, device="cuda", requires_grad=True)
+    seen = []
+
+    def call(mod):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            mod(x).float().sum().backward()
+    hook = t.norm.register_forward_hook(lambda *a: seen.append("norm"))
+    call(t)
+    hook.remove()
+    assert seen == ["norm"]
+    for mod, sub in ((t, t.norm), (t, t.wq), (t, t.wo), (m, m.wo)):
+        inner = sub.forward
+        sub.forward = lambda *a, inner=inner: (seen.append(1), inner(*a))[1]
+        call(mod)
+        del sub.forward
+    assert seen == ["norm", 1, 1, 1, 1]
