@@ -101,8 +101,9 @@ class TrainedSdm(nn.Module):
         layer through TableSdmFunction, wo; under bfloat16 autocast the normed input and the read go from one op to the
         next in the bfloat16 that the maps would round them to."""
         B, T, _ = x.shape
-        if (x.dtype in (torch.float32, torch.bfloat16) and self.d % 8 == 0
-                and core.plain_module(self.norm, RMSNorm)):   # what the norm kernel serves
+        types = (torch.float32, torch.bfloat16)
+        if (x.dtype in types and self.d % 8 == 0 and self.d <= 2048 and core.plain_module(self.norm, RMSNorm)
+                and self.norm.w.dtype in types):   # what the norm kernel serves
             w = self.norm.w
             amp = core.train_linear_fits(self.wq)
             hx = core.RmsNormFunction.apply(x, w, self.norm.eps,

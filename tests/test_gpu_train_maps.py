@@ -229,3 +229,16 @@ def test_hooks_and_replaced_forwards_of_the_table_layer_and_the_output_map_run()
         call(mod)
         del sub.forward
     assert seen == ["norm", 1, 1, 1, 1]
+
+
+def test_the_table_layer_trains_past_the_norm_kernels_width():
+    """Rows wider than the norm kernel holds go through the norm module, as those of a width it does not divide."""
+    for d in (2056, 60):
+        t = TrainedSdm(d, 8, heads=1, d_a=8, k=4).to("cuda").train()
+        torch.nn.init.normal_(t.values)
+        x = torch.randn(2, 9, d, device="cuda", requires_grad=True)
+        y = t(x)
+        y.square().sum().backward()
+        q = t.wq(t.norm(x).float())
+        r = core.TableSdmFunction.apply(q, t.keys1, t.keys2, t.log_scale, t.values, dict(k=4))
+        assert torch.equal(y, t.wo(r)) and bool(torch.isfinite(x.grad).all())
