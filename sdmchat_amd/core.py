@@ -568,6 +568,8 @@ def rms_norm(x, w, eps=1e-6, out_dtype=None, out=None):
     if x.dtype not in _DT:
         raise ValueError(f"rms_norm: dtype {x.dtype} is not float32 or bfloat16")
     d = x.shape[-1]
+    if tuple(w.shape) != (d,):
+        raise RuntimeError(f"rms_norm: weight of shape {tuple(w.shape)} for rows of {d}")
     x2 = x.reshape(-1, d)
     if x2.numel():
         x2 = _own_rows(x2)
@@ -1058,13 +1060,13 @@ def _decay_grad(decay, log_decay):
     return torch.where(lam > 0, log_decay / lam, 0.0).to(decay.dtype)
 
 
-def mixer_train_fits(x, weights):
+def mixer_train_fits(x, weights, rows):
     """Whether MixerFunction serves a training forward: rows of float32 or bfloat16 whose width is a multiple of 8, the
-    projection weights of one type on x's device, run in bfloat16 under bfloat16 autocast or in float32 without
-    autocast on float32 weights.  Returns the compute dtype, or None."""
-    dt = weights[0].dtype
-    if not (x.is_cuda and x.dtype in _DT and x.numel() > 0 and x.shape[-1] % 8 == 0 and dt in _DT
-            and all(w.dtype == dt and w.device == x.device for w in weights)):
+    projection weights (of so many ``rows`` each) of one type on x's device, run in bfloat16 under bfloat16 autocast or in
+    float32 without autocast on float32 weights.  Returns the compute dtype, or None."""
+    dt, d = weights[0].dtype, x.shape[-1]
+    if not (x.is_cuda and x.dtype in _DT and x.numel() > 0 and d % 8 == 0 and dt in _DT
+            and all(w.dtype == dt and w.device == x.device and w.shape == (n, d) for w, n in zip(weights, rows))):
         return None
     if torch.is_autocast_enabled("cuda"):
         return torch.bfloat16 if autocast_bf16() else None

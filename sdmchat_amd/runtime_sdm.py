@@ -217,7 +217,7 @@ class RunTimeSdm(nn.Module):
         onorm_w = self.onorm_w if self.out_norm else None
         gate = (self.wg.weight, self.wg.bias) if self.write_gate else (None, None)
         weights = [self.wk.weight, self.wq.weight, self.wv.weight] + ([gate[0]] if self.write_gate else [])
-        dt = core.mixer_train_fits(x, weights)
+        dt = core.mixer_train_fits(x, weights, (H * self.d_a, H * self.d_a, self.d, H))
         if dt is not None:   # a wo that is not a plain map gets r in float32
             cfg.update(dtype=dt, out_dtype=dt if core.train_linear_fits(self.wo) else torch.float32, eps=self.norm.eps,
                        first_rows=self._rows_a())

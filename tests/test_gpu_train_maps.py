@@ -231,6 +231,19 @@ def test_hooks_and_replaced_forwards_of_the_table_layer_and_the_output_map_run()
     assert seen == ["norm", 1, 1, 1, 1]
 
 
+def test_projections_and_norms_of_other_shapes_are_refused():
+    """A projection or a norm replaced by one of another width raises, as the products and the norm raised op by op."""
+    x = torch.randn(2, 40, 64, device="cuda", requires_grad=True)
+    m = RunTimeSdm(64, heads=2, n_sub=8, d_a=16, k=4, decays=(0.5, 0.9)).to("cuda").train()
+    m.wq = torch.nn.Linear(32, 32, bias=False).cuda()
+    with pytest.raises(RuntimeError):
+        m(x)
+    t = TrainedSdm(64, 8, heads=2, d_a=8, k=4).to("cuda").train()
+    t.norm = type(t.norm)(32).cuda()
+    with pytest.raises(RuntimeError):
+        t(x)
+
+
 def test_the_table_layer_trains_past_the_norm_kernels_width():
     """Rows wider than the norm kernel holds go through the norm module, as those of a width it does not divide."""
     for d in (2056, 60):
