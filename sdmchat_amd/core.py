@@ -1073,6 +1073,15 @@ def mixer_train_fits(x, weights, rows):
     return torch.float32 if dt == torch.float32 else None
 
 
+def _input_grad(dp, W, ra):
+    """dp W for row gradients dp of the two maps whose weights W holds, the first ``ra`` rows and the rest, in float32:
+    one product of bfloat16 operands whose sums are not rounded to bfloat16 (rows of 16,384 x 2,560 x 768: 68 us either
+    way); in float32 the maps' products apart, as their sums in one chain were 2% further from 64 bits."""
+    if dp.dtype == torch.bfloat16:
+        return torch.mm(dp, W, out_dtype=torch.float32)
+    return torch.mm(dp[:, :ra], W[:ra]).addmm_(dp[:, ra:], W[ra:])
+
+
 class MixerFunction(torch.autograd.Function):
     """RunTimeSdm's training forward up to wo as one autograd function: the input norm, the two projection maps
     [wk; wq; wg] and wv (prepare, track4_onesdm_models.py:195-206) and the SDM core, in bfloat16 or float32.
@@ -1140,7 +1149,8 @@ class MixerFunction(torch.autograd.Function):
                                                                   dp[..., 2 * za:live] if gated else None), **ctx.opts)
             dx = dnw = None
             if need[0] or need[1]:
-                dx, dnw = rms_norm_backward(x, norm_w, torch.matmul(dp, W), ctx.eps, need[0], need[1])
+                dx, dnw = rms_norm_backward(x, norm_w, _input_grad(dp.view(B * T, ra + d), W, ra).view(B, T, d), ctx.eps,
+                                            need[0], need[1])
             dws = [None] * 4
             if any(need[2:6]):
                 d2, h2 = dp.view(B * T, ra + d), hx.view(B * T, d)

@@ -255,3 +255,25 @@ def test_the_table_layer_trains_past_the_norm_kernels_width():
         q = t.wq(t.norm(x).float())
         r = core.TableSdmFunction.apply(q, t.keys1, t.keys2, t.log_scale, t.values, dict(k=4))
         assert torch.equal(y, t.wo(r)) and bool(torch.isfinite(x.grad).all())
+
+
+def test_the_mixers_input_gradient_is_held_in_float32(monkeypatch):
+    """Under autocast the norm's backward gets the projections' input gradient in float32: a product of bfloat16 operands
+    within the bound of a float32 sum in any order, n 2^-24 of the sum of magnitudes, and not rounded to bfloat16."""
+    torch.manual_seed(7)
+    m = RunTimeSdm(96, heads=4, n_sub=8, d_a=16, k=8, decays=(0.6, 0.8, 0.95, 0.99)).to("cuda").train()
+    torch.nn.init.xavier_uniform_(m.wo.weight)
+    seen, prod = [], []
+    norm_bwd, input_grad = core.rms_norm_backward, core._input_grad
+    monkeypatch.setattr(core, "rms_norm_backward", lambda x, w, dy, *a: (seen.append(dy), norm_bwd(x, w, dy, *a))[1])
+    monkeypatch.setattr(core, "_input_grad", lambda *a: (prod.append(a[:2]), input_grad(*a))[1])
+    x = torch.randn(3, 130, 96, device="cuda", requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = m(x)
+    y.sum().backward()
+    dhx, (dp, W) = seen[0], prod[0]
+    assert dhx.dtype == torch.float32 and dp.dtype == W.dtype == torch.bfloat16
+    assert not torch.equal(dhx, dhx.bfloat16().float())
+    want = (dp.double() @ W.double()).view_as(dhx)
+    bound = (dp.shape[1] + 1) * 2.0 ** -24 * (dp.double().abs() @ W.double().abs()).view_as(dhx)
+    assert bool(((dhx.double() - want).abs() <= bound).all())
