@@ -191,8 +191,20 @@ def test_crowded_chunks_read_past_the_staged_plan():
     assert int(sizes.max()) > 4096
 
 
-@pytest.mark.parametrize("n_sub,H,dh", [(32, 2, 16), (60, 1, 8)])
-def test_crowded_plans_of_sixteen_picks(n_sub, H, dh):
+@pytest.mark.parametrize("n_sub,H,dh,staged", [(32, 2, 16, 4096), (60, 1, 8, 5120)])
+def test_crowded_plans_of_sixteen_picks(n_sub, H, dh, staged):
     """Plans whose variable part is past 4 KB: 1,024 locations leave LDS for the largest one, 3,600 for 5 KB, past which
-    the scan reads the plan from memory."""
-    check_core(*core_inputs(1, 150, H, dh, 32, n_sub, seed=93, addr_bias=4.0), 16)
+    the scan reads the plan from memory.  The workspace's plan sizes show that they got there."""
+    import torch
+    from sdmchat_amd import core
+    kz, qz, V, g, p = core_inputs(1, 150, H, dh, 32, n_sub, seed=93, addr_bias=4.0)
+    check_core(kz, qz, V, g, p, 16)
+    tp = {n: torch.from_numpy(v).cuda() for n, v in p.items()}
+    ws = core.CoreWorkspace()
+    core.core_forward(*(torch.from_numpy(a).cuda() for a in (kz, qz, V, g)), keys1=tp["keys1"], keys2=tp["keys2"],
+                      log_scale=tp["log_scale"], decay=tp["decay"], addr_b=tp["addr_b"], onorm_w=tp["onorm_w"],
+                      gate_bias=tp["gate_bias"], k=16, workspace=ws)
+    torch.cuda.synchronize()
+    sizes = ws.buf[:4 * H * 3].cpu().view(torch.int32)
+    say(f"variable-part bytes per plan: {sizes.tolist()}")
+    assert int(sizes.max()) > staged

@@ -265,6 +265,16 @@ def test_backward_is_deterministic():
             assert torch.equal(g1[n], g2[n]), n
 
 
+@pytest.mark.parametrize("dtype,reset_p,overlap", [(torch.float32, 0.0, 0.9), (torch.bfloat16, 0.003, 0.7)])
+def test_gradients_of_a_forward_in_segments(dtype, reset_p, overlap):
+    """One long sequence: the training forward's scan runs segments side by side, and the backward takes
+    the read-outs and the counts that they kept."""
+    B, T, H, dh, d_a, n_sub, k = 1, 1100, 12, 64, 32, 16, 8
+    b = [core.workspace_bytes(core.make_dims(B, 64 * c, H, dh, d_a, n_sub, k)) for c in (2, 3, 18)]
+    assert b[2] > b[1] + 15 * (b[1] - b[0]) + 4 * H * dh * n_sub * n_sub   # room for the segments' states
+    check_case("segments", 45, B, T, H, dh, d_a, n_sub, k, dtype=dtype, reset_p=reset_p, overlap=overlap)
+
+
 def test_training_forward_equals_inference_forward():
     t, reset = make(17, 2, 190, 3, 16, 16, 8, overlap=0.7, reset_p=0.02)
     cfg = dict(k=8, read_mode="mean", out_norm=True, read_eps=1e-3, out_norm_eps=1e-2)

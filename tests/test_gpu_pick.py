@@ -429,6 +429,24 @@ def test_segments_of_crowded_prompts(pattern, dtype):
         np.testing.assert_allclose(c, st[1], atol=2e-5 * scale, rtol=2e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_segments_of_value_rows_of_any_alignment(dtype):
+    """Value rows that start on no multiple of four values give the aligned rows' bits, segmented."""
+    B, T, H, dh = 1, 1100, 12, 64
+    kz, qz, V, g, p = core_inputs(B, T, H, dh, 64, 32, seed=72)
+    assert _segmented(B, T, H, dh, 32)
+    tp = {n: torch.from_numpy(v).cuda() for n, v in p.items()}
+    kzd, qzd, Vd, gd = (torch.from_numpy(a).cuda().to(dtype) for a in (kz, qz, V, g))
+    wide = torch.zeros(B, T, H * dh + 3, device="cuda", dtype=dtype)
+    wide[..., 1:1 + H * dh] = Vd
+    kw = dict(keys1=tp["keys1"], keys2=tp["keys2"], log_scale=tp["log_scale"], decay=tp["decay"], addr_b=tp["addr_b"],
+              onorm_w=tp["onorm_w"], gate_bias=tp["gate_bias"], k=8, want_state=True)
+    r0, (m0, c0) = core.core_forward(kzd, qzd, Vd, gd, **kw)
+    r1, (m1, c1) = core.core_forward(kzd, qzd, wide[..., 1:1 + H * dh], gd, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(r0, r1) and torch.equal(m0, m1) and torch.equal(c0, c1)
+
+
 def test_segments_state_written_over_its_input():
     """A state written back over the one it came from takes the unsegmented scan: the last segment could end before the
     first has read."""
