@@ -60,7 +60,10 @@ def _rows16(t2):
 def _own_rows(t2):
     """A 2-D view as rows that the kernels take: itself where the rows are 16-byte aligned (_rows16) and do not overlap (a
     row broadcast over many has stride 0), else a copy."""
-    return t2 if _rows16(t2) and t2.stride(0) >= t2.shape[1] else t2.clone(memory_format=torch.contiguous_format)
+    row, step = t2.stride()
+    if step == 1 and row >= t2.shape[1] and row * t2.element_size() % 16 == 0 and t2.data_ptr() % 16 == 0:
+        return t2
+    return t2.clone(memory_format=torch.contiguous_format)
 
 
 def _f32(t, device):
@@ -568,7 +571,7 @@ def rms_norm(x, w, eps=1e-6, out_dtype=None, out=None):
     if x.dtype not in _DT:
         raise ValueError(f"rms_norm: dtype {x.dtype} is not float32 or bfloat16")
     d = x.shape[-1]
-    if tuple(w.shape) != (d,):
+    if w.numel() != d:
         raise RuntimeError(f"rms_norm: weight of shape {tuple(w.shape)} for rows of {d}")
     x2 = x.reshape(-1, d)
     if x2.numel():
@@ -1079,7 +1082,8 @@ def _input_grad(dp, W, ra):
     way); in float32 the maps' products apart, as their sums in one chain were 2% further from 64 bits."""
     if dp.dtype == torch.bfloat16:
         return torch.mm(dp, W, out_dtype=torch.float32)
-    return torch.mm(dp[:, :ra], W[:ra]).addmm_(dp[:, ra:], W[ra:])
+    (da, dv), (wa, wv) = dp.split((ra, dp.shape[1] - ra), 1), W.split((ra, W.shape[0] - ra))
+    return torch.mm(da, wa).addmm_(dv, wv)
 
 
 class MixerFunction(torch.autograd.Function):
