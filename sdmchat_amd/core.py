@@ -1091,10 +1091,11 @@ class MixerFunction(torch.autograd.Function):
     [wk; wq; wg] and wv (prepare, track4_onesdm_models.py:195-206) and the SDM core, in bfloat16 or float32.
 
     The backward writes the core's row gradients straight into one [rows, [kz; qz; gate; zeros; v]] buffer in the
-    compute type, so the projections' input gradient and weight gradients are one product each, and the norm's backward
-    takes the product as it is.  Op by op (slices of the maps' outputs, casts, two products each way, their sums) the
-    same step moved every row about thirty times: a training step of the layer at B=8, T=2048 under bfloat16 autocast took
-    1.99 ms that way; as one function 1.25 ms (84 launches, then 40), with the core backward of today 1.12 ms.
+    compute type, so the projections' weight gradients are one product, their input gradient too under autocast
+    (_input_grad), and the norm's backward takes that as it is.  It cannot be differentiated again.  Op by op (slices of
+    the maps' outputs, casts, two products each way, their sums) the same step moved every row about thirty times: a
+    training step of the layer at B=8, T=2048 under bfloat16 autocast took 1.99 ms that way; as one function 1.25 ms (84
+    launches, then 40), with the core backward of today 1.12 ms.
 
     apply(x, norm_w, wk, wq, wv, wg, bg, keys1, keys2, addr_b, log_scale, decay, onorm_w, cfg) -> r [B, T, H * dh].
     wg and bg may be None (no write gate), onorm_w too.  cfg: dict with dtype (mixer_train_fits), out_dtype (r's), eps,

@@ -10,11 +10,13 @@
 //   dww[s,j]  = sum_{t>s} lam^(t-1-s) sum_i wr[t,i] [match] X[t][s]  = <V_s, B_s[siw_j]> + Bc_s[siw_j]
 //   dV_s      = sum_j ww[s,j] B_s[siw_j]
 // where mem/cnt is the forward memory and B/Bc the adjoint memory written by the reads (slots sir, weights wr,
-// values dnum, counts dden) and read by the writes, in reverse time.  Both are one kernel, grad_scan_kernel: a strict
-// causal scan whose reads return, per pick, the dot of the row read with a per-position vector (and optionally the
+// values dnum, counts dden) and read by the writes, in reverse time.  What a chunk of 64 tokens reads of its own writes
+// is chunk_grad_kernel's, for both directions; the memory carried over chunks is one kernel, grad_scan_kernel: a strict
+// causal scan whose reads return, per pick, the dot of the row read with a per-position vector (and, in reverse, the
 // weighted sum of the rows).  The forward direction gives dwr, the reverse direction dww and dV.  Then
-// addr_grad_kernel takes the softmax, gate, address normalisation and sub-key products back (pk_address :134-148,
-// prepare :199-207) and grad_reduce / keys_grad_kernel sum the parameter gradients in a fixed order.
+// addr_grad_tile_kernel (addr_grad_kernel past 64 sub-keys per half) takes the softmax, gate, address normalisation and
+// sub-key products back (pk_address :134-148, prepare :199-207) and grad_sums_kernel sums the parameter gradients in a
+// fixed order.
 //
 // lam * dL/dlam (the gradient with respect to log lam) needs no extra pass: sum_{t,s} (t-1-s) K[t][s] X[t][s]
 // = sum_t t P_t - sum_s (s+1) Q_s with P_t = sum_i wr[t,i] dwr[t,i] and Q_s = sum_j ww[s,j] dww[s,j].
@@ -1270,12 +1272,14 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
 //   dz      from du, u and |z|, held in the product's own layout: lane l keeps column l % 32 of 16 tokens, so the
 //           sums over an address half are sums over lanes of a half-wave
 //   dk^    += G^T U (the products' tokens in the order U's registers hold them)
-// Everything stays float32 (the products are fused multiply-adds in float32).  The kernel below does the same one
+// Everything stays float32 (the products are fused multiply-adds in float32).  addr_grad_kernel does the same one
 // token at a time, one lane per address element: per token 8 dependent LDS read-modify-writes for dk^, 24 readlanes
-// and the pick math on 8 of 64 lanes.  B=8, T=2048, 12 heads, k=8, bfloat16: 218 -> 117 us; the table layer's
-// (B=4, T=1024, one head, 64 sub-keys, k=16, float32): 50 -> 28 us.  What bounds it: 220 MB in and out (46 us at a
-// copy's rate) and the latency of a tile's chain (loads, k LDS additions, products) with two waves per SIMD: the
-// kernel takes 256 registers, and at three waves (168, 73 of them spilled) it took 141 us.
+// and the pick math on 8 of 64 lanes.  B=8, T=2048, 12 heads, k=8, bfloat16: 218 us so, 117 here on the same two partials
+// of a pick's dot, 130 on the three that it has with chunk_grad_kernel's; the table layer's (B=4, T=1024, one head, 64
+// sub-keys, k=16, float32): 50 and 33 us.  What bounds it: 176 MB in and out (36 us at a
+// copy's rate; 226 with row gradients in float32), and the latency of a tile's chain (loads, k LDS additions, products) with two waves per SIMD: the
+// kernel takes 256 registers (with two blocks of sub-keys 10 to 73 of them spilled), and at three waves (168, 73 of them
+// spilled with one) it took 141 us.
 // Sub-keys past n_sub, columns past the address and tokens past the end are zero rows and columns of the tiles.
 // The products run over every sub-key and 32 tokens, and 0 times an infinity is NaN: a block that meets an address or a
 // sub-key that is not finite does all its tokens again one at a time (addr_grad_block), so that it reaches no more than
@@ -1283,7 +1287,7 @@ __global__ void __launch_bounds__(64 * addr_grad_max_waves(KP)) addr_grad_kernel
 // Waves per block 4; tiles per wave chosen by addr_tiles (enough blocks for the chip first, then longer waves, since
 // every wave loads the head's sub-keys and leaves a partial sum).
 constexpr int kAddrTile = 32;
-constexpr int kAddrTileWaves = 4;
+constexpr int kAddrTileWaves = 4;   // (the waves' flags at the kernel's end are four)
 
 // sum over the 32 lanes of the lane's half-wave
 __device__ __forceinline__ float sum32(float v) {
@@ -1639,7 +1643,7 @@ __global__ void __launch_bounds__(64 * kAddrTileWaves, 2) addr_grad_tile_kernel(
 }
 
 // The parameter gradients from the blocks' partial records, all in one launch (seven of them, each a few microseconds
-// of launch and round trips, took 34 us of a backward; this one takes 8): block ranges by what they sum, 64 items a
+// of launch and round trips, took 34 us of a backward of B=8, T=2048; this one takes 10): block ranges by what they sum, 64 items a
 // block (reduce_item), in float64.
 //   keys    whole sub-key rows, 64 / half a block; from the summed unit sub-key gradient dk^ the raw one (F.normalize
 //           backward): dK = (dk^ - k^ <k^, dk^>) / |K|   (dk^ / 1e-12 below the floor)
@@ -1971,7 +1975,9 @@ int addr_grad_waves(int n_sub, int half, int KP) {
 }
 
 // 32-token tiles per wave of addr_grad_tile_kernel: the fewest that leave no more than two blocks for each of the 256
-// compute units (two fit), at most 8; 0 for more than 64 sub-keys per half, which addr_grad_kernel serves
+// compute units, at most 8; 0 for more than 64 sub-keys per half, which addr_grad_kernel serves.  Two blocks fit a
+// compute unit by their registers, and by their LDS with up to 32 sub-keys (43 KB a block); with more (84 KB) one fits,
+// and the second of a unit's two follows the first
 int addr_tiles(const Plan& p, int sets) {
   if (p.n_sub > 64) return 0;
   const int64_t N = static_cast<int64_t>(p.B) * p.T;

@@ -8,8 +8,8 @@ the HIP mixer (RunTimeSdm) and the per-token step is either ``x + SwiGLU(RMSNorm
 run on the RMSNorm kernel; the dense maps are hipBLASLt GEMMs through torch.  The reference's archive memory is a
 separate subsystem and is not built here (archive=True raises).
 
-Training: with autograd recording the mixers run their differentiable path (RunTimeSdm's SdmCoreFunction, backward
-on the HIP kernels), the TrainedSdm layers theirs (TableSdmFunction, sdm_rt_table_backward) and the norms the
+Training: with autograd recording the mixers run their differentiable path (core.MixerFunction, backward on the HIP
+kernels), the TrainedSdm layers theirs (core.TableSdmFunction, sdm_rt_table_backward) and the model's own norms the
 reference's torch ops, so every arm (ffn="mlp", "sdm", "none") trains.
 """
 import math

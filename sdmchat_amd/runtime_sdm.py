@@ -13,11 +13,12 @@ faded write / causal read of the memory and the mean read with its per-head norm
 ``libsdm_rt.so`` (sdm_rt_forward).  There is no CPU or pure-torch fallback: a missing library, a CPU tensor or an
 unsupported option raises.
 
-Training: with autograd recording (grad enabled and x or a parameter requiring grad) forward takes the reference's
-own torch path for the input norm (with grad_scale), the projections and wo, and runs the core through
-``core.SdmCoreFunction``, whose backward is ``sdm_rt_backward``: the gradients reach every parameter (the sub-keys,
-addr_b, log_scale, decay_logit with learn_decay, onorm_w, the projections and the gate bias) as under the
-reference's autograd of its chunked form (:259-268).
+Training: with autograd recording (grad enabled and x or a parameter requiring grad) forward runs the input norm, the
+projections and the core as one autograd function, ``core.MixerFunction`` (in bfloat16 under bfloat16 autocast, in
+float32 without autocast), and wo through ``core.train_linear``; other types take the projections as torch ops and the
+core through ``core.SdmCoreFunction``.  Either way the core's backward is ``sdm_rt_backward``: the gradients reach every
+parameter (the sub-keys, addr_b, log_scale, decay_logit with learn_decay, onorm_w, the projections and the gate bias) as
+under the reference's autograd of its chunked form (:259-268).
 """
 import math
 
@@ -238,7 +239,7 @@ class RunTimeSdm(nn.Module):
         """x [B, T, d] -> y [B, T, d] in x.dtype; every call starts from an empty memory
         (track4_onesdm_models.py:249-274).  reset [B, T] bool: where True the memory is emptied before that position
         reads (a BOS starts a new document, :229-233).  With ``keep_state`` set, ``last_state`` receives (mem, cnt)
-        (inference only).  With autograd recording the forward is differentiable (SdmCoreFunction).  hx: the input
+        (inference only).  With autograd recording the forward is differentiable (_forward_train).  hx: the input
         norm rms_norm(x) in the compute dtype, when the caller has it (inference only)."""
         B, T, _ = x.shape
         if not self.enabled:

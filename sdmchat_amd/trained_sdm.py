@@ -7,8 +7,9 @@ A drop-in for the reference module: the same constructor, parameter names, shape
 (sdm_rt_address: top-k of the n_sub^2 slots and the softmax weights) and the weighted table read (sdm_rt_table_read,
 the reference's embedding_bag), then the output map.  There is no CPU or torch fallback.
 
-Training: with autograd recording the norm, the query map and wo run as the reference's torch ops (under the
-caller's autocast) and the layer between them through ``core.TableSdmFunction``, whose backward is the HIP
+Training: with autograd recording the norm runs through ``core.RmsNormFunction``, the query map and wo through
+``core.train_linear`` (on the library's weight gradient under bfloat16 autocast), a norm or a map that is not plain as
+the module it is, and the layer between the maps through ``core.TableSdmFunction``, whose backward is the HIP
 ``sdm_rt_table_backward`` (gradients of the query, the sub-keys, log_scale and the value tables).
 """
 import math

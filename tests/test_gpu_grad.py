@@ -2,8 +2,8 @@
 training path against the float64 autograd oracle (oracle/sdm_grad64.py) for the same picks.
 
 Reference: the reference trains RunTimeSdm by autograd of prepare / _chunk / finish (track4_onesdm_models.py:195-274);
-topk carries no gradient, so the picks are taken from the HIP addressing (core.address, the kernel the training
-forward runs) and the oracle differentiates the rest in float64.  The oracle is pinned against finite differences of
+topk carries no gradient, so the picks are taken from the HIP addressing (core.address, which picks what the plan kernel
+of the training forward picks) and the oracle differentiates the rest in float64.  The oracle is pinned against finite differences of
 the fp64 token recurrence (tests/test_oracle_grad.py).
 
 Bar: every gradient within 1e-4 of the oracle's, relative to its largest entry (1e-6 absolute for a gradient whose
@@ -69,7 +69,7 @@ def run_hip(t, reset, cfg, dtype, wgt):
 
 
 def picks(dev, k):
-    """The HIP picks of both address sets, (B, T, H, kk) int64 (core.address runs the training forward's kernel)."""
+    """The HIP picks of both address sets, (B, T, H, kk) int64 (core.address picks as the training forward's plan)."""
     kw = dict(addr_b=dev["addr_b"].detach())
     sw, _, _ = core.address(dev["kz"].detach(), dev["keys1"].detach(), dev["keys2"].detach(), k,
                             dev["log_scale"].detach(), **kw)
