@@ -1161,8 +1161,9 @@ struct PlanGeom {
 // The pick plan (picks of at most 8, at most 1,024 locations; written by plan_kernel<..., PICK = true>, executed by
 // pick_scan_kernel):
 //   read records R[8][64], 12 bytes each, record (i, p) for pick i of position p:
-//     w0  read slot (bits 0..15; pads and positions past the chunk's end: M) | q (bits 16..21) | n_in (bits 24..31)
-//     w1  read weight (0 for pads and when a reset earlier in the chunk hides the carried state)
+//     w0  read slot (bits 0..15; M for pads, for positions past the chunk's end and where a reset earlier in the chunk
+//         hides the carried state) | q (bits 16..21) | n_in (bits 24..31)
+//     w1  read weight (0 for those)
 //     w2  coefficient of the position's in-chunk read contribution number i (q its source position), 0 if i >= n_in
 //   write records W[8][64], 12 bytes each:
 //     w0  write slot if p owns it (the first writer of the slot the chunk keeps), else M (bits 0..10) | q (bits

@@ -5,9 +5,9 @@
 //
 // One plan per (batch row, head, chunk) at a fixed stride (PlanGeom) in the workspace.
 //   position records [64], 16 KP + 48 bytes each, for position p of the chunk:
-//     u32 roff[KP]    read picks as byte offsets of their slab rows in the scan's LDS (slot * row_bytes; pads: row M,
-//                     which stays zero)
-//     f32 rw[KP]      read weights (0 for pads and when a reset earlier in the chunk hides the carried state)
+//     u32 roff[KP]    read picks as byte offsets of their slab rows in the scan's LDS (slot * row_bytes; pads, and all
+//                     when a reset earlier in the chunk hides the carried state: row M, which stays zero)
+//     f32 rw[KP]      read weights (0 for those)
 //     u32 woff[KP]    write picks owned by p (p is the first writer of the slot among the writers the chunk keeps) as
 //                     row byte offsets; picks p does not own: row M
 //     f32 wc[KP]      owned pick: lam^(L-1-p) * ww, p's faded write coefficient; else 0
@@ -158,8 +158,9 @@ __device__ __forceinline__ void emit_pick_plan(const PlanArgs& a, int b, int h, 
     }
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
-      const uint32_t slot = (p < L && i < kk) ? static_cast<uint32_t>(ms[i]) : mrow;
-      const float rw = (p < L && i < kk && seg0 < 0) ? ws[i] : 0.f;
+      const bool carried = p < L && i < kk && seg0 < 0;   // else the row that stays zero: 0 times an infinity is NaN
+      const uint32_t slot = carried ? static_cast<uint32_t>(ms[i]) : mrow;
+      const float rw = carried ? ws[i] : 0.f;
       *reinterpret_cast<uint3*>(plan + PickGeom::kRec * (i * kChunk + p)) =
           make_uint3(slot | (qj[i] << 16) | (static_cast<uint32_t>(n_in) << 24), __float_as_uint(rw),
                      __float_as_uint(cj[i]));
@@ -373,11 +374,14 @@ __global__ void __launch_bounds__(128, 3) plan_kernel(PlanArgs a) {
   uint32_t* tail = reinterpret_cast<uint32_t*>(prec + pg.off_tail());
   const uint32_t null_row = static_cast<uint32_t>(M) * static_cast<uint32_t>(a.row_bytes);
   if (set == 1) {
-    // read picks as row offsets and their weights (no carried state after a reset in this chunk)
+    // read picks as row offsets and their weights (no carried state after a reset in this chunk: the row that stays
+    // zero, since a weight of 0 times an infinity is NaN)
 #pragma unroll
     for (int i = 0; i < KP; i += 4) {
       *reinterpret_cast<uint4*>(prec + 4 * i) =
-          make_uint4(ms[i] * a.row_bytes, ms[i + 1] * a.row_bytes, ms[i + 2] * a.row_bytes, ms[i + 3] * a.row_bytes);
+          seg0 >= 0 ? make_uint4(null_row, null_row, null_row, null_row)
+                    : make_uint4(ms[i] * a.row_bytes, ms[i + 1] * a.row_bytes, ms[i + 2] * a.row_bytes,
+                                 ms[i + 3] * a.row_bytes);
       *reinterpret_cast<uint4*>(prec + pg.off_rw() + 4 * i) =
           seg0 >= 0 ? make_uint4(0u, 0u, 0u, 0u)
                     : make_uint4(__float_as_uint(ws[i]), __float_as_uint(ws[i + 1]), __float_as_uint(ws[i + 2]),

@@ -208,3 +208,24 @@ def test_crowded_plans_of_sixteen_picks(n_sub, H, dh, staged):
     sizes = ws.buf[:4 * H * 3].cpu().view(torch.int32)
     say(f"variable-part bytes per plan: {sizes.tolist()}")
     assert int(sizes.max()) > staged
+
+
+@pytest.mark.parametrize("k,n_sub,dh,T", [(8, 16, 64, 300), (8, 16, 24, 300), (16, 8, 32, 300), (8, 32, 64, 1100)])
+def test_a_reset_keeps_a_non_finite_document_out_of_the_next(k, n_sub, dh, T):
+    """Packed documents, an infinity in the values of one: the others' read-outs and the final state keep their bits (the
+    pick scan, the scan of eight and of sixteen picks, and segments).  A reset also shuts out a start state."""
+    H, cuts = 12, [100, 230, T - 50]
+    kz, qz, V, g, p = core_inputs(1, T, H, dh, 32, n_sub, seed=95, addr_bias=0.5)
+    qz = 0.3 * qz + kz
+    reset = np.zeros((1, T), bool)
+    reset[0, cuts] = True
+    r0, (m0, c0) = gpu_core(kz, qz, V, g, p, k, want_state=True, reset=reset)
+    bad = V.copy()
+    bad[0, 150] = np.inf
+    r1, (m1, c1) = gpu_core(kz, qz, bad, g, p, k, want_state=True, reset=reset)
+    other = [*range(100), *range(230, T)]
+    assert not np.isfinite(r1[:, 100:230]).all()
+    assert np.array_equal(r1[:, other], r0[:, other]) and np.array_equal(m1, m0) and np.array_equal(c1, c0)
+    full = (np.full((1, H, n_sub * n_sub, dh), np.nan, np.float32), np.full((1, H, n_sub * n_sub), np.inf, np.float32))
+    r2, (m2, c2) = gpu_core(kz, qz, V, g, p, k, state_in=full, want_state=True, reset=reset)
+    assert np.array_equal(r2[:, 100:], r0[:, 100:]) and np.array_equal(m2, m0) and np.array_equal(c2, c0)
